@@ -16,7 +16,8 @@
 //   device from context_lens.  A workgroup is 4 waves = hg KV heads x wph = 4 / hg
 //   slices; "virtual wave" vw = w * wph + slice owns one KV head of the group and the
 //   contiguous unit range [total * W(vw) / W(V), total * W(vw + 1) / W(V)), V = grid *
-//   wph, of a grid of resident workgroups (W sums per-wave weights; RangeWeights).  Every
+//   wph, of a grid of resident workgroups (W sums per-wave weights; RangeWeights); a call with
+//   few units gives one or two to each range instead.  Every
 //   wave streams its range alone (no work queue, no barrier, no cross-wave merge): pairs
 //   of tiles DMA (buffer loads into LDS) into its 16 KB slot one pair ahead, S^T = K Q^T
 //   and O^T += V^T P^T run on 16x16 MFMAs with the group's G <= 16 query heads as columns,
@@ -723,8 +724,22 @@ __global__ __launch_bounds__(kDecodeThreads, 2) void decode_split_kernel(DecodeP
   const int wl = __builtin_ctz(wph);  // wph is 1, 2 or 4
   const int64_t vw = (int64_t)blockIdx.x * wph + slice;
   const int64_t wt = Split::weight_before((int64_t)p.grid * wph, p.first_wgs, wl);
-  const int64_t ustart = Split::at(total, Split::weight_before(vw, p.first_wgs, wl), wt);
-  const int64_t uend = Split::at(total, Split::weight_before(vw + 1, p.first_wgs, wl), wt);
+  int64_t ustart, uend;
+  // Few units (at most two per workgroup that has a CU to itself): one or two to a range, and
+  // only as many ranges as that takes.  Spread over every resident wave, a sequence's units
+  // would lie between empty ranges, which the merge walks as well: one sequence of 1023 keys
+  // (16 query, 8 KV heads) had 256 ranges to merge, 39.8 us; with one unit a range 10.3 us (two:
+  // 12.4, four: 16.4).  One sequence of 8192 keys (32 and 8 heads) 45.7 us before, 17.2 with one
+  // unit a range (two workgroups per CU), 15.3 with two, 17.7 with four.
+  const int64_t alone = (int64_t)p.first_wgs * wph;
+  if (total <= 2 * alone) {
+    const int64_t per = total <= alone ? 1 : 2;
+    ustart = vw * per < total ? vw * per : total;
+    uend = ustart + per < total ? ustart + per : total;
+  } else {
+    ustart = Split::at(total, Split::weight_before(vw, p.first_wgs, wl), wt);
+    uend = Split::at(total, Split::weight_before(vw + 1, p.first_wgs, wl), wt);
+  }
   if (ustart >= uend) {
     // An empty range: the merge of a sequence that spans it reads its slot 0, which says
     // "no keys" (m = -inf, l = 0; o is not read then).  No barrier follows: waves leave on
@@ -1140,11 +1155,18 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_prefix_kernel(DecodePar
 // and the lane's two dims) and are merged online (running max, rescaled sums).  An empty
 // range inside a sequence wrote m = -inf there and adds nothing.  Pairs of empty
 // sequences get zeros; pairs finished by the split kernel are left alone.
+// WAVES > 1: a workgroup of that many waves per pair, wave w taking rows 16 w .. + 15 of
+// every 16 WAVES, merged through LDS; a pair of at most 16 rows is wave 0's alone.  Few
+// pairs (a small batch, whose sequences lie in many ranges) leave the chip to it: with at
+// most kCombineWide pairs 16 waves each, at most kCombineMid 4, i.e. at most 4096 waves
+// (half of what the chip holds).  32 sequences of 28 heads 53.1 -> 52.5 us; the 2048 pairs of
+// 64 sequences of 32 heads, each in few ranges, keep one wave (190 us either way).
 constexpr int kCombineRows = 16;
+constexpr int kCombineWide = 256, kCombineMid = 1024;
 
-template <int D, bool FP8>
-__global__ __launch_bounds__(kCombineThreads) void decode_split_combine_kernel(DecodeParams p,
-                                                                               int batch) {
+template <int D, int WAVES>
+__global__ __launch_bounds__(WAVES == 1 ? kCombineThreads : WAVES * kWave) void
+decode_split_combine_kernel(DecodeParams p, int batch) {
   static_assert(D <= 2 * kWave, "two output dims per lane");
   // Every parameter, and then the pair's three prefix entries, in one round of loads each:
   // left to itself the compiler loads each parameter on first use, behind the branches, and
@@ -1153,7 +1175,8 @@ __global__ __launch_bounds__(kCombineThreads) void decode_split_combine_kernel(D
                "s"(p.out_b), "s"(p.out_h), "s"(p.q_group), "s"(p.ws_rec), "s"(p.sp_ml),
                "s"(p.sp_o));
   const int lane = threadIdx.x & (kWave - 1);
-  const int pair = blockIdx.x * (kCombineThreads / kWave) + (threadIdx.x >> 6);
+  const int wave = uniform(threadIdx.x >> 6);
+  const int pair = WAVES > 1 ? blockIdx.x : blockIdx.x * (kCombineThreads / kWave) + wave;
   const int b = pair / p.num_heads;
   const int bl = b < batch ? b : batch - 1;  // the loads stay inside the prefix
   const int h = pair - b * p.num_heads;
@@ -1171,7 +1194,7 @@ __global__ __launch_bounds__(kCombineThreads) void decode_split_combine_kernel(D
   bf16_t* out = reinterpret_cast<bf16_t*>(p.out) + (int64_t)b * p.out_b +
                 (int64_t)(hk * p.q_group + gq) * p.out_h;
   if (n_units <= 0) {
-    if (has_dims) *reinterpret_cast<uint32_t*>(out + d0) = 0u;
+    if (has_dims && (WAVES == 1 || wave == 0)) *reinterpret_cast<uint32_t*>(out + d0) = 0u;
     return;
   }
   // the ranges f .. e that hold the sequence's units (recorded by the split kernel); f's
@@ -1179,9 +1202,11 @@ __global__ __launch_bounds__(kCombineThreads) void decode_split_combine_kernel(D
   const int f = rec.x >> 1, e = rec.y;
   if (f == e) return;  // one wave had the whole sequence and wrote it
   const int n = e - f + 1;
+  const int first = WAVES > 1 ? wave * kCombineRows : 0;
+  if (WAVES > 1 && n <= kCombineRows && wave > 0) return;  // one wave's worth of rows
   float m_run = -INFINITY, l_run = 0.f;
   float2 acc = make_float2(0.f, 0.f);
-  for (int c0 = 0; c0 < n; c0 += kCombineRows) {
+  for (int c0 = first; c0 < n; c0 += WAVES * kCombineRows) {
     float2 ml[kCombineRows], o[kCombineRows];
 #pragma unroll
     for (int i = 0; i < kCombineRows; ++i) {
@@ -1214,6 +1239,26 @@ __global__ __launch_bounds__(kCombineThreads) void decode_split_combine_kernel(D
       }
     }
     m_run = cm;
+  }
+  if constexpr (WAVES > 1) {
+    if (n > kCombineRows) {  // the same for every wave of the workgroup
+      __shared__ float2 s_ml[WAVES], s_acc[WAVES][kWave];
+      if (wave > 0) {
+        if (lane == 0) s_ml[wave] = make_float2(m_run, l_run);
+        s_acc[wave][lane] = acc;
+      }
+      __syncthreads();
+      if (wave > 0) return;
+      const int used = min(WAVES, (n + kCombineRows - 1) / kCombineRows);
+      for (int i = 1; i < used; ++i) {
+        float m, wa, wb;
+        softmax_merge_weights(m_run, s_ml[i].x, m, wa, wb);
+        m_run = m;
+        l_run = l_run * wa + s_ml[i].y * wb;
+        acc.x = acc.x * wa + s_acc[i][lane].x * wb;
+        acc.y = acc.y * wa + s_acc[i][lane].y * wb;
+      }
+    }
   }
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
   if (has_dims) *reinterpret_cast<uint32_t*>(out + d0) = pack_bf16x2(acc.x * inv, acc.y * inv);
@@ -1314,9 +1359,16 @@ int launch_split(DecodeParams& p, int batch, hipStream_t s) {
              batch);
   constexpr int kPairsPerGroup = kCombineThreads / kWave;
   const int64_t pairs = (int64_t)batch * p.num_heads;
-  nia_launch((decode_split_combine_kernel<D, FP8>),
-             dim3((unsigned)((pairs + kPairsPerGroup - 1) / kPairsPerGroup)),
-             dim3(kCombineThreads), s, p, batch);
+  if (pairs <= kCombineWide)
+    nia_launch((decode_split_combine_kernel<D, 16>), dim3((unsigned)pairs), dim3(16 * kWave), s, p,
+               batch);
+  else if (pairs <= kCombineMid)
+    nia_launch((decode_split_combine_kernel<D, 4>), dim3((unsigned)pairs), dim3(4 * kWave), s, p,
+               batch);
+  else
+    nia_launch((decode_split_combine_kernel<D, 1>),
+               dim3((unsigned)((pairs + kPairsPerGroup - 1) / kPairsPerGroup)),
+               dim3(kCombineThreads), s, p, batch);
   return hipGetLastError() == hipSuccess ? NIA_OK : NIA_ERR_LAUNCH;
 }
 
