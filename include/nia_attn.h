@@ -351,6 +351,29 @@ int32_t nia_dequant_gather_fp8(const void* k_cache, const void* v_cache, const f
                                void* out_k, void* out_v, int64_t seq_stride, void* stream);
 
 /*
+ * nia_prefill_paged over an fp8 cache (k_cache / v_cache / k_scale / v_scale as
+ * nia_paged_decode_fp8; q and out bf16, head_dim 128, any block_size >= 1): the keys are
+ * gathered and dequantised into the workspace (as nia_dequant_gather_fp8 does, keys in
+ * blocks outside [0, num_blocks) as zero rows), then attended by nia_prefill.  `workspace`:
+ * 256-byte aligned device memory of at least nia_prefill_paged_fp8_workspace_size(...)
+ * bytes; nothing in it needs initialising.
+ */
+size_t nia_prefill_paged_fp8_workspace_size(int32_t num_seqs, int32_t num_kv_heads,
+                                            int32_t max_blocks_per_seq, int32_t block_size,
+                                            int32_t head_dim);
+int32_t nia_prefill_paged_fp8(void* out, int64_t out_tok_stride, int64_t out_head_stride,
+                              const void* q, int64_t q_tok_stride, int64_t q_head_stride,
+                              const void* k_cache, const void* v_cache, const float* k_scale,
+                              const float* v_scale, const int32_t* block_tables,
+                              int32_t bt_stride, int32_t max_blocks_per_seq,
+                              const int32_t* q_start, const int32_t* q_len,
+                              const int64_t* context_lens, int32_t num_seqs, int32_t max_q_len,
+                              int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                              int32_t block_size, int64_t num_blocks, float scale,
+                              int32_t causal, void* workspace, size_t workspace_bytes,
+                              void* stream);
+
+/*
  * Step metadata: the padded model inputs and attention metadata of one engine
  * step, expanded on the device from a compact descriptor (one upload per step).
  * Replaces the loops of src/nano_inference/engine/context_builder.py:83-193

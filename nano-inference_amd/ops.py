@@ -652,7 +652,7 @@ def prefill_paged(
     q_start[s], sitting at absolute positions context_lens[s] - q_len[s] + j,
     and reads keys [0, context_lens[s]) through block_tables (B, max_blocks) int32.
     fp8 caches (with ``k_scale`` / ``v_scale``): the keys are first dequantised into
-    contiguous bf16 rows (nia_dequant_gather_fp8), then attended by nia_prefill.
+    contiguous bf16 rows, then attended as nia_prefill does (nia_prefill_paged_fp8).
     """
     if is_fp8_cache(k_cache):
         return _prefill_paged_fp8(q, k_cache, v_cache, block_tables, q_start, q_len,
@@ -722,18 +722,29 @@ def _prefill_paged_fp8(q, k_cache, v_cache, block_tables, q_start, q_len, contex
         raise ValueError("context_lens must be (B,) int64")
     context_lens = context_lens.contiguous()
     mb = block_tables.shape[1]
-    stride = mb * bs
-    keys = torch.empty((n * stride, hkv, d), dtype=torch.bfloat16, device=dev)
-    vals = torch.empty_like(keys)
+    _, h, dq = q.shape
+    if dq != d:
+        raise ValueError("head_dim mismatch between q and k/v")
+    if h % hkv != 0:
+        raise ValueError(f"num_heads must be divisible by num_kv_heads, got {h=} and {hkv=}")
+    _last_contig("q", q)
+    qs, ql = _i32("q_start", q_start, n), _i32("q_len", q_len, n)
+    if out is None:
+        out = torch.empty_like(q, memory_format=torch.contiguous_format)
+    elif out.shape != q.shape or out.dtype != q.dtype:
+        raise ValueError("out must match q's shape and dtype")
+    _last_contig("out", out)
     lib = _lib.load()
-    st = lib.nia_dequant_gather_fp8(
+    ws = torch.empty(lib.nia_prefill_paged_fp8_workspace_size(n, hkv, mb, bs, d),
+                     dtype=torch.uint8, device=dev)
+    st = lib.nia_prefill_paged_fp8(
+        out.data_ptr(), out.stride(0), out.stride(1), q.data_ptr(), q.stride(0), q.stride(1),
         k_cache.data_ptr(), v_cache.data_ptr(), k_scale.data_ptr(), v_scale.data_ptr(),
-        block_tables.data_ptr(), block_tables.stride(0), mb, context_lens.data_ptr(), n, hkv, d,
-        bs, nb, keys.data_ptr(), vals.data_ptr(), stride, _stream(dev))
-    _lib.check("nia_dequant_gather_fp8", st)
-    k_start = torch.arange(n, device=dev, dtype=torch.int32) * stride
-    k_len = context_lens.clamp(0, stride).to(torch.int32)
-    return prefill(q, keys, vals, q_start, q_len, k_start, k_len, max_q_len, causal, scale, out)
+        block_tables.data_ptr(), block_tables.stride(0), mb, qs.data_ptr(), ql.data_ptr(),
+        context_lens.data_ptr(), n, int(max_q_len), h, hkv, d, bs, nb,
+        _default_scale(d, scale), int(causal), ws.data_ptr(), ws.numel(), _stream(dev))
+    _lib.check("nia_prefill_paged_fp8", st)
+    return out
 
 
 # ---------------------------------------------------------------------------------
