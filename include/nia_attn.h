@@ -231,6 +231,39 @@ int32_t nia_prefill_paged(void* out, int64_t out_tok_stride, int64_t out_head_st
                           void* stream);
 
 /*
+ * nia_prefill and nia_prefill_paged with caller memory: a call whose workgroups leave the
+ * chip idle (few query rows over long keys) cuts each row block's keys into ranges that run
+ * side by side and merges their fp32 partials from the workspace in a second launch.
+ * `max_k_len`: a bound of the sequences' key counts (paged calls: the table width).
+ * `workspace`: 256-byte aligned device memory; nia_prefill_split_workspace_size gives the
+ * bytes that a call can use, 0 where it would not cut (fp32, enough rows, short keys).  A
+ * null, unaligned or smaller workspace runs the call uncut.  Nothing in it needs
+ * initialising; calls one after another on a stream may share it.
+ */
+size_t nia_prefill_split_workspace_size(int32_t num_seqs, int32_t max_q_len, int64_t max_k_len,
+                                        int32_t num_heads, int32_t num_kv_heads,
+                                        int32_t head_dim, int32_t causal, int32_t dtype);
+int32_t nia_prefill_split(void* out, int64_t out_tok_stride, int64_t out_head_stride,
+                          const void* q, int64_t q_tok_stride, int64_t q_head_stride,
+                          const void* k, int64_t k_tok_stride, int64_t k_head_stride,
+                          const void* v, int64_t v_tok_stride, int64_t v_head_stride,
+                          const int32_t* q_start, const int32_t* q_len, const int32_t* k_start,
+                          const int32_t* k_len, int32_t num_seqs, int32_t max_q_len,
+                          int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, float scale,
+                          int32_t causal, int32_t dtype, int64_t max_k_len, void* workspace,
+                          size_t workspace_bytes, void* stream);
+int32_t nia_prefill_paged_split(void* out, int64_t out_tok_stride, int64_t out_head_stride,
+                                const void* q, int64_t q_tok_stride, int64_t q_head_stride,
+                                const void* k_cache, const void* v_cache,
+                                const int32_t* block_tables, int32_t bt_stride,
+                                int32_t max_blocks_per_seq, const int32_t* q_start,
+                                const int32_t* q_len, const int64_t* context_lens,
+                                int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
+                                int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                                int64_t num_blocks, float scale, int32_t causal, int32_t dtype,
+                                void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Fused QK-RMSNorm + RoPE / mRoPE + KV-cache write, in place on q and k.
  * Replaces the steps between the projections and attention in
  * src/nano_inference/layers/attention.py:254-278: q_norm / k_norm
@@ -358,9 +391,10 @@ int32_t nia_dequant_gather_fp8(const void* k_cache, const void* v_cache, const f
  * 256-byte aligned device memory of at least nia_prefill_paged_fp8_workspace_size(...)
  * bytes; nothing in it needs initialising.
  */
-size_t nia_prefill_paged_fp8_workspace_size(int32_t num_seqs, int32_t num_kv_heads,
+size_t nia_prefill_paged_fp8_workspace_size(int32_t num_seqs, int32_t max_q_len,
+                                            int32_t num_heads, int32_t num_kv_heads,
                                             int32_t max_blocks_per_seq, int32_t block_size,
-                                            int32_t head_dim);
+                                            int32_t head_dim, int32_t causal);
 int32_t nia_prefill_paged_fp8(void* out, int64_t out_tok_stride, int64_t out_head_stride,
                               const void* q, int64_t q_tok_stride, int64_t q_head_stride,
                               const void* k_cache, const void* v_cache, const float* k_scale,

@@ -101,7 +101,20 @@ SIGNATURES = {
         _i32,
         [_p, _p, _p, _p, _p, _i32, _i32, _p, _i32, _i32, _i32, _i32, _i64, _p, _p, _i64, _p],
     ),
-    "nia_prefill_paged_fp8_workspace_size": (_sz, [_i32, _i32, _i32, _i32, _i32]),
+    "nia_prefill_split_workspace_size": (
+        _sz, [_i32, _i32, _i64, _i32, _i32, _i32, _i32, _i32]),
+    "nia_prefill_split": (
+        _i32,
+        [_p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64,
+         _p, _p, _p, _p, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _i64, _p, _sz, _p],
+    ),
+    "nia_prefill_paged_split": (
+        _i32,
+        [_p, _i64, _i64, _p, _i64, _i64, _p, _p, _p, _i32, _i32, _p, _p, _p,
+         _i32, _i32, _i32, _i32, _i32, _i32, _i64, _f32, _i32, _i32, _p, _sz, _p],
+    ),
+    "nia_prefill_paged_fp8_workspace_size": (
+        _sz, [_i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "nia_prefill_paged_fp8": (
         _i32,
         [_p, _i64, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _i32, _i32, _p, _p, _p, _i32,

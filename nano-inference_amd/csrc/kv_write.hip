@@ -385,14 +385,19 @@ size_t fp8_index_bytes(int32_t num_seqs) { return ((size_t)num_seqs * 8 + 255) /
 
 }  // namespace
 
-extern "C" size_t nia_prefill_paged_fp8_workspace_size(int32_t num_seqs, int32_t num_kv_heads,
+extern "C" size_t nia_prefill_paged_fp8_workspace_size(int32_t num_seqs, int32_t max_q_len,
+                                                       int32_t num_heads, int32_t num_kv_heads,
                                                        int32_t max_blocks_per_seq,
-                                                       int32_t block_size, int32_t head_dim) {
+                                                       int32_t block_size, int32_t head_dim,
+                                                       int32_t causal) {
   if (num_seqs <= 0 || num_kv_heads <= 0 || max_blocks_per_seq < 0 || block_size <= 0 ||
       head_dim <= 0)
     return 0;
   return fp8_index_bytes(num_seqs) + 2 * (size_t)num_seqs * max_blocks_per_seq * block_size *
-                                         num_kv_heads * head_dim * sizeof(bf16_t);
+                                         num_kv_heads * head_dim * sizeof(bf16_t) +
+         nia_prefill_split_workspace_size(num_seqs, max_q_len,
+                                          (int64_t)max_blocks_per_seq * block_size, num_heads,
+                                          num_kv_heads, head_dim, causal, NIA_DTYPE_BF16);
 }
 
 extern "C" int32_t nia_prefill_paged_fp8(
@@ -414,17 +419,19 @@ extern "C" int32_t nia_prefill_paged_fp8(
     return NIA_ERR_UNSUPPORTED;
   uint8_t* ws = (uint8_t*)workspace;
   int32_t *k_start = nullptr, *k_len = nullptr;
-  uint8_t *keys = nullptr, *vals = nullptr;
+  uint8_t *keys = nullptr, *vals = nullptr, *split = nullptr;
+  size_t split_bytes = 0;
   if (num_seqs > 0 && max_blocks_per_seq > 0) {
-    if (!ws || workspace_bytes < nia_prefill_paged_fp8_workspace_size(
-                                     num_seqs, num_kv_heads, max_blocks_per_seq, block_size,
-                                     head_dim))
-      return NIA_ERR_WORKSPACE;
+    const size_t half =
+        (size_t)num_seqs * rows * num_kv_heads * head_dim * sizeof(bf16_t);
+    if (!ws || workspace_bytes < fp8_index_bytes(num_seqs) + 2 * half) return NIA_ERR_WORKSPACE;
     if (!aligned(ws, 256)) return NIA_ERR_MISALIGNED;
     k_start = (int32_t*)ws;
     k_len = k_start + num_seqs;
     keys = ws + fp8_index_bytes(num_seqs);
-    vals = keys + (size_t)num_seqs * rows * num_kv_heads * head_dim * sizeof(bf16_t);
+    vals = keys + half;
+    split = vals + half;
+    split_bytes = workspace_bytes - (size_t)(split - ws);
     GatherParams p{};
     int32_t st = gather_params(p, k_cache, v_cache, k_scale, v_scale, block_tables, bt_stride,
                                max_blocks_per_seq, context_lens, num_kv_heads, block_size,
@@ -439,8 +446,8 @@ extern "C" int32_t nia_prefill_paged_fp8(
     st = launch_gather(p, num_seqs, (hipStream_t)stream);
     if (st != NIA_OK) return st;
   }
-  return nia_prefill(out, out_tok_stride, out_head_stride, q, q_tok_stride, q_head_stride, keys, tok,
+  return nia_prefill_split(out, out_tok_stride, out_head_stride, q, q_tok_stride, q_head_stride, keys, tok,
                      head_dim, vals, tok, head_dim, q_start, q_len, k_start, k_len, num_seqs,
                      max_q_len, num_heads, num_kv_heads, head_dim, scale, causal, NIA_DTYPE_BF16,
-                     stream);
+                     rows, split, split_bytes, stream);
 }

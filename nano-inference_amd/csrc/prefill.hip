@@ -76,6 +76,14 @@ struct PrefillParams {
   int32_t num_heads;
   int32_t num_kv_heads;
   int32_t group;
+  // Rows of an m-block: row r of a (sequence, head index) item is query token r / pack, head
+  // pack * index + r % pack: a KV head's whole group (pack = group, map_group = 1 head index
+  // per KV head) or one head (pack = 1, map_group = group); set_rows says when.
+  int32_t pack;
+  uint32_t pack_magic;  // r / pack = key_block(r, ...) for pack > 1
+  int32_t pack_shift;
+  int32_t map_group;
+  int32_t q_span;  // bytes 16 consecutive rows of q span (DMA kernel)
   int32_t num_m_blocks;
   int32_t num_seqs;
   int32_t groups_per_xcd;  // ceil(num_seqs * num_kv_heads / kXcds)
@@ -87,7 +95,19 @@ struct PrefillParams {
   const float* bias;
   int64_t bias_seq, bias_head, bias_q;
   float scale;
+  // SPLIT: key ranges per m-block at most (grid y), and their partials, row-major per
+  // (range, workgroup, row): o[D] and (m, l) in fp32
+  int32_t splits;
+  float* part_o;
+  float* part_ml;
 };
+
+// Key tiles of an m-block of `tiles` tiles are cut into this many ranges (kSplitMinTiles each
+// at least); range s takes tiles [tiles s / n, tiles (s + 1) / n).
+constexpr int kSplitMinTiles = 4;
+NIA_DEVICE int key_ranges(int tiles, int splits) {
+  return max(1, min(splits, tiles / kSplitMinTiles));
+}
 
 // Workgroup -> (sequence, head, m-block) mapping of the 1-D prefill grid.
 //
@@ -99,21 +119,33 @@ struct PrefillParams {
 // so the longest rows of every group start first and the short ones fill the
 // tail.  Ids that map past the real work (ragged sequences, uneven groups per
 // XCD) return false.
+// The hardware hands an XCD's workgroups to its shader engines in turn, whatever each still
+// has to do, so workgroups that follow each other must do about the same work: consecutive
+// ones are the heads of one group and level, or where a KV head's heads are packed into the
+// rows, kLevelRun adjacent levels of one group.  One level of every group in turn put each
+// sequence on one engine: causal prefill of eight sequences of 256-4096 tokens 585 us
+// instead of 320-335.
 constexpr int kXcds = 8;
+constexpr int kLevelRun = 4;
 
 NIA_DEVICE bool prefill_map(const PrefillParams& p, int& seq, int& h, int& mb) {
   const int id = blockIdx.x;
   const int x = id % kXcds;
   const int t = id / kXcds;
-  const int per_z = p.groups_per_xcd * p.group;
-  const int z = t / per_z;
-  const int rem = t - z * per_z;
-  const int j = rem / p.group;
-  const int g = rem - j * p.group;
+  // `run` workgroups of one group follow each other: its heads of one level, or (one head
+  // index per KV head) kLevelRun levels of it
+  const bool heads = p.map_group > 1;
+  const int run = heads ? p.map_group : kLevelRun;
+  const int per_z = p.groups_per_xcd * run;
+  const int z0 = t / per_z;
+  const int rem = t - z0 * per_z;
+  const int j = rem / run;
+  const int g = rem - j * run;
   const int gid = x + kXcds * j;
+  const int z = heads ? z0 : z0 * kLevelRun + g;
   if (z >= p.num_m_blocks || gid >= p.num_seqs * p.num_kv_heads) return false;
   seq = gid / p.num_kv_heads;
-  h = (gid - seq * p.num_kv_heads) * p.group + g;
+  h = (gid - seq * p.num_kv_heads) * p.map_group + (heads ? g : 0);
   mb = p.num_m_blocks - 1 - z;
   return true;
 }
@@ -145,16 +177,16 @@ NIA_DEVICE bool prefill_map_ranked(const PrefillParams& p, const int* s_order, i
   const int id = blockIdx.x;
   const int x = id % kXcds;
   const int t = id / kXcds;
-  const int per_j = p.num_m_blocks * p.group;
+  const int per_j = p.num_m_blocks * p.map_group;
   const int j = t / per_j;
   const int rem = t - j * per_j;
-  const int z = rem / p.group;
-  const int g = rem - z * p.group;
+  const int z = rem / p.map_group;
+  const int g = rem - z * p.map_group;
   const int gid = x + kXcds * j;
   if (j >= p.groups_per_xcd || gid >= p.num_seqs * p.num_kv_heads) return false;
   const int r = gid / p.num_kv_heads;
   seq = s_order[r];
-  h = (gid - r * p.num_kv_heads) * p.group + g;
+  h = (gid - r * p.num_kv_heads) * p.map_group + g;
   mb = p.num_m_blocks - 1 - z;
   return true;
 }
@@ -519,12 +551,17 @@ constexpr int kTileBytes = kBlockN * kTileRowBytes;  // 16 KB
 // COMPACT (paired heads, D < 128): K/V rows keep their own D * 2 bytes in LDS (no swizzle)
 // instead of 256, so three workgroups fit a CU instead of two: the short windows are bound
 // by the latency of their loads, which more resident workgroups hide.
+// PACK: the item's rows are the packed query heads of a KV head (p.pack rows a token, one
+// possible); a variant of its own, since the division and its parameters cost the
+// workgroups of one small image 3% at their start.
+// SPLIT: workgroup y takes the y-th range of its m-block's key tiles and writes fp32
+// partials for prefill_merge_kernel, unless the m-block has one range.
 // DIV: paged, with a block size that is a multiple of 16 but not a power of two (a key's
 // block by division instead of a shift).  QUAD (with DIV): a multiple of 4 but not of 16, so
 // a wave's 16-row DMA group may cross blocks: each DMA instruction (4 rows, which lie in
 // one block) gets the block and buffer resource of its own rows.
 template <int D, bool PAGED, bool PAIR = false, bool BIAS = false, bool COMPACT = false,
-          bool DIV = false, bool QUAD = false>
+          bool DIV = false, bool QUAD = false, bool PACK = false, bool SPLIT = false>
 __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_kernel(
     PrefillParams p) {
   static_assert(D % 16 == 0 && D <= 128, "head_dim a multiple of 16, at most 128");
@@ -533,6 +570,9 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
   static_assert(!COMPACT || (PAIR && D < 128), "compact rows serve paired heads, D < 128");
   static_assert(!DIV || PAGED, "block division serves paged calls");
   static_assert(!QUAD || DIV, "4-row groups take a key's block by division");
+  static_assert(!(PACK || SPLIT) || !(PAIR || BIAS || DIV),
+                "packed heads and key ranges: plain contiguous or paged calls");
+  static_assert(!SPLIT || PACK, "key ranges take either row form");
   constexpr int DK = D / 16;              // QK steps of 16 dims
   constexpr int DT = (D + 31) / 32;       // PV output tiles of 32 dims (the last one padded)
   constexpr int kChunks = D / 8;          // 16-byte chunks per K/V row
@@ -603,24 +643,47 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
   // the others past it, a second round trip).  Windows 18.2 -> 17.4 us.
   if constexpr (PAIR) asm volatile("" ::"s"(qstart), "s"(klen), "s"(kstart));
   const int m0 = mb * (PAIR ? kBlockM / 2 : kBlockM);
-  if (m0 >= qlen) return;
+  const int pack = PACK ? p.pack : 1;
+  const int rows = qlen * pack;  // the item's rows (host: at most INT32_MAX)
+  if (m0 >= rows) return;
+  h *= pack;  // head of row 0
   const int hk = h / p.group;
+  // the query token of row r (its head: h + r - pack * tok_of(r))
+  auto tok_of = [&](int r) __attribute__((always_inline)) -> int {
+    return !PACK || pack == 1 ? r : key_block(r, p.pack_magic, p.pack_shift);
+  };
   const bool causal = p.causal != NIA_CAUSAL_NONE;
   const int q_pos0 = p.causal == NIA_CAUSAL_BOTTOM_RIGHT ? klen - qlen : 0;
   int n_end = klen;
-  if (causal) n_end = min(klen, q_pos0 + min(m0 + kBlockM, qlen));
+  if (causal) n_end = min(klen, q_pos0 + uniform(tok_of(min(m0 + kBlockM, rows) - 1)) + 1);
   if (n_end < 0) n_end = 0;
+
+  // keys [n_begin, n_stop) are this workgroup's
+  int n_begin = 0, n_stop = n_end, ranges = 1;
+  if constexpr (SPLIT) {
+    const int tiles = (n_end + kBlockN - 1) / kBlockN;
+    ranges = key_ranges(tiles, p.splits);
+    const int s = blockIdx.y;
+    if (s >= ranges) return;
+    n_begin = tiles * s / ranges * kBlockN;
+    n_stop = min(n_end, tiles * (s + 1) / ranges * kBlockN);
+  }
 
   const int r0 = m0 + wrow * 32;
   const int qrow = r0 + col;
-  const bool row_ok = qrow < qlen;
-  const int kb = causal ? min(klen, q_pos0 + qrow + 1) : klen;
-  const int wave_kmin = causal ? min(klen, q_pos0 + r0 + 1) : klen;
-  const int wave_kend = r0 < qlen ? (causal ? min(klen, q_pos0 + min(r0 + 32, qlen)) : klen) : 0;
+  const bool row_ok = qrow < rows;
+  const int qtok = tok_of(qrow);        // this lane's query token
+  const int qhead = qrow - qtok * pack;  // and its head past h
+  const int kb = causal ? min(klen, q_pos0 + qtok + 1) : klen;
+  const int wave_kmin = causal ? min(klen, q_pos0 + uniform(tok_of(r0)) + 1) : klen;
+  const int wave_kend =
+      r0 < rows
+          ? (causal ? min(klen, q_pos0 + uniform(tok_of(min(r0 + 32, rows) - 1)) + 1) : klen)
+          : 0;
 
   uint4 qreg[DK];
   if constexpr (PAIR) {
-    const bf16_t* qp = p.q + (qstart + (row_ok ? qrow : 0)) * p.q_tok + (int64_t)h * p.q_head;
+    const bf16_t* qp = p.q + (qstart + (row_ok ? qtok : 0)) * p.q_tok + (int64_t)h * p.q_head;
 #pragma unroll
     for (int kk = 0; kk < DK; ++kk)
       qreg[kk] = row_ok ? *reinterpret_cast<const uint4*>(qp + 16 * kk + 8 * half)
@@ -798,8 +861,9 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
   const float sl = BIAS ? kLog2e : p.scale_log2;
   const float* bias_row = nullptr;  // BIAS: this lane's query row of the mask
   if constexpr (BIAS)
-    bias_row = p.bias + (int64_t)seq * p.bias_seq + (int64_t)h * p.bias_head +
-               (int64_t)(row_ok ? qrow : 0) * p.bias_q;
+    bias_row = p.bias + (int64_t)seq * p.bias_seq +
+               (int64_t)(h + (row_ok ? qhead : 0)) * p.bias_head +
+               (int64_t)(row_ok ? qtok : 0) * p.bias_q;
   auto compute_tile = [&](int n0, int stage) __attribute__((always_inline)) {
     const uint8_t* kt = tile_k(stage);
     const uint8_t* vt = tile_v(stage);
@@ -1004,7 +1068,7 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
         issue_pair(n0 + kBlockN);
       }
     }
-  } else if (n_end > 0) {
+  } else if (n_begin < n_stop) {
   // ---- main loop: tile n0 in one stage while tile n0 + 64 streams into the other ---------
   // Unrolled by two so that each stage's LDS offsets are compile-time constants.
     // This wave's 32 query rows stream into stage 1 (free until tile 1 streams in) by DMA,
@@ -1012,27 +1076,30 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
     // B-operand layout exactly as the K operand is.  Rows past the sequence repeat its last
     // row (finite data, their outputs are never stored).
     uint8_t* qbuf = (wave < 2 ? lds_k1 : lds_v1) + (wave & 1) * (32 * kTileRowBytes);
-    if (r0 < qlen) {
+    if (r0 < rows) {
 #pragma unroll
       for (int grp = 0; grp < 2; ++grp) {
         const int g0 = r0 + 16 * grp;
-        const int gk = min(g0, qlen - 1);
+        const int t0 = uniform(tok_of(min(g0, rows - 1)));  // token of the group's first row
+        // 16 rows lie within 15 / pack + 1 tokens after t0 (host: a span below 2^31 bytes)
         const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(p.q + (qstart + gk) * p.q_tok + (int64_t)h * p.q_head), 0,
-            (int)((15 * p.q_tok + D) * 2), kBufferWord3);
+            (void*)(p.q + (qstart + t0) * p.q_tok + (int64_t)h * p.q_head), 0, p.q_span,
+            kBufferWord3);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int r = 4 * i + ld_sub;
-          const int dr = min(g0 + r, qlen - 1) - gk;
+          const int r = min(g0 + 4 * i + ld_sub, rows - 1);
+          const int t = tok_of(r);
           if (kChunks == 16 || chunk_ok[i])
-            lds_dma16(rq, (uint32_t)(dr * p.q_tok + 8 * (ld_pc ^ tile_swz(r))) * 2u,
+            lds_dma16(rq,
+                      (uint32_t)((t - t0) * p.q_tok + (r - t * pack) * p.q_head +
+                                 8 * (ld_pc ^ tile_swz(4 * i + ld_sub))) * 2u,
                       qbuf + grp * 16 * kTileRowBytes + i * 1024);
         }
       }
     }
-    BlkT blk_nxt = block_of(0);
-    issue_tile(0, 0, blk_nxt);
-    if (kBlockN < n_end) blk_nxt = block_of(kBlockN);
+    BlkT blk_nxt = block_of(n_begin);
+    issue_tile(n_begin, 0, blk_nxt);
+    if (n_begin + kBlockN < n_stop) blk_nxt = block_of(n_begin + kBlockN);
     __builtin_amdgcn_s_waitcnt(0);
 #pragma unroll
     for (int kk = 0; kk < DK; ++kk)
@@ -1041,15 +1108,15 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
       constexpr int kStage = decltype(stage_c)::value;
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
-      if (n0 + kBlockN < n_end) {
+      if (n0 + kBlockN < n_stop) {
         issue_tile(n0 + kBlockN, kStage ^ 1, blk_nxt);
-        if (n0 + 2 * kBlockN < n_end) blk_nxt = block_of(n0 + 2 * kBlockN);
+        if (n0 + 2 * kBlockN < n_stop) blk_nxt = block_of(n0 + 2 * kBlockN);
       }
       if (n0 < wave_kend) compute_tile(n0, kStage);
     };
-    for (int n0 = 0; n0 < n_end; n0 += 2 * kBlockN) {
+    for (int n0 = n_begin; n0 < n_stop; n0 += 2 * kBlockN) {
       step(n0, std::integral_constant<int, 0>());
-      if (n0 + kBlockN < n_end) step(n0 + kBlockN, std::integral_constant<int, 1>());
+      if (n0 + kBlockN < n_stop) step(n0 + kBlockN, std::integral_constant<int, 1>());
     }
   }
 
@@ -1059,8 +1126,26 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
   const float lt = kSumRow ? __shfl(oacc[DT - 1][8], col, kWave)
                            : l_run + __shfl_xor(l_run, 32, kWave);
   if (!row_ok) return;
+  if constexpr (SPLIT) {
+    if (ranges > 1) {  // un-normalised, for prefill_merge_kernel
+      const int64_t prow =
+          ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kBlockM + (qrow - m0);
+      float* po = p.part_o + prow * D;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int d = 32 * dt + 8 * g + 4 * half;
+          if (d < D)
+            *reinterpret_cast<f32x4_t*>(po + d) = f32x4_t{oacc[dt][4 * g], oacc[dt][4 * g + 1],
+                                                          oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]};
+        }
+      if (half == 0) *reinterpret_cast<float2*>(p.part_ml + 2 * prow) = make_float2(m_run, lt);
+      return;
+    }
+  }
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
-  bf16_t* op = p.o + (qstart + qrow) * p.o_tok + (int64_t)h * p.o_head;
+  bf16_t* op = p.o + (qstart + qtok) * p.o_tok + (int64_t)(h + qhead) * p.o_head;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
@@ -1076,6 +1161,84 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
   }
 }
 
+// Merges the key ranges' partials of every row that has more than one (SPLIT): D / 4 lanes a
+// row (four dims each), the workgroup's rows kMergeRows at a time over grid y.
+constexpr int kMergeRows = 8;
+
+template <int D, bool PAGED>
+__global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillParams p) {
+  constexpr int kLanes = 32;  // per row; D / 4 of them hold dims
+  int seq, h, mb;
+  if (!map_workgroup<PAGED>(p, seq, h, mb)) return;
+  const int qlen = p.q_len[seq];
+  const int pack = p.pack;
+  const int rows = qlen * pack;
+  const int m0 = mb * kBlockM;
+  if (m0 >= rows) return;
+  int klen;
+  if constexpr (PAGED) {
+    int64_t c = p.ctx_len[seq];
+    const int64_t cap = (int64_t)p.max_blocks * p.bs;
+    klen = (int)(c < 0 ? 0 : (c > cap ? cap : c));
+  } else {
+    klen = p.k_len[seq];
+  }
+  auto tok_of = [&](int r) { return pack == 1 ? r : key_block(r, p.pack_magic, p.pack_shift); };
+  const int q_pos0 = p.causal == NIA_CAUSAL_BOTTOM_RIGHT ? klen - qlen : 0;
+  int n_end = klen;
+  if (p.causal != NIA_CAUSAL_NONE)
+    n_end = min(klen, q_pos0 + tok_of(min(m0 + kBlockM, rows) - 1) + 1);
+  const int ranges = key_ranges((max(n_end, 0) + kBlockN - 1) / kBlockN, p.splits);
+  if (ranges == 1) return;  // written by the prefill kernel
+  const int d = 4 * (threadIdx.x % kLanes);
+  const int r_end = min(rows - m0, ((int)blockIdx.y + 1) * kMergeRows);
+  const int64_t step = (int64_t)gridDim.x * kBlockM;  // rows between ranges
+  for (int r = blockIdx.y * kMergeRows + threadIdx.x / kLanes; r < r_end;
+       r += kPrefillThreads / kLanes) {
+    const int64_t prow = (int64_t)blockIdx.x * kBlockM + r;
+    const float2* ml = reinterpret_cast<const float2*>(p.part_ml);
+    const bool has = d < D;
+    float m = -INFINITY, l = 0.f;
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr int kAhead = 8;  // ranges loaded together
+    for (int s0 = 0; s0 < ranges; s0 += kAhead) {
+      float2 st[kAhead];
+      f32x4_t o[kAhead];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        st[i] = make_float2(-INFINITY, 0.f);
+        o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (s0 + i < ranges) {
+          const int64_t pr = (s0 + i) * step + prow;
+          st[i] = ml[pr];
+          if (has) o[i] = *reinterpret_cast<const f32x4_t*>(p.part_o + pr * D + d);
+        }
+      }
+      float mn = m;
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) mn = fmaxf(mn, st[i].x);
+      if (mn == -INFINITY) continue;  // no visible key so far
+      const float corr = m == -INFINITY ? 0.f : fast_exp2(m - mn);
+      l *= corr;
+      acc *= corr;
+      m = mn;
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const float w = st[i].x == -INFINITY ? 0.f : fast_exp2(st[i].x - mn);
+        l = fmaf(st[i].y, w, l);
+        if (w > 0.f) acc += o[i] * w;
+      }
+    }
+    if (!has) continue;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const int tok = tok_of(m0 + r);
+    bf16_t* op = p.o + (p.q_start[seq] + (int64_t)tok) * p.o_tok +
+                 (int64_t)(h * pack + m0 + r - tok * pack) * p.o_head + d;
+    *reinterpret_cast<uint2*>(op) =
+        make_uint2(pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv));
+  }
+}
+
 constexpr int64_t kMaxRowStride = (int64_t)1 << 26;  // elements
 
 // The register-staged kernel: paged calls whose block size is not a power of two take the
@@ -1088,11 +1251,83 @@ void launch_staged(const PrefillParams& p, dim3 grid, hipStream_t s) {
     nia_launch((prefill_kernel<D, PAGED>), grid, dim3(kPrefillThreads), s, p);
 }
 
+// Bytes that 16 consecutive packed rows of q span from the first one's token, head 0 of the
+// group: at most 15 / pack + 1 tokens further (one token's rows may straddle two groups).
+int64_t q_span_bytes(const PrefillParams& p, int32_t pack, int head_dim) {
+  const int64_t toks = pack == 1 ? 15 : 15 / pack + 1;
+  return 2 * (toks * p.q_tok + (pack - 1) * p.q_head + head_dim);
+}
+
+// Key ranges per m-block for a grid of nwg workgroups whose m-blocks have at most `tiles` key
+// tiles.  A lone workgroup takes about 1.1 us a tile, and the fp32 partials of a full chip's
+// 512 workgroups about 13.6 us to write and read back, so n ranges cost 1.1 tiles / n +
+// 13.6 n nwg / 512 us: least at n = sqrt(41 tiles / nwg).  At most what the chip holds at
+// once (two workgroups a CU), and none where fewer than kSplitGain tiles are saved (the
+// second launch).  A 64-row chunk after 8000 keys (32 and 8 heads) 145 us uncut, 30 in 31
+// ranges, 26 in 15; 24 rows after 16000 keys 279 -> 26; eight 40-row chunks after 500-8192
+// keys 139 -> 75; 1024 rows after 12000 keys 242 -> 216.  Top-left causal calls stay uncut:
+// their m-blocks average half the longest one's tiles, and a prompt of 2000 tokens (16 and 8
+// heads) in two ranges ran 42-44 us, uncut 38.
+constexpr int kSplitSlots = 512;
+constexpr int kSplitMax = 32;
+constexpr int kSplitGain = 12;
+
+int32_t split_count(int64_t nwg, int64_t tiles, int32_t causal) {
+  if (causal == NIA_CAUSAL_TOP_LEFT) return 1;
+  int64_t n = kSplitSlots / nwg;
+  if (n > kSplitMax) n = kSplitMax;
+  if (n > tiles / kSplitMinTiles) n = tiles / kSplitMinTiles;
+  while (n > 1 && n * n * nwg > 41 * tiles) --n;
+  return n < 2 || tiles * (n - 1) < kSplitGain * n ? 1 : (int32_t)n;
+}
+
+size_t split_bytes(int64_t nwg, int32_t splits, int head_dim) {
+  return splits > 1 ? (size_t)nwg * splits * kBlockM * ((size_t)head_dim + 2) * sizeof(float) : 0;
+}
+
+// Rows per item and m-blocks.  A KV head's query heads are packed into the rows where that
+// takes fewer 128-row blocks than a block of its own for each head's remainder: a 40-row
+// chunk of 4 heads is 2 blocks instead of 4.  Where the count is the same the heads keep
+// their own blocks (packed, a prompt of 1531 tokens ran 34.9 instead of 34.2 us: each lane
+// divides its rows).
+void set_rows(PrefillParams& p, int max_q_len, bool packable) {
+  const int64_t per_head = ((int64_t)max_q_len + kBlockM - 1) / kBlockM;
+  const int64_t all = ((int64_t)max_q_len * p.group + kBlockM - 1) / kBlockM;
+  const bool packed = packable && all < per_head * p.group &&
+                      (int64_t)max_q_len * p.group <= INT32_MAX;
+  p.pack = packed ? p.group : 1;
+  p.map_group = packed ? 1 : p.group;
+  p.num_m_blocks = (int32_t)(packed ? all : per_head);
+  block_divisor(p.pack, p.pack_magic, p.pack_shift);
+}
+
+// The workgroups of a packed or unpacked grid.
+int64_t grid_size(const PrefillParams& p) {
+  const int64_t levels =
+      p.map_group > 1 || p.order_by_len
+          ? p.num_m_blocks
+          : ((int64_t)p.num_m_blocks + kLevelRun - 1) / kLevelRun * kLevelRun;
+  return (int64_t)kXcds * p.groups_per_xcd * p.map_group * levels;
+}
+
+// Caller memory for the key ranges' partials, and the longest key run (a bound).
+struct SplitArgs {
+  void* ws = nullptr;
+  size_t bytes = 0;
+  int64_t max_k_len = 0;
+};
+
+template <int D, bool PAGED>
+void launch_dma_split(const PrefillParams& p, dim3 grid, hipStream_t s) {
+  nia_launch((prefill_dma_kernel<D, PAGED, false, false, false, false, false, true, true>),
+             dim3(grid.x, (unsigned)p.splits), dim3(kPrefillThreads), s, p);
+  nia_launch((prefill_merge_kernel<D, PAGED>), dim3(grid.x, kBlockM / kMergeRows),
+             dim3(kPrefillThreads), s, p);
+}
+
 template <bool PAGED, bool BIAS = false>
-int launch_prefill(const PrefillParams& p, int head_dim, int num_seqs, hipStream_t s) {
-  const int64_t nwg = (int64_t)kXcds * p.groups_per_xcd * p.group * p.num_m_blocks;
-  if (nwg >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
-  const dim3 grid((unsigned)nwg);
+int launch_prefill(PrefillParams& p, int head_dim, int max_q_len, hipStream_t s,
+                   const SplitArgs& sp = SplitArgs()) {
   // The DMA kernel needs 4-row groups inside one KV block (block sizes that are multiples of
   // 4; 16-row groups for the shift and DIV forms, 4-row ones for QUAD) and 32-bit lane
   // offsets; the register-staged kernel serves the rest.
@@ -1101,10 +1336,30 @@ int launch_prefill(const PrefillParams& p, int head_dim, int num_seqs, hipStream
                              : (p.k_tok >= 0 && p.k_tok < kMaxRowStride && p.v_tok >= 0 &&
                                 p.v_tok < kMaxRowStride));
   if (BIAS && !dma_ok) return NIA_ERR_UNSUPPORTED;
+  // packed rows: the lane offsets must fit 32 bits and not be negative
+  const bool plain = !BIAS && dma_ok && (!PAGED || (p.bs % 16 == 0 && (p.bs & (p.bs - 1)) == 0));
+  set_rows(p, max_q_len,
+           plain && p.q_head >= 0 && p.q_head < kMaxRowStride &&
+               q_span_bytes(p, p.group, head_dim) <= INT32_MAX);
+  p.q_span = (int32_t)q_span_bytes(p, p.pack, head_dim);
+  const int64_t nwg = grid_size(p);
+  if (nwg >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)nwg);
+  p.splits = 1;
+  if (sp.ws && plain) {
+    const int32_t n = split_count(nwg, (sp.max_k_len + kBlockN - 1) / kBlockN, p.causal);
+    if (n > 1 && split_bytes(nwg, n, head_dim) <= sp.bytes) {
+      p.splits = n;
+      p.part_o = (float*)sp.ws;
+      p.part_ml = p.part_o + (size_t)nwg * n * kBlockM * head_dim;
+    }
+  }
   switch (head_dim) {
 #define NIA_PREFILL_CASE(DD)                                                                 \
   case DD:                                                                                   \
-    if (BIAS)                                                                                \
+    if (!BIAS && p.splits > 1)                                                               \
+      launch_dma_split<DD, PAGED>(p, grid, s);                                               \
+    else if (BIAS)                                                                           \
       nia_launch((prefill_dma_kernel<DD, false, false, true>), grid, dim3(kPrefillThreads),  \
                  s, p);                                                                      \
     else if (dma_ok && PAGED && p.bs % 16 != 0)                                              \
@@ -1113,6 +1368,9 @@ int launch_prefill(const PrefillParams& p, int head_dim, int num_seqs, hipStream
     else if (dma_ok && PAGED && (p.bs & (p.bs - 1)))                                         \
       nia_launch((prefill_dma_kernel<DD, PAGED, false, false, false, PAGED>), grid,          \
                  dim3(kPrefillThreads), s, p);                                               \
+    else if (p.pack > 1)                                                                     \
+      nia_launch((prefill_dma_kernel<DD, PAGED, false, false, false, false, false, true>),   \
+                 grid, dim3(kPrefillThreads), s, p);                                         \
     else if (dma_ok)                                                                         \
       nia_launch((prefill_dma_kernel<DD, PAGED>), grid, dim3(kPrefillThreads), s, p);        \
     else                                                                                     \
@@ -1152,7 +1410,8 @@ int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride
                       int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
                       int32_t num_kv_heads, int32_t head_dim, float scale, int32_t causal,
                       int32_t dtype, const float* mask, int64_t mask_seq_stride,
-                      int64_t mask_head_stride, int64_t mask_q_stride, void* stream) {
+                      int64_t mask_head_stride, int64_t mask_q_stride, void* stream,
+                      const SplitArgs& split = SplitArgs()) {
   if (num_seqs < 0 || max_q_len < 0 || num_heads <= 0 || num_kv_heads <= 0 ||
       num_heads % num_kv_heads != 0)
     return NIA_ERR_INVALID_ARGUMENT;
@@ -1225,7 +1484,6 @@ int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride
   p.num_heads = num_heads;
   p.num_kv_heads = num_kv_heads;
   p.group = num_heads / num_kv_heads;
-  p.num_m_blocks = (max_q_len + kBlockM - 1) / kBlockM;
   p.num_seqs = num_seqs;
   p.groups_per_xcd = (num_seqs * num_kv_heads + kXcds - 1) / kXcds;
   p.causal = causal;
@@ -1239,7 +1497,7 @@ int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride
     p.bias_head = mask_head_stride;
     p.bias_q = mask_q_stride;
     p.scale = scale;
-    return launch_prefill<false, true>(p, head_dim, num_seqs, (hipStream_t)stream);
+    return launch_prefill<false, true>(p, head_dim, max_q_len, (hipStream_t)stream);
   }
   // Short unmasked sequences with one query head per KV head (the vision windows):
   // two heads per workgroup, 64 rows each (see prefill_dma_kernel's PAIR mode).
@@ -1249,6 +1507,7 @@ int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride
     p.num_kv_heads = num_kv_heads / 2;  // the workgroup map numbers head pairs
     p.groups_per_xcd = (num_seqs * p.num_kv_heads + kXcds - 1) / kXcds;
     p.num_m_blocks = 1;
+    p.pack = 1;
     const int64_t nwg = (int64_t)kXcds * ((num_seqs + kXcds - 1) / kXcds) * p.num_kv_heads;
     if (nwg >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
@@ -1268,7 +1527,7 @@ int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride
     }
     return hipGetLastError() == hipSuccess ? NIA_OK : NIA_ERR_LAUNCH;
   }
-  return launch_prefill<false>(p, head_dim, num_seqs, (hipStream_t)stream);
+  return launch_prefill<false>(p, head_dim, max_q_len, (hipStream_t)stream, split);
 }
 
 }  // namespace
@@ -1307,7 +1566,9 @@ extern "C" int32_t nia_prefill_masked(void* out, int64_t out_tok_stride, int64_t
                        mask_q_stride, stream);
 }
 
-extern "C" int32_t nia_prefill_paged(void* out, int64_t out_tok_stride, int64_t out_head_stride,
+namespace {
+
+int32_t prefill_paged_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride,
                                      const void* q, int64_t q_tok_stride, int64_t q_head_stride,
                                      const void* k_cache, const void* v_cache,
                                      const int32_t* block_tables, int32_t bt_stride,
@@ -1316,7 +1577,7 @@ extern "C" int32_t nia_prefill_paged(void* out, int64_t out_tok_stride, int64_t 
                                      int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
                                      int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
                                      int64_t num_blocks, float scale, int32_t causal,
-                                     int32_t dtype, void* stream) {
+                                     int32_t dtype, void* stream, const SplitArgs& split) {
   if (num_seqs < 0 || max_q_len < 0 || num_heads <= 0 || num_kv_heads <= 0 ||
       num_heads % num_kv_heads != 0 || max_blocks_per_seq < 0 ||
       bt_stride < max_blocks_per_seq || num_blocks < 0)
@@ -1396,11 +1657,86 @@ extern "C" int32_t nia_prefill_paged(void* out, int64_t out_tok_stride, int64_t 
   p.num_heads = num_heads;
   p.num_kv_heads = num_kv_heads;
   p.group = num_heads / num_kv_heads;
-  p.num_m_blocks = (max_q_len + kBlockM - 1) / kBlockM;
   p.num_seqs = num_seqs;
   p.groups_per_xcd = (num_seqs * num_kv_heads + kXcds - 1) / kXcds;
   p.causal = causal;
   p.scale_log2 = scale * kLog2e;
   p.order_by_len = causal != NIA_CAUSAL_TOP_LEFT && num_seqs <= kOrderMaxSeqs;
-  return launch_prefill<true>(p, head_dim, num_seqs, (hipStream_t)stream);
+  return launch_prefill<true>(p, head_dim, max_q_len, (hipStream_t)stream, split);
+}
+
+SplitArgs split_args(void* ws, size_t bytes, int64_t max_k_len) {
+  SplitArgs a;
+  a.ws = (uintptr_t)ws % 256 ? nullptr : ws;
+  a.bytes = bytes;
+  a.max_k_len = max_k_len;
+  return a;
+}
+
+}  // namespace
+
+extern "C" int32_t nia_prefill_paged(void* out, int64_t out_tok_stride, int64_t out_head_stride,
+                                     const void* q, int64_t q_tok_stride, int64_t q_head_stride,
+                                     const void* k_cache, const void* v_cache,
+                                     const int32_t* block_tables, int32_t bt_stride,
+                                     int32_t max_blocks_per_seq, const int32_t* q_start,
+                                     const int32_t* q_len, const int64_t* context_lens,
+                                     int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
+                                     int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                                     int64_t num_blocks, float scale, int32_t causal,
+                                     int32_t dtype, void* stream) {
+  return prefill_paged_entry(out, out_tok_stride, out_head_stride, q, q_tok_stride, q_head_stride,
+                             k_cache, v_cache, block_tables, bt_stride, max_blocks_per_seq,
+                             q_start, q_len, context_lens, num_seqs, max_q_len, num_heads,
+                             num_kv_heads, head_dim, block_size, num_blocks, scale, causal, dtype,
+                             stream, SplitArgs());
+}
+
+// ---- the same with caller memory for key ranges ------------------------------------------
+
+extern "C" size_t nia_prefill_split_workspace_size(int32_t num_seqs, int32_t max_q_len,
+                                                   int64_t max_k_len, int32_t num_heads,
+                                                   int32_t num_kv_heads, int32_t head_dim,
+                                                   int32_t causal, int32_t dtype) {
+  if (num_seqs <= 0 || max_q_len <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 ||
+      max_k_len <= 0 || num_heads % num_kv_heads != 0 || dtype != NIA_DTYPE_BF16)
+    return 0;
+  PrefillParams p{};
+  p.group = num_heads / num_kv_heads;
+  set_rows(p, max_q_len, true);
+  p.groups_per_xcd = (int32_t)(((int64_t)num_seqs * num_kv_heads + kXcds - 1) / kXcds);
+  p.order_by_len = causal != NIA_CAUSAL_TOP_LEFT && num_seqs <= kOrderMaxSeqs;
+  const int64_t nwg = grid_size(p);
+  return split_bytes(nwg, split_count(nwg, (max_k_len + kBlockN - 1) / kBlockN, causal), head_dim);
+}
+
+extern "C" int32_t nia_prefill_split(
+    void* out, int64_t out_tok_stride, int64_t out_head_stride, const void* q,
+    int64_t q_tok_stride, int64_t q_head_stride, const void* k, int64_t k_tok_stride,
+    int64_t k_head_stride, const void* v, int64_t v_tok_stride, int64_t v_head_stride,
+    const int32_t* q_start, const int32_t* q_len, const int32_t* k_start, const int32_t* k_len,
+    int32_t num_seqs, int32_t max_q_len, int32_t num_heads, int32_t num_kv_heads,
+    int32_t head_dim, float scale, int32_t causal, int32_t dtype, int64_t max_k_len,
+    void* workspace, size_t workspace_bytes, void* stream) {
+  return prefill_entry(out, out_tok_stride, out_head_stride, q, q_tok_stride, q_head_stride, k,
+                       k_tok_stride, k_head_stride, v, v_tok_stride, v_head_stride, q_start,
+                       q_len, k_start, k_len, num_seqs, max_q_len, num_heads, num_kv_heads,
+                       head_dim, scale, causal, dtype, nullptr, 0, 0, 0, stream,
+                       split_args(workspace, workspace_bytes, max_k_len));
+}
+
+extern "C" int32_t nia_prefill_paged_split(
+    void* out, int64_t out_tok_stride, int64_t out_head_stride, const void* q,
+    int64_t q_tok_stride, int64_t q_head_stride, const void* k_cache, const void* v_cache,
+    const int32_t* block_tables, int32_t bt_stride, int32_t max_blocks_per_seq,
+    const int32_t* q_start, const int32_t* q_len, const int64_t* context_lens, int32_t num_seqs,
+    int32_t max_q_len, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+    int32_t block_size, int64_t num_blocks, float scale, int32_t causal, int32_t dtype,
+    void* workspace, size_t workspace_bytes, void* stream) {
+  return prefill_paged_entry(
+      out, out_tok_stride, out_head_stride, q, q_tok_stride, q_head_stride, k_cache, v_cache,
+      block_tables, bt_stride, max_blocks_per_seq, q_start, q_len, context_lens, num_seqs,
+      max_q_len, num_heads, num_kv_heads, head_dim, block_size, num_blocks, scale, causal, dtype,
+      stream,
+      split_args(workspace, workspace_bytes, (int64_t)max_blocks_per_seq * block_size));
 }

@@ -467,6 +467,20 @@ def _i32(name: str, t: torch.Tensor, n: int) -> torch.Tensor:
     return t.to(torch.int32).contiguous()
 
 
+# Calls with fewer keys a sequence, or more query rows, are not worth cutting
+# (nia_prefill_split_workspace_size says which of the others are): they skip the question.
+_SPLIT_MIN_KEYS, _SPLIT_MAX_ROWS = 768, 256 * 128
+
+
+def _split_workspace(n, max_q_len, keys, h, hkv, d, causal, dt, dev) -> Optional[torch.Tensor]:
+    """Memory for the key ranges of a prefill call with few query rows over long keys (the
+    callers ask _SPLIT_MIN_KEYS and _SPLIT_MAX_ROWS first), or None when the call runs uncut.  Allocated per call: the caching allocator then orders
+    its reuse by stream, under graph capture too."""
+    nbytes = _lib.load().nia_prefill_split_workspace_size(n, max_q_len, keys, h, hkv, d, causal,
+                                                          dt)
+    return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+
+
 def prefill(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -528,6 +542,23 @@ def prefill(
             m4.data_ptr(), *strides, _stream(dev),
         )
         _lib.check("nia_prefill_masked", st)
+        return out
+    ws = None
+    keys = k.shape[0]  # bounds every sequence's keys
+    if causal != CAUSAL_TOP_LEFT and keys >= n * _SPLIT_MIN_KEYS and dt == _lib.DTYPE_BF16 and \
+            n * h * max_q_len <= _SPLIT_MAX_ROWS:
+        ws = _split_workspace(n, int(max_q_len), keys, h, hkv, d, int(causal), dt, dev)
+    if ws is not None:
+        st = _lib.load().nia_prefill_split(
+            out.data_ptr(), out.stride(0), out.stride(1),
+            q.data_ptr(), q.stride(0), q.stride(1),
+            k.data_ptr(), k.stride(0), k.stride(1),
+            v.data_ptr(), v.stride(0), v.stride(1),
+            qs.data_ptr(), ql.data_ptr(), ks.data_ptr(), kl.data_ptr(),
+            n, int(max_q_len), h, hkv, d, _default_scale(d, scale), int(causal), dt, keys,
+            ws.data_ptr(), ws.numel(), _stream(dev),
+        )
+        _lib.check("nia_prefill_split", st)
         return out
     lib = _lib.calls()
     st = lib.nia_prefill(
@@ -688,6 +719,23 @@ def prefill_paged(
     elif out.shape != q.shape or out.dtype != q.dtype:
         raise ValueError("out must match q's shape and dtype")
     _last_contig("out", out)
+    ws = None
+    keys = block_tables.shape[1] * bs
+    if keys >= _SPLIT_MIN_KEYS and dt == _lib.DTYPE_BF16 and causal != CAUSAL_TOP_LEFT and \
+            n * h * max_q_len <= _SPLIT_MAX_ROWS:
+        ws = _split_workspace(n, int(max_q_len), keys, h, hkv, d, int(causal), dt, dev)
+    if ws is not None:
+        st = _lib.load().nia_prefill_paged_split(
+            out.data_ptr(), out.stride(0), out.stride(1),
+            q.data_ptr(), q.stride(0), q.stride(1),
+            k_cache.data_ptr(), v_cache.data_ptr(),
+            block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1],
+            qs.data_ptr(), ql.data_ptr(), context_lens.data_ptr(),
+            n, int(max_q_len), h, hkv, d, bs, nb, _default_scale(d, scale), int(causal), dt,
+            ws.data_ptr(), ws.numel(), _stream(dev),
+        )
+        _lib.check("nia_prefill_paged_split", st)
+        return out
     lib = _lib.calls()
     st = lib.nia_prefill_paged(
         out.data_ptr(), out.stride(0), out.stride(1),
@@ -735,7 +783,8 @@ def _prefill_paged_fp8(q, k_cache, v_cache, block_tables, q_start, q_len, contex
         raise ValueError("out must match q's shape and dtype")
     _last_contig("out", out)
     lib = _lib.load()
-    ws = torch.empty(lib.nia_prefill_paged_fp8_workspace_size(n, hkv, mb, bs, d),
+    ws = torch.empty(lib.nia_prefill_paged_fp8_workspace_size(n, int(max_q_len), h, hkv, mb, bs,
+                                                              d, int(causal)),
                      dtype=torch.uint8, device=dev)
     st = lib.nia_prefill_paged_fp8(
         out.data_ptr(), out.stride(0), out.stride(1), q.data_ptr(), q.stride(0), q.stride(1),
