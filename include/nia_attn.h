@@ -236,7 +236,7 @@ int32_t nia_prefill_paged(void* out, int64_t out_tok_stride, int64_t out_head_st
  * side by side and merges their fp32 partials from the workspace in a second launch.
  * `max_k_len`: a bound of the sequences' key counts (paged calls: the table width).
  * `workspace`: 256-byte aligned device memory; nia_prefill_split_workspace_size gives the
- * bytes that a call can use, 0 where it would not cut (fp32, enough rows, short keys).  A
+ * bytes that a call can use, 0 where it would not cut (enough rows, short keys).  A
  * null, unaligned or smaller workspace runs the call uncut.  Nothing in it needs
  * initialising; calls one after another on a stream may share it.
  */

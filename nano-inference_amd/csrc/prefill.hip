@@ -1458,7 +1458,8 @@ int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride
     f.bias_seq = mask_seq_stride;
     f.bias_head = mask_head_stride;
     f.bias_q = mask_q_stride;
-    return launch_prefill_f32(f, false, head_dim, num_seqs, max_q_len, (hipStream_t)stream);
+    return launch_prefill_f32(f, false, head_dim, num_seqs, max_q_len, (hipStream_t)stream,
+                              kElemF32, split.ws, split.bytes, split.max_k_len);
   }
   if (dtype != NIA_DTYPE_BF16) return NIA_ERR_UNSUPPORTED;
   if (!vec_ok(q, q_tok_stride, q_head_stride) || !vec_ok(k, k_tok_stride, k_head_stride) ||
@@ -1628,7 +1629,8 @@ int32_t prefill_paged_entry(void* out, int64_t out_tok_stride, int64_t out_head_
     f.causal = causal;
     f.scale_log2 = (double)scale * 1.4426950408889634;
     return launch_prefill_f32(f, true, head_dim, num_seqs, max_q_len, (hipStream_t)stream,
-                              f32 ? kElemF32 : kElemBf16);
+                              f32 ? kElemF32 : kElemBf16, split.ws, split.bytes,
+                              split.max_k_len);
   }
   // bf16, block size >= 2: a key's block is a multiply-shift division (block_divisor); block
   // sizes that are multiples of 16 keep a wave's 16-row DMA group in one block
@@ -1699,8 +1701,12 @@ extern "C" size_t nia_prefill_split_workspace_size(int32_t num_seqs, int32_t max
                                                    int32_t num_kv_heads, int32_t head_dim,
                                                    int32_t causal, int32_t dtype) {
   if (num_seqs <= 0 || max_q_len <= 0 || num_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0 ||
-      max_k_len <= 0 || num_heads % num_kv_heads != 0 || dtype != NIA_DTYPE_BF16)
+      max_k_len <= 0 || num_heads % num_kv_heads != 0)
     return 0;
+  if (dtype == NIA_DTYPE_F32)
+    return prefill_f32_split_bytes(num_seqs, max_q_len, max_k_len, num_heads, num_kv_heads,
+                                   head_dim);
+  if (dtype != NIA_DTYPE_BF16) return 0;
   PrefillParams p{};
   p.group = num_heads / num_kv_heads;
   set_rows(p, max_q_len, true);

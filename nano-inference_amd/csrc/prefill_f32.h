@@ -36,13 +36,28 @@ struct PrefillF32Params {
   int32_t causal;
   int32_t decode;  // one query row per sequence: row s of q / o (q_start, q_len unused)
   double scale_log2;
+  // set by launch_prefill_f32: r / group = key_block(r, magic, shift) for group > 1, the grid
+  int32_t num_seqs;
+  uint32_t group_magic;
+  int32_t group_shift;
+  int32_t num_m_blocks, level_run, groups_per_xcd;
+  // key ranges per row block at most (grid y) and their partials, per (range, workgroup, row)
+  int32_t splits;
+  double* part_m;
+  float* part_l;
+  float* part_o;
   // additive mask (contiguous mode, optional): bias[s * bias_seq + h * bias_head +
   // i * bias_q + j] joins the scaled score of query row i and key j
   const float* bias;
   int64_t bias_seq, bias_head, bias_q;
 };
 
-// Grid (m-blocks of 64 rows, heads, sequences); returns an NIA_* status.  `elem` other
+// Row blocks of 64 packed rows (query token, head of the group); returns an NIA_* status.  `elem` other
 // than kElemF32 takes a paged cache (fp8: head_dim 128, both scale arrays).
-int32_t launch_prefill_f32(const PrefillF32Params& p, bool paged, int head_dim, int num_seqs,
-                           int max_q_len, hipStream_t stream, int elem = kElemF32);
+int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int num_seqs,
+                           int max_q_len, hipStream_t stream, int elem = kElemF32,
+                           void* ws = nullptr, size_t ws_bytes = 0, int64_t max_k_len = 0);
+
+// Workspace bytes of a call that would cut its row blocks' keys into ranges, or 0.
+size_t prefill_f32_split_bytes(int32_t num_seqs, int64_t max_q_len, int64_t max_k_len,
+                               int32_t num_heads, int32_t num_kv_heads, int head_dim);

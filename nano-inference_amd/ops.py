@@ -467,9 +467,12 @@ def _i32(name: str, t: torch.Tensor, n: int) -> torch.Tensor:
     return t.to(torch.int32).contiguous()
 
 
-# Calls with fewer keys a sequence, or more query rows, are not worth cutting
+# bf16 calls with fewer keys a sequence, or more query rows, are not worth cutting
 # (nia_prefill_split_workspace_size says which of the others are): they skip the question.
 _SPLIT_MIN_KEYS, _SPLIT_MAX_ROWS = 768, 256 * 128
+# fp32 calls of more rows (640 blocks of 64) fill the chip evenly enough uncut: four prompts
+# of 1000 tokens of 16 heads 279 us uncut, 315 in ranges of 256 keys; one 146 and 114.
+_SPLIT_MAX_ROWS_F32 = 640 * 64
 
 
 def _split_workspace(n, max_q_len, keys, h, hkv, d, causal, dt, dev) -> Optional[torch.Tensor]:
@@ -545,7 +548,12 @@ def prefill(
         return out
     ws = None
     keys = k.shape[0]  # bounds every sequence's keys
-    if causal != CAUSAL_TOP_LEFT and keys >= n * _SPLIT_MIN_KEYS and dt == _lib.DTYPE_BF16 and \
+    if dt != _lib.DTYPE_BF16:
+        if q.shape[0] * h <= _SPLIT_MAX_ROWS_F32:
+            if causal == CAUSAL_TOP_LEFT:  # its rows see no key past their own position
+                keys = min(keys, int(max_q_len))
+            ws = _split_workspace(n, int(max_q_len), keys, h, hkv, d, int(causal), dt, dev)
+    elif causal != CAUSAL_TOP_LEFT and keys >= n * _SPLIT_MIN_KEYS and \
             n * h * max_q_len <= _SPLIT_MAX_ROWS:
         ws = _split_workspace(n, int(max_q_len), keys, h, hkv, d, int(causal), dt, dev)
     if ws is not None:
@@ -721,8 +729,9 @@ def prefill_paged(
     _last_contig("out", out)
     ws = None
     keys = block_tables.shape[1] * bs
-    if keys >= _SPLIT_MIN_KEYS and dt == _lib.DTYPE_BF16 and causal != CAUSAL_TOP_LEFT and \
-            n * h * max_q_len <= _SPLIT_MAX_ROWS:
+    if q.shape[0] * h <= _SPLIT_MAX_ROWS_F32 if dt != _lib.DTYPE_BF16 else (
+            keys >= _SPLIT_MIN_KEYS and causal != CAUSAL_TOP_LEFT and
+            n * h * max_q_len <= _SPLIT_MAX_ROWS):
         ws = _split_workspace(n, int(max_q_len), keys, h, hkv, d, int(causal), dt, dev)
     if ws is not None:
         st = _lib.load().nia_prefill_paged_split(
