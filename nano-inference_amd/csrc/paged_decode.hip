@@ -31,9 +31,9 @@
 //   (fp8: 128), any G: groups of more than 16 query heads per KV head run as launches of
 //   at most 16 heads each (the MFMA columns), one after another on the stream.
 // fp32 caches (the reference's CPU default; tolerance 1e-5):
-//   head_dim 128, block size 16, G <= 8: paged_decode_partial_kernel, grid (partition,
-//   KV head, sequence); wave w takes blocks w, w + 4, ... of the partition; 32 lanes per
-//   token; q . k is summed in fp64; partials merged by paged_decode_combine_kernel.
+//   head_dim 128, block size 16, G <= 8: paged_decode_f32_kernel, grid (partition, KV head,
+//   sequence); q . k is summed on the fp64 matrix cores; partials merged by
+//   paged_decode_combine_kernel.
 //   Other fp32 shapes run the fp32 prefill kernel with one query row per sequence.
 // Softmax (all): scores in log2 units (scale * log2 e applied in fp32 to the raw
 // scores).  A running max is only raised when a block exceeds it by more than
@@ -96,311 +96,256 @@ struct DecodeParams {
   float* sp_o;      // [grid * wph][2][hg][G][D]
 };
 
-// Element-type specific pieces: how 16 loaded bytes enter a dot product and
-// how they widen to fp32.
-template <typename T>
-struct Elem;
+// ---- fp32 caches: head_dim 128, block size 16, at most 8 query heads per KV head ----------
+// Grid (512-key partition, KV head, sequence); wave w of 8 takes blocks w, w + 8, ... of the
+// partition.  Bound by HBM once the scores are off the vector unit: q . k summed there in fp64
+// over 32 lanes (five exchanges a score) took 47 us with the merge for 16 sequences of 339-2304
+// keys (16 and 8 heads, 164 MB), 77 with 32 and 8 heads, 107 for 8 sequences of 28 and 4
+// heads; now 43, 47 and 22 (32 sequences of 4096 keys stream at 5.7 TB/s; the rest is the
+// start, about 8 us, and the merge's launch, 5).  Eight waves, one workgroup a CU: four waves
+// and three workgroups 51 us, two workgroups in 128 registers 45.
+//   Scores: v_mfma_f64_4x4x4 (16.6 cycles; fp32 inputs widened exactly), four 4 x 4 products
+//   a time: A lane l holds key l % 16 (block (l / 4) % 4 is the keys 4 b .. + 3), dim slot
+//   l / 16; B lane l query head l % 4 of a group of four, the same dim, from LDS in fp64; the
+//   result lane (l / 16, (l / 4) % 4, l % 4) is key 4 ((l / 4) % 4) + l / 16, head l % 4 (pinned
+//   on the device by an in-bounds probe).
+//   Output: O^T += V^T P^T on v_mfma_f32_16x16x4: k step u pairs slot l / 16 with key
+//   4 u + l / 16, whose weight for head l % 16 < 4 lies 4 u lanes up the lane's row of 16: one
+//   DPP rotation, no exchange through LDS.  Columns without a head hold other keys' weights;
+//   they are never read.  Row i of output tile t is dim 64 (t / 4) + 4 i + t % 4, so that one
+//   16-byte load of a V row feeds four tiles.
+//   Each operand of the next block is loaded as soon as this block's has been consumed.
+constexpr int kF32Waves = 8;
+constexpr int kF32Threads = kF32Waves * kWave;
 
-template <>
-struct Elem<bf16_t> {
-  static constexpr int kPerLoad = 8;
-  // q kept as 4 packed bf16 pairs
-  struct QReg {
-    uint32_t w[4];
-  };
-  static NIA_DEVICE void load_q(QReg& r, const bf16_t* p) {
-    const uint4 u = *reinterpret_cast<const uint4*>(p);
-    r.w[0] = u.x; r.w[1] = u.y; r.w[2] = u.z; r.w[3] = u.w;
-  }
-  static NIA_DEVICE float dot(const QReg& q, const uint4& k) {
-    float s = dot2_bf16(q.w[0], k.x, 0.f);
-    s = dot2_bf16(q.w[1], k.y, s);
-    s = dot2_bf16(q.w[2], k.z, s);
-    return dot2_bf16(q.w[3], k.w, s);
-  }
-  static NIA_DEVICE void widen(const uint4& v, float (&f)[8]) {
-    f[0] = bf16_lo(v.x); f[1] = bf16_hi(v.x);
-    f[2] = bf16_lo(v.y); f[3] = bf16_hi(v.y);
-    f[4] = bf16_lo(v.z); f[5] = bf16_hi(v.z);
-    f[6] = bf16_lo(v.w); f[7] = bf16_hi(v.w);
-  }
-  static NIA_DEVICE bf16_t from_f32(float x) { return (bf16_t)x; }
-};
-
-template <>
-struct Elem<float> {
-  static constexpr int kPerLoad = 4;
-  struct QReg {
-    float f[4];
-  };
-  static NIA_DEVICE void load_q(QReg& r, const float* p) {
-    const float4 u = *reinterpret_cast<const float4*>(p);
-    r.f[0] = u.x; r.f[1] = u.y; r.f[2] = u.z; r.f[3] = u.w;
-  }
-  static NIA_DEVICE float dot(const QReg& q, const uint4& k) {
-    float s = q.f[0] * as_f32(k.x);
-    s = fmaf(q.f[1], as_f32(k.y), s);
-    s = fmaf(q.f[2], as_f32(k.z), s);
-    return fmaf(q.f[3], as_f32(k.w), s);
-  }
-  // The lane's share of q . k in fp64: the fp32 path's scores carry no accumulated
-  // rounding (an fp32 sum of 128 products is off by ~1e-7 of the largest partial sum,
-  // which at logits of ~100 nats moves the softmax weights by ~1e-5).
-  static NIA_DEVICE double dot64(const QReg& q, const uint4& k) {
-    double s = (double)q.f[0] * (double)as_f32(k.x);
-    s = fma((double)q.f[1], (double)as_f32(k.y), s);
-    s = fma((double)q.f[2], (double)as_f32(k.z), s);
-    return fma((double)q.f[3], (double)as_f32(k.w), s);
-  }
-  static NIA_DEVICE void widen(const uint4& v, float (&f)[4]) {
-    f[0] = as_f32(v.x); f[1] = as_f32(v.y); f[2] = as_f32(v.z); f[3] = as_f32(v.w);
-  }
-  static NIA_DEVICE float from_f32(float x) { return x; }
-};
-
-// Sum of doubles over aligned groups of N lanes (N a power of two, at most 64).
+// x of the lane N up the row of 16 (wrapping).
 template <int N>
-NIA_DEVICE double group_sum_f64(double x) {
-#pragma unroll
-  for (int off = 1; off < N; off <<= 1) x += __shfl_xor(x, off, kWave);
-  return x;
+NIA_DEVICE float row_up(float x) {
+  if constexpr (N == 0) return x;
+  // row_ror by 16 - N moves lane l + N's value to lane l
+  else return as_f32(__builtin_amdgcn_update_dpp(0, (int)as_u32(x), 0x120 + 16 - N, 0xF, 0xF, false));
 }
 
-// Merge the per-wave softmax states of a workgroup held in LDS and store either the
-// final output (single-partition sequence) or the partition's partial (m, l,
-// un-normalised o) for the combine kernel.  Wave w's o row of head g is at
-// sm_o + w * STRIDE + g * D, its m and l at [w * G + g].  Every thread calls it, after
-// the barrier that follows the stores.
-template <typename T, int D, int G, int STRIDE>
-NIA_DEVICE void merge_lds_and_store(const DecodeParams& p, const float* sm_o, const float* sm_m,
-                                    const float* sm_l, int b, int hk, int part, int nparts) {
-  for (int idx = threadIdx.x; idx < G * D; idx += kDecodeThreads) {
-    const int g = idx / D;
-    const int d = idx - g * D;
-    float mt = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kDecodeWaves; ++w) mt = fmaxf(mt, sm_m[w * G + g]);
-    float lt = 0.f, ot = 0.f;
-#pragma unroll
-    for (int w = 0; w < kDecodeWaves; ++w) {
-      const float mw = sm_m[w * G + g];
-      const float wt = (mw == -INFINITY) ? 0.f : fast_exp2(mw - mt);
-      lt = fmaf(sm_l[w * G + g], wt, lt);
-      ot = fmaf(sm_o[w * STRIDE + g * D + d], wt, ot);
-    }
-    const int h = hk * G + g;
-    if (nparts == 1) {
-      T* out = reinterpret_cast<T*>(p.out) + (int64_t)b * p.out_b + (int64_t)h * p.out_h;
-      out[d] = (T)(lt > 0.f ? ot / lt : 0.f);
-    } else {
-      const int64_t slot = ((int64_t)b * p.num_heads + h) * p.max_parts + part;
-      p.ws_o[slot * D + d] = ot;
-      if (d == 0) {
-        p.ws_ml[slot * 2 + 0] = mt;
-        p.ws_ml[slot * 2 + 1] = lt;
-      }
-    }
-  }
-}
-
-// The per-wave states of the vector-unit loops: on entry the lanes with row == 0 hold
-// o[g][col * EL .. +EL) and every lane holds the wave's m, l.
-template <typename T, int D, int G, int EL>
-NIA_DEVICE void merge_waves_and_store(const DecodeParams& p, const float (&o)[G][EL],
-                                      const float (&m)[G], const float (&l)[G], int row,
-                                      int col, int wave, int b, int hk, int part, int nparts) {
-  __shared__ float sm_o[kDecodeWaves * G * D];
-  __shared__ float sm_m[kDecodeWaves * G];
-  __shared__ float sm_l[kDecodeWaves * G];
-  if (row == 0) {
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-#pragma unroll
-      for (int e = 0; e < EL; ++e) sm_o[(wave * G + g) * D + col * EL + e] = o[g][e];
-      if (col == 0) {
-        sm_m[wave * G + g] = m[g];
-        sm_l[wave * G + g] = l[g];
-      }
-    }
-  }
-  __syncthreads();
-  merge_lds_and_store<T, D, G, G * D>(p, sm_o, sm_m, sm_l, b, hk, part, nparts);
-}
-
-template <typename T, int D, int G, int BS, int PART_BLOCKS>
-__global__ __launch_bounds__(kDecodeThreads) void paged_decode_partial_kernel(DecodeParams p) {
-  using E = Elem<T>;
-  constexpr int EL = E::kPerLoad;        // elements per lane per load
-  constexpr int LPT = D / EL;            // lanes per token row
-  constexpr int TPL = kWave / LPT;       // tokens per wave-wide load
-  constexpr int LOADS = BS / TPL;        // wave-wide loads per block-head
-  static_assert(D % EL == 0 && kWave % LPT == 0 && BS % TPL == 0, "lane layout");
+// CG: groups of four query heads (1 or 2).
+template <int CG, int PART_BLOCKS>
+__global__ __launch_bounds__(kF32Threads, 2) void paged_decode_f32_kernel(DecodeParams p) {
+  constexpr int D = 128, BS = 16, kTiles = D / 16;
   constexpr int PART_TOKENS = PART_BLOCKS * BS;
-
   const int part = blockIdx.x;
   const int hk = blockIdx.y;
   const int b = blockIdx.z;
+  const int G = p.group;
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int row = lane / LPT;
-  const int col = lane % LPT;
+  const int wave = uniform(threadIdx.x / kWave);
+  const int slot = lane >> 4, col = lane & 15;
 
   int64_t ctx64 = p.context_lens[b];
   const int64_t cap = (int64_t)p.max_blocks * BS;
   if (ctx64 > cap) ctx64 = cap;
   const int ctx = ctx64 > 0 ? (int)ctx64 : 0;
-  const int tok_begin = part * PART_TOKENS;
-  if (tok_begin >= ctx) {
+  float* ob = reinterpret_cast<float*>(p.out) + (int64_t)b * p.out_b + (int64_t)hk * G * p.out_h;
+  if (part * PART_TOKENS >= ctx) {
     // Whole workgroup leaves together.  A sequence without keys gets zeros from
     // its first partition.
-    if (part == 0 && ctx == 0) {
-      T* ob = reinterpret_cast<T*>(p.out) + (int64_t)b * p.out_b;
-      for (int idx = threadIdx.x; idx < G * D; idx += kDecodeThreads)
-        ob[(int64_t)(hk * G + idx / D) * p.out_h + idx % D] = E::from_f32(0.f);
-    }
+    if (part == 0 && ctx == 0)
+      for (int idx = threadIdx.x; idx < G * D; idx += kF32Threads)
+        ob[(int64_t)(idx / D) * p.out_h + idx % D] = 0.f;
     return;
   }
   const int nparts = (ctx + PART_TOKENS - 1) / PART_TOKENS;
-  const int blk_begin = part * PART_BLOCKS;
-  const int ctx_blocks = (ctx + BS - 1) / BS;
-  const int blk_end = min(blk_begin + PART_BLOCKS, ctx_blocks);
-
-  const T* kc = reinterpret_cast<const T*>(p.k_cache);
-  const T* vc = reinterpret_cast<const T*>(p.v_cache);
+  const int blk_end = min((part + 1) * PART_BLOCKS, (ctx + BS - 1) / BS);
+  int jb = part * PART_BLOCKS + wave;
+  const float* kc = reinterpret_cast<const float*>(p.k_cache);
+  const float* vc = reinterpret_cast<const float*>(p.v_cache);
   const int32_t* bt = p.block_tables + (int64_t)b * p.bt_stride;
 
-  // ---- query registers -------------------------------------------------------
-  typename E::QReg qr[G];
-  {
-    const T* qb = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_b;
+  // block jb's rows of this KV head, or -1: no block, or one outside the pool
+  auto block_base = [&](int j) __attribute__((always_inline)) -> int64_t {
+    if (j >= blk_end) return -1;
+    const int pb = uniform(bt[j]);
+    if (pb < 0 || (int64_t)pb >= p.num_blocks) return -1;
+    return ((int64_t)pb * p.num_kv_heads + hk) * (BS * D);
+  };
+  float4 kr[8], vr[8];
+  auto load_k = [&](int64_t base) __attribute__((always_inline)) {
+    if (base < 0) return;
+    const float* x = kc + base + col * D + 4 * slot;
 #pragma unroll
-    for (int g = 0; g < G; ++g)
-      E::load_q(qr[g], qb + (int64_t)(hk * G + g) * p.q_h + col * EL);
-  }
+    for (int c = 0; c < 8; ++c) kr[c] = *reinterpret_cast<const float4*>(x + 16 * c);
+  };
+  auto load_v = [&](int64_t base) __attribute__((always_inline)) {
+    if (base < 0) return;
+    const float* x = vc + base + slot * D + 4 * col;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+        vr[2 * u + g] = *reinterpret_cast<const float4*>(x + 4 * u * D + 64 * g);
+  };
+  int64_t base = block_base(jb);
+  load_k(base);
+  load_v(base);
 
-  float m[G], l[G], o[G][EL];
+  // the query heads in fp64, [group][c][e pair][slot][head] pairs of dims 16 c + 4 slot + e
+  __shared__ __attribute__((aligned(16))) double s_q[CG * 4 * D];
+  for (int idx = threadIdx.x; idx < CG * 4 * D; idx += kF32Threads) {
+    const int e = idx & 1, j = (idx >> 1) & 3, k = (idx >> 3) & 3, ep = (idx >> 5) & 1,
+              c = (idx >> 6) & 7, g = idx >> 9;
+    const int h = 4 * g + j;
+    s_q[idx] = h < G ? (double)reinterpret_cast<const float*>(
+                           p.q)[(int64_t)b * p.q_b + (int64_t)(hk * G + h) * p.q_h + 16 * c +
+                                4 * k + 2 * ep + e]
+                     : 0.0;
+  }
+  __syncthreads();
+  const double2* sq = reinterpret_cast<const double2*>(s_q) + (slot * 4 + (lane & 3));
+
+  f32x4_t oacc[kTiles];
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
+  for (int t = 0; t < kTiles; ++t) oacc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m[CG], l[CG];  // head 4 g + l % 4: its running max, this lane's share of its sum
+#pragma unroll
+  for (int g = 0; g < CG; ++g) {
     m[g] = -INFINITY;
     l[g] = 0.f;
+  }
+  const int my_key = 4 * ((lane >> 2) & 3) + slot;  // of the scores
+
+  while (jb < blk_end) {
+    const int64_t nbase = block_base(jb + kF32Waves);
+    const bool ok = base >= 0;  // uniform: an invalid block id contributes nothing
+    float x[CG];
+    if (ok) {
+      double acc[CG][2];
 #pragma unroll
-    for (int e = 0; e < EL; ++e) o[g][e] = 0.f;
+      for (int g = 0; g < CG; ++g) acc[g][0] = acc[g][1] = 0.0;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const double k0 = kr[c].x, k1 = kr[c].y, k2 = kr[c].z, k3 = kr[c].w;
+#pragma unroll
+        for (int g = 0; g < CG; ++g) {
+          const double2 q0 = sq[((8 * g + c) * 2 + 0) * 16], q1 = sq[((8 * g + c) * 2 + 1) * 16];
+          acc[g][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(k0, q0.x, acc[g][0], 0, 0, 0);
+          acc[g][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(k1, q0.y, acc[g][1], 0, 0, 0);
+          acc[g][0] = __builtin_amdgcn_mfma_f64_4x4x4f64(k2, q1.x, acc[g][0], 0, 0, 0);
+          acc[g][1] = __builtin_amdgcn_mfma_f64_4x4x4f64(k3, q1.y, acc[g][1], 0, 0, 0);
+        }
+      }
+      const bool valid = jb * BS + my_key < ctx;
+#pragma unroll
+      for (int g = 0; g < CG; ++g)
+        x[g] = valid ? (float)((acc[g][0] + acc[g][1]) * (double)p.scale_log2) : -INFINITY;
+    }
+    load_k(nbase);
+    if (ok) {
+      bool need = false;
+#pragma unroll
+      for (int g = 0; g < CG; ++g) need |= x[g] > m[g] + kLazyRescale;
+      if (wave_any(need)) {
+        float corr[CG];
+#pragma unroll
+        for (int g = 0; g < CG; ++g) {
+          float mx = x[g];
+#pragma unroll
+          for (int off = 4; off < kWave; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+          const float mn = fmaxf(m[g], mx);
+          corr[g] = (m[g] == -INFINITY) ? 0.f : fast_exp2(m[g] - mn);
+          m[g] = mn;
+          l[g] *= corr[g];
+        }
+        // column col of O^T is head col: lane col < 4 (8) holds its factor
+        const float oc = CG == 1 || col < 4 ? corr[0] : corr[CG - 1];
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) oacc[t] *= oc;
+      }
+      float pr[CG];
+#pragma unroll
+      for (int g = 0; g < CG; ++g) {
+        pr[g] = x[g] == -INFINITY ? 0.f : fast_exp2(x[g] - m[g]);
+        l[g] += pr[g];
+      }
+      if ((jb + 1) * BS > ctx) {
+        // rows past the context hold stale data of any value: keep it out
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (jb * BS + 4 * u + slot >= ctx)
+            vr[2 * u] = vr[2 * u + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+      auto pv = [&](auto uc) __attribute__((always_inline)) {
+        constexpr int u = decltype(uc)::value;
+        float w = row_up<4 * u>(pr[0]);
+        if constexpr (CG == 2) {
+          // heads 4 .. 7 in columns 4 .. 7: from lane col - 4 + 4 u of the row
+          const float w1 = row_up<(4 * u + 12) % 16>(pr[1]);
+          w = col < 4 ? w : w1;
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          const float4 v = vr[2 * u + g];
+          oacc[4 * g + 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.x, w, oacc[4 * g + 0], 0, 0, 0);
+          oacc[4 * g + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.y, w, oacc[4 * g + 1], 0, 0, 0);
+          oacc[4 * g + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.z, w, oacc[4 * g + 2], 0, 0, 0);
+          oacc[4 * g + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(v.w, w, oacc[4 * g + 3], 0, 0, 0);
+        }
+      };
+      pv(std::integral_constant<int, 0>());
+      pv(std::integral_constant<int, 1>());
+      pv(std::integral_constant<int, 2>());
+      pv(std::integral_constant<int, 3>());
+    }
+    load_v(nbase);
+    base = nbase;
+    jb += kF32Waves;
   }
 
-  // ---- block loads -------------------------------------------------------------
-  struct Buf {
-    uint4 k[LOADS];
-    uint4 v[LOADS];
-    bool ok;
-  };
-  auto load_block = [&](int jb, Buf& buf) {
-    const int pb = uniform(bt[jb]);
-    buf.ok = pb >= 0 && (int64_t)pb < p.num_blocks;
-    if (buf.ok) {
-      const int64_t base = ((int64_t)pb * p.num_kv_heads + hk) * (BS * D) + lane * EL;
-      const uint4* kp = reinterpret_cast<const uint4*>(kc + base);
-      const uint4* vp = reinterpret_cast<const uint4*>(vc + base);
+  // ---- merge the waves' states: the final output (single-partition sequence) or the
+  // partition's partial (m, l, un-normalised o) for the combine kernel ------------------------
+  __shared__ float sm_o[kF32Waves][CG * 4][D];
+  __shared__ float sm_m[kF32Waves][CG * 4], sm_l[kF32Waves][CG * 4];
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) buf.k[i] = kp[i * (TPL * D / EL)];
+  for (int g = 0; g < CG; ++g) {
 #pragma unroll
-      for (int i = 0; i < LOADS; ++i) buf.v[i] = vp[i * (TPL * D / EL)];
-    }
-  };
-
-  auto compute_block = [&](int jb, const Buf& buf) {
-    if (!buf.ok) return;  // uniform: an invalid block id contributes nothing
-    const bool full = (jb + 1) * BS <= ctx;
-    float x[LOADS][G];
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const bool valid = full || (jb * BS + i * TPL + row) < ctx;
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        float s;
-        if constexpr (std::is_same<T, float>::value)
-          s = (float)(group_sum_f64<LPT>(E::dot64(qr[g], buf.k[i])) * (double)p.scale_log2);
-        else
-          s = group_sum<LPT>(E::dot(qr[g], buf.k[i])) * p.scale_log2;
-        x[i][g] = valid ? s : -INFINITY;
-      }
-    }
-    bool need = false;
-    float bmax[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      float mx = x[0][g];
-#pragma unroll
-      for (int i = 1; i < LOADS; ++i) mx = fmaxf(mx, x[i][g]);
-      bmax[g] = mx;
-      need |= mx > m[g] + kLazyRescale;
-    }
-    if (wave_any(need)) {
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float mn = fmaxf(m[g], bmax[g]);
-        const float corr = (m[g] == -INFINITY) ? 0.f : fast_exp2(m[g] - mn);
-        m[g] = mn;
-        l[g] *= corr;
-#pragma unroll
-        for (int e = 0; e < EL; ++e) o[g][e] *= corr;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      float vf[EL];
-      E::widen(buf.v[i], vf);
-      const bool valid = full || (jb * BS + i * TPL + row) < ctx;
-      if (!full) {
-        // Slots past the context hold stale data of any value; keep it out.
-#pragma unroll
-        for (int e = 0; e < EL; ++e) vf[e] = valid ? vf[e] : 0.f;
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float pr = valid ? fast_exp2(x[i][g] - m[g]) : 0.f;
-        l[g] += pr;
-#pragma unroll
-        for (int e = 0; e < EL; ++e) o[g][e] = fmaf(pr, vf[e], o[g][e]);
-      }
-    }
-  };
-
-  // ---- main loop: two register buffers, next block in flight -------------------
-  {
-    Buf A, B;
-    int jb = blk_begin + wave;
-    if (jb < blk_end) load_block(jb, A);
-    while (jb < blk_end) {
-      if (jb + kDecodeWaves < blk_end) load_block(jb + kDecodeWaves, B);
-      compute_block(jb, A);
-      jb += kDecodeWaves;
-      if (jb >= blk_end) break;
-      if (jb + kDecodeWaves < blk_end) load_block(jb + kDecodeWaves, A);
-      compute_block(jb, B);
-      jb += kDecodeWaves;
+    for (int off = 4; off < kWave; off <<= 1) l[g] += __shfl_xor(l[g], off, kWave);
+    if (lane < 4) {
+      sm_m[wave][4 * g + lane] = m[g];
+      sm_l[wave][4 * g + lane] = l[g];
     }
   }
-
-  // ---- merge the TPL lane rows of the wave ---------------------------------------
+  if (col < 4 * CG) {
 #pragma unroll
-  for (int off = LPT; off < kWave; off <<= 1) {
+    for (int g = 0; g < 2; ++g)
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const float mo = __shfl_xor(m[g], off, kWave);
-      const float lo = __shfl_xor(l[g], off, kWave);
-      float mn, wa, wb;
-      softmax_merge_weights(m[g], mo, mn, wa, wb);
-      m[g] = mn;
-      l[g] = l[g] * wa + lo * wb;
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<float4*>(&sm_o[wave][col][64 * g + 4 * (4 * slot + i)]) =
+            make_float4(oacc[4 * g][i], oacc[4 * g + 1][i], oacc[4 * g + 2][i], oacc[4 * g + 3][i]);
+  }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < G * D; idx += kF32Threads) {
+    const int g = idx / D;
+    const int d = idx - g * D;
+    float mt = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < EL; ++e) {
-        const float oo = __shfl_xor(o[g][e], off, kWave);
-        o[g][e] = o[g][e] * wa + oo * wb;
+    for (int w = 0; w < kF32Waves; ++w) mt = fmaxf(mt, sm_m[w][g]);
+    float lt = 0.f, ot = 0.f;
+#pragma unroll
+    for (int w = 0; w < kF32Waves; ++w) {
+      const float mw = sm_m[w][g];
+      const float wt = (mw == -INFINITY) ? 0.f : fast_exp2(mw - mt);
+      lt = fmaf(sm_l[w][g], wt, lt);
+      ot = fmaf(sm_o[w][g][d], wt, ot);
+    }
+    const int h = hk * G + g;
+    if (nparts == 1) {
+      ob[(int64_t)g * p.out_h + d] = lt > 0.f ? ot / lt : 0.f;
+    } else {
+      const int64_t at = ((int64_t)b * p.num_heads + h) * p.max_parts + part;
+      p.ws_o[at * D + d] = ot;
+      if (d == 0) {
+        p.ws_ml[at * 2 + 0] = mt;
+        p.ws_ml[at * 2 + 1] = lt;
       }
     }
   }
-
-  merge_waves_and_store<T, D, G>(p, o, m, l, row, col, wave, b, hk, part, nparts);
 }
 
 // Wave-wide max (every lane receives the maximum over all 64 lanes).
@@ -425,10 +370,9 @@ NIA_DEVICE float wave_sum(float x) {
 // partition were finished by the partial kernel.
 constexpr int kCombinePrefetch = 16;
 
-template <typename T, int D, int BS, int PART_BLOCKS>
+template <int D, int BS, int PART_BLOCKS>
 __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine_kernel(DecodeParams p,
                                                                                int batch) {
-  using E = Elem<T>;
   constexpr int PART_TOKENS = PART_BLOCKS * BS;
   constexpr int DL = D / kWave;  // dims per lane
   static_assert(DL == 2, "one float2 of output per lane");
@@ -492,9 +436,10 @@ __global__ __launch_bounds__(kCombineThreads) void paged_decode_combine_kernel(D
   }
   lt = wave_sum(lt);
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
-  T* out = reinterpret_cast<T*>(p.out) + (int64_t)b * p.out_b + (int64_t)h * p.out_h + DL * lane;
-  out[0] = E::from_f32(acc.x * inv);
-  out[1] = E::from_f32(acc.y * inv);
+  float* out =
+      reinterpret_cast<float*>(p.out) + (int64_t)b * p.out_b + (int64_t)h * p.out_h + DL * lane;
+  out[0] = acc.x * inv;
+  out[1] = acc.y * inv;
 }
 
 // Inclusive prefix sum over the lanes of a wave, by DPP moves (no LDS round trips): shifts
@@ -1374,28 +1319,15 @@ int launch_split(DecodeParams& p, int batch, hipStream_t s) {
 
 int launch_f32_partitions(const DecodeParams& p, int G, int batch, hipStream_t s) {
   const dim3 grid(p.max_parts, p.num_kv_heads, batch);
-  switch (G) {
-#define NIA_CASE(GG)                                                                          \
-  case GG:                                                                                    \
-    nia_launch((paged_decode_partial_kernel<float, 128, GG, 16, kPartBlocks>), grid,          \
-               dim3(kDecodeThreads), s, p);                                                   \
-    break;
-    NIA_CASE(1)
-    NIA_CASE(2)
-    NIA_CASE(3)
-    NIA_CASE(4)
-    NIA_CASE(5)
-    NIA_CASE(6)
-    NIA_CASE(7)
-    NIA_CASE(8)
-#undef NIA_CASE
-    default:
-      return NIA_ERR_UNSUPPORTED;
-  }
+  if (G > 8) return NIA_ERR_UNSUPPORTED;
+  if (G <= 4)
+    nia_launch((paged_decode_f32_kernel<1, kPartBlocks>), grid, dim3(kF32Threads), s, p);
+  else
+    nia_launch((paged_decode_f32_kernel<2, kPartBlocks>), grid, dim3(kF32Threads), s, p);
   if (p.max_parts > 1) {
     constexpr int kPairsPerGroup = kCombineThreads / kWave;
     const int pairs = batch * p.num_heads;
-    nia_launch((paged_decode_combine_kernel<float, 128, 16, kPartBlocks>),
+    nia_launch((paged_decode_combine_kernel<128, 16, kPartBlocks>),
                dim3((pairs + kPairsPerGroup - 1) / kPairsPerGroup), dim3(kCombineThreads), s, p,
                batch);
   }
