@@ -507,77 +507,87 @@ def prefill(
     an additive float mask indexed [sequence, head, query row, key] (size-1 dimensions
     broadcast), added to the scaled scores; -inf masks a key.
     """
-    dev = _require_gpu(q, k, v, q_start, q_len, k_start, k_len)
-    if q.dim() != 3 or k.dim() != 3 or v.dim() != 3 or k.shape != v.shape:
+    # the checks read every attribute once: a call with new lengths (a prefill's are new on
+    # nearly every call) pays them all
+    idx = q.get_device()
+    if idx < 0 or k.get_device() != idx or v.get_device() != idx or \
+            q_start.get_device() != idx or q_len.get_device() != idx or \
+            k_start.get_device() != idx or k_len.get_device() != idx:
+        _require_gpu(q, k, v, q_start, q_len, k_start, k_len)
+    q_shape, k_shape = q.shape, k.shape
+    if len(q_shape) != 3 or len(k_shape) != 3 or k_shape != v.shape:
         raise ValueError("q must be (Tq, H, D) and k, v (Tk, H_kv, D)")
-    _, h, d = q.shape
-    hkv = k.shape[1]
-    if k.shape[2] != d:
+    rows, h, d = q_shape
+    keys, hkv, dk = k_shape
+    if dk != d:
         raise ValueError("head_dim mismatch between q and k/v")
     if h % hkv != 0:
         raise ValueError(f"num_heads must be divisible by num_kv_heads, got {h=} and {hkv=}")
-    if not (q.dtype == k.dtype == v.dtype):
+    dtype = q.dtype
+    if not (dtype == k.dtype == v.dtype):
         raise ValueError("q, k and v must share one dtype")
-    dt = _dtype_code(q)
-    for name, t in (("q", q), ("k", k), ("v", v)):
-        _last_contig(name, t)
+    dt = _DTYPES.get(dtype)
+    if dt is None:
+        dt = _dtype_code(q)
+    q_st, k_st, v_st = q.stride(), k.stride(), v.stride()
+    if q_st[2] != 1 or k_st[2] != 1 or v_st[2] != 1:
+        for name, t in (("q", q), ("k", k), ("v", v)):
+            _last_contig(name, t)
     n = q_start.shape[0]
-    qs, ql, ks, kl = (_i32(nm, t, n) for nm, t in
-                      (("q_start", q_start), ("q_len", q_len), ("k_start", k_start),
-                       ("k_len", k_len)))
+    qs, ql, ks, kl = _i32("q_start", q_start, n), _i32("q_len", q_len, n), \
+        _i32("k_start", k_start, n), _i32("k_len", k_len, n)
     if out is None:
         out = torch.empty_like(q, memory_format=torch.contiguous_format)
-    elif out.shape != q.shape or out.dtype != q.dtype:
-        raise ValueError("out must match q's shape and dtype")
-    _last_contig("out", out)
+        o_st = out.stride()
+    else:
+        if out.shape != q_shape or out.dtype != dtype:
+            raise ValueError("out must match q's shape and dtype")
+        o_st = out.stride()
+    if o_st[2] != 1:
+        _last_contig("out", out)
+    max_q_len, causal = int(max_q_len), int(causal)
+    scale = _default_scale(d, scale)
     if mask is not None:
         # the mask must cover every key the kernels read: one read of the key lengths (general
         # masks are rare; prefix masks take the key-length path and never come here)
         max_keys = int(kl.max()) if n > 0 else 0
-        m4, strides = _mask_operand(mask, n, h, int(max_q_len), max_keys, dev)
+        m4, strides = _mask_operand(mask, n, h, max_q_len, max_keys, q.device)
         st = _lib.load().nia_prefill_masked(
-            out.data_ptr(), out.stride(0), out.stride(1),
-            q.data_ptr(), q.stride(0), q.stride(1),
-            k.data_ptr(), k.stride(0), k.stride(1),
-            v.data_ptr(), v.stride(0), v.stride(1),
+            out.data_ptr(), o_st[0], o_st[1], q.data_ptr(), q_st[0], q_st[1],
+            k.data_ptr(), k_st[0], k_st[1], v.data_ptr(), v_st[0], v_st[1],
             qs.data_ptr(), ql.data_ptr(), ks.data_ptr(), kl.data_ptr(),
-            n, int(max_q_len), h, hkv, d, _default_scale(d, scale), int(causal), dt,
-            m4.data_ptr(), *strides, _stream(dev),
+            n, max_q_len, h, hkv, d, scale, causal, dt,
+            m4.data_ptr(), *strides, _raw_stream(idx),
         )
         _lib.check("nia_prefill_masked", st)
         return out
     ws = None
-    keys = k.shape[0]  # bounds every sequence's keys
     if dt != _lib.DTYPE_BF16:
-        if q.shape[0] * h <= _SPLIT_MAX_ROWS_F32:
+        if rows * h <= _SPLIT_MAX_ROWS_F32:
             if causal == CAUSAL_TOP_LEFT:  # its rows see no key past their own position
-                keys = min(keys, int(max_q_len))
-            ws = _split_workspace(n, int(max_q_len), keys, h, hkv, d, int(causal), dt, dev)
+                keys = min(keys, max_q_len)
+            ws = _split_workspace(n, max_q_len, keys, h, hkv, d, causal, dt, q.device)
     elif causal != CAUSAL_TOP_LEFT and keys >= n * _SPLIT_MIN_KEYS and \
             n * h * max_q_len <= _SPLIT_MAX_ROWS:
-        ws = _split_workspace(n, int(max_q_len), keys, h, hkv, d, int(causal), dt, dev)
+        ws = _split_workspace(n, max_q_len, keys, h, hkv, d, causal, dt, q.device)
     if ws is not None:
         st = _lib.load().nia_prefill_split(
-            out.data_ptr(), out.stride(0), out.stride(1),
-            q.data_ptr(), q.stride(0), q.stride(1),
-            k.data_ptr(), k.stride(0), k.stride(1),
-            v.data_ptr(), v.stride(0), v.stride(1),
+            out.data_ptr(), o_st[0], o_st[1], q.data_ptr(), q_st[0], q_st[1],
+            k.data_ptr(), k_st[0], k_st[1], v.data_ptr(), v_st[0], v_st[1],
             qs.data_ptr(), ql.data_ptr(), ks.data_ptr(), kl.data_ptr(),
-            n, int(max_q_len), h, hkv, d, _default_scale(d, scale), int(causal), dt, keys,
-            ws.data_ptr(), ws.numel(), _stream(dev),
+            n, max_q_len, h, hkv, d, scale, causal, dt, keys,
+            ws.data_ptr(), ws.numel(), _raw_stream(idx),
         )
         _lib.check("nia_prefill_split", st)
         return out
-    lib = _lib.calls()
-    st = lib.nia_prefill(
-        out.data_ptr(), out.stride(0), out.stride(1),
-        q.data_ptr(), q.stride(0), q.stride(1),
-        k.data_ptr(), k.stride(0), k.stride(1),
-        v.data_ptr(), v.stride(0), v.stride(1),
+    st = _lib.calls().nia_prefill(
+        out.data_ptr(), o_st[0], o_st[1], q.data_ptr(), q_st[0], q_st[1],
+        k.data_ptr(), k_st[0], k_st[1], v.data_ptr(), v_st[0], v_st[1],
         qs.data_ptr(), ql.data_ptr(), ks.data_ptr(), kl.data_ptr(),
-        n, int(max_q_len), h, hkv, d, _default_scale(d, scale), int(causal), dt, _stream(dev),
+        n, max_q_len, h, hkv, d, scale, causal, dt, _raw_stream(idx),
     )
-    _lib.check("nia_prefill", st)
+    if st:
+        _lib.check("nia_prefill", st)
     return out
 
 
@@ -696,25 +706,36 @@ def prefill_paged(
     if is_fp8_cache(k_cache):
         return _prefill_paged_fp8(q, k_cache, v_cache, block_tables, q_start, q_len,
                                    context_lens, max_q_len, causal, scale, out, k_scale, v_scale)
-    dev = _require_gpu(q, k_cache, v_cache, block_tables, q_start, q_len, context_lens)
-    if q.dim() != 3:
+    # as in prefill: every attribute is read once
+    idx = q.get_device()
+    if idx < 0 or k_cache.get_device() != idx or v_cache.get_device() != idx or \
+            block_tables.get_device() != idx or q_start.get_device() != idx or \
+            q_len.get_device() != idx or context_lens.get_device() != idx:
+        _require_gpu(q, k_cache, v_cache, block_tables, q_start, q_len, context_lens)
+    q_shape, c_shape, bt_shape = q.shape, k_cache.shape, block_tables.shape
+    if len(q_shape) != 3:
         raise ValueError("q must be (Tq, H, D)")
-    _, h, d = q.shape
-    if k_cache.dim() != 4 or v_cache.shape != k_cache.shape:
+    rows, h, d = q_shape
+    if len(c_shape) != 4 or v_cache.shape != c_shape:
         raise ValueError("k_cache/v_cache must be [num_blocks, H_kv, block_size, head_dim]")
     if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
         raise ValueError("k_cache/v_cache layer slices must be contiguous")
-    nb, hkv, bs, dc = k_cache.shape
+    nb, hkv, bs, dc = c_shape
     if dc != d:
         raise ValueError("head_dim mismatch between q and the cache")
     if h % hkv != 0:
         raise ValueError(f"num_heads must be divisible by num_kv_heads, got {h=} and {hkv=}")
-    if not (q.dtype == k_cache.dtype == v_cache.dtype):
+    dtype = q.dtype
+    if not (dtype == k_cache.dtype == v_cache.dtype):
         raise ValueError("q and the caches must share one dtype")
-    dt = _dtype_code(q)
-    _last_contig("q", q)
+    dt = _DTYPES.get(dtype)
+    if dt is None:
+        dt = _dtype_code(q)
+    q_st = q.stride()
+    if q_st[2] != 1:
+        _last_contig("q", q)
     n = q_start.shape[0]
-    if block_tables.dtype != torch.int32 or block_tables.dim() != 2 or block_tables.shape[0] != n:
+    if block_tables.dtype != torch.int32 or len(bt_shape) != 2 or bt_shape[0] != n:
         raise ValueError("block_tables must be (B, max_blocks) int32")
     if block_tables.stride(1) != 1:
         block_tables = block_tables.contiguous()
@@ -724,38 +745,38 @@ def prefill_paged(
     context_lens = context_lens.contiguous()
     if out is None:
         out = torch.empty_like(q, memory_format=torch.contiguous_format)
-    elif out.shape != q.shape or out.dtype != q.dtype:
+    elif out.shape != q_shape or out.dtype != dtype:
         raise ValueError("out must match q's shape and dtype")
-    _last_contig("out", out)
+    o_st = out.stride()
+    if o_st[2] != 1:
+        _last_contig("out", out)
+    max_q_len, causal, mb = int(max_q_len), int(causal), bt_shape[1]
+    scale = _default_scale(d, scale)
     ws = None
-    keys = block_tables.shape[1] * bs
-    if q.shape[0] * h <= _SPLIT_MAX_ROWS_F32 if dt != _lib.DTYPE_BF16 else (
-            keys >= _SPLIT_MIN_KEYS and causal != CAUSAL_TOP_LEFT and
+    if rows * h <= _SPLIT_MAX_ROWS_F32 if dt != _lib.DTYPE_BF16 else (
+            mb * bs >= _SPLIT_MIN_KEYS and causal != CAUSAL_TOP_LEFT and
             n * h * max_q_len <= _SPLIT_MAX_ROWS):
-        ws = _split_workspace(n, int(max_q_len), keys, h, hkv, d, int(causal), dt, dev)
+        ws = _split_workspace(n, max_q_len, mb * bs, h, hkv, d, causal, dt, q.device)
     if ws is not None:
         st = _lib.load().nia_prefill_paged_split(
-            out.data_ptr(), out.stride(0), out.stride(1),
-            q.data_ptr(), q.stride(0), q.stride(1),
+            out.data_ptr(), o_st[0], o_st[1], q.data_ptr(), q_st[0], q_st[1],
             k_cache.data_ptr(), v_cache.data_ptr(),
-            block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1],
+            block_tables.data_ptr(), block_tables.stride(0), mb,
             qs.data_ptr(), ql.data_ptr(), context_lens.data_ptr(),
-            n, int(max_q_len), h, hkv, d, bs, nb, _default_scale(d, scale), int(causal), dt,
-            ws.data_ptr(), ws.numel(), _stream(dev),
+            n, max_q_len, h, hkv, d, bs, nb, scale, causal, dt,
+            ws.data_ptr(), ws.numel(), _raw_stream(idx),
         )
         _lib.check("nia_prefill_paged_split", st)
         return out
-    lib = _lib.calls()
-    st = lib.nia_prefill_paged(
-        out.data_ptr(), out.stride(0), out.stride(1),
-        q.data_ptr(), q.stride(0), q.stride(1),
+    st = _lib.calls().nia_prefill_paged(
+        out.data_ptr(), o_st[0], o_st[1], q.data_ptr(), q_st[0], q_st[1],
         k_cache.data_ptr(), v_cache.data_ptr(),
-        block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1],
+        block_tables.data_ptr(), block_tables.stride(0), mb,
         qs.data_ptr(), ql.data_ptr(), context_lens.data_ptr(),
-        n, int(max_q_len), h, hkv, d, bs, nb, _default_scale(d, scale), int(causal), dt,
-        _stream(dev),
+        n, max_q_len, h, hkv, d, bs, nb, scale, causal, dt, _raw_stream(idx),
     )
-    _lib.check("nia_prefill_paged", st)
+    if st:
+        _lib.check("nia_prefill_paged", st)
     return out
 
 
