@@ -1161,13 +1161,18 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
   }
 }
 
-// Merges the key ranges' partials of every row that has more than one (SPLIT): D / 4 lanes a
-// row (four dims each), the workgroup's rows kMergeRows at a time over grid y.
-constexpr int kMergeRows = 8;
+// Merges the key ranges' partials of every row that has more than one (SPLIT): 32 lanes a row
+// (four dims each), ROWS rows a thread, eight partials of a thread in flight together.  A
+// workgroup pays for the grid's map and the lengths before its first partial, so calls of
+// few ranges, which have many rows, give it more of them: 1024 rows of 32 heads in two
+// ranges 16 us with one row a thread, 10.7 with four.
+constexpr int kMergeLanes = 32;
+constexpr int kMergeFew = 4;  // ranges up to which a thread takes four rows
 
-template <int D, bool PAGED>
+template <int D, bool PAGED, int ROWS>
 __global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillParams p) {
-  constexpr int kLanes = 32;  // per row; D / 4 of them hold dims
+  constexpr int kAhead = 8 / ROWS;  // ranges loaded together
+  constexpr int kStep = kPrefillThreads / kMergeLanes;  // rows of the workgroup at a time
   int seq, h, mb;
   if (!map_workgroup<PAGED>(p, seq, h, mb)) return;
   const int qlen = p.q_len[seq];
@@ -1175,6 +1180,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillP
   const int rows = qlen * pack;
   const int m0 = mb * kBlockM;
   if (m0 >= rows) return;
+  const int64_t qstart = p.q_start[seq];
   int klen;
   if constexpr (PAGED) {
     int64_t c = p.ctx_len[seq];
@@ -1190,52 +1196,63 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillP
     n_end = min(klen, q_pos0 + tok_of(min(m0 + kBlockM, rows) - 1) + 1);
   const int ranges = key_ranges((max(n_end, 0) + kBlockN - 1) / kBlockN, p.splits);
   if (ranges == 1) return;  // written by the prefill kernel
-  const int d = 4 * (threadIdx.x % kLanes);
-  const int r_end = min(rows - m0, ((int)blockIdx.y + 1) * kMergeRows);
+  const int d = 4 * (threadIdx.x % kMergeLanes);
+  if (d >= D) return;
+  const int r0 = blockIdx.y * (ROWS * kStep) + threadIdx.x / kMergeLanes;  // then kStep apart
+  const int last = min(rows - m0, kBlockM) - 1;
   const int64_t step = (int64_t)gridDim.x * kBlockM;  // rows between ranges
-  for (int r = blockIdx.y * kMergeRows + threadIdx.x / kLanes; r < r_end;
-       r += kPrefillThreads / kLanes) {
-    const int64_t prow = (int64_t)blockIdx.x * kBlockM + r;
-    const float2* ml = reinterpret_cast<const float2*>(p.part_ml);
-    const bool has = d < D;
-    float m = -INFINITY, l = 0.f;
-    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    constexpr int kAhead = 8;  // ranges loaded together
-    for (int s0 = 0; s0 < ranges; s0 += kAhead) {
-      float2 st[kAhead];
-      f32x4_t o[kAhead];
+  const float2* ml = reinterpret_cast<const float2*>(p.part_ml);
+  float m[ROWS], l[ROWS];
+  f32x4_t acc[ROWS];
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) {
-        st[i] = make_float2(-INFINITY, 0.f);
-        o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        if (s0 + i < ranges) {
-          const int64_t pr = (s0 + i) * step + prow;
-          st[i] = ml[pr];
-          if (has) o[i] = *reinterpret_cast<const f32x4_t*>(p.part_o + pr * D + d);
-        }
+  for (int j = 0; j < ROWS; ++j) {
+    m[j] = -INFINITY;
+    l[j] = 0.f;
+    acc[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int s0 = 0; s0 < ranges; s0 += kAhead) {
+    float2 st[kAhead][ROWS];
+    f32x4_t o[kAhead][ROWS];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+      for (int j = 0; j < ROWS; ++j) {
+        // past the ranges: the last one again, with weight 0; past the rows: the last row
+        const int64_t pr = min(s0 + i, ranges - 1) * step + (int64_t)blockIdx.x * kBlockM +
+                           min(r0 + j * kStep, last);
+        st[i][j] = ml[pr];
+        o[i][j] = *reinterpret_cast<const f32x4_t*>(p.part_o + pr * D + d);
       }
-      float mn = m;
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) mn = fmaxf(mn, st[i].x);
-      if (mn == -INFINITY) continue;  // no visible key so far
-      const float corr = m == -INFINITY ? 0.f : fast_exp2(m - mn);
-      l *= corr;
-      acc *= corr;
-      m = mn;
+    for (int j = 0; j < ROWS; ++j) {
+      float mn = m[j];
 #pragma unroll
       for (int i = 0; i < kAhead; ++i) {
-        const float w = st[i].x == -INFINITY ? 0.f : fast_exp2(st[i].x - mn);
-        l = fmaf(st[i].y, w, l);
-        if (w > 0.f) acc += o[i] * w;
+        if (s0 + i >= ranges) st[i][j] = make_float2(-INFINITY, 0.f);
+        mn = fmaxf(mn, st[i][j].x);
+      }
+      if (mn == -INFINITY) continue;  // no visible key so far
+      const float corr = m[j] == -INFINITY ? 0.f : fast_exp2(m[j] - mn);
+      l[j] *= corr;
+      acc[j] *= corr;
+      m[j] = mn;
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        const float w = st[i][j].x == -INFINITY ? 0.f : fast_exp2(st[i][j].x - mn);
+        l[j] = fmaf(st[i][j].y, w, l[j]);
+        if (w > 0.f) acc[j] += o[i][j] * w;
       }
     }
-    if (!has) continue;
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+  }
+#pragma unroll
+  for (int j = 0; j < ROWS; ++j) {
+    const int r = r0 + j * kStep;
+    if (r > last) break;
+    const float inv = l[j] > 0.f ? 1.f / l[j] : 0.f;
     const int tok = tok_of(m0 + r);
-    bf16_t* op = p.o + (p.q_start[seq] + (int64_t)tok) * p.o_tok +
-                 (int64_t)(h * pack + m0 + r - tok * pack) * p.o_head + d;
-    *reinterpret_cast<uint2*>(op) =
-        make_uint2(pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv));
+    bf16_t* op = p.o + (qstart + tok) * p.o_tok + (int64_t)(h * pack + m0 + r - tok * pack) * p.o_head + d;
+    *reinterpret_cast<uint2*>(op) = make_uint2(pack_bf16x2(acc[j][0] * inv, acc[j][1] * inv),
+                                               pack_bf16x2(acc[j][2] * inv, acc[j][3] * inv));
   }
 }
 
@@ -1321,8 +1338,13 @@ template <int D, bool PAGED>
 void launch_dma_split(const PrefillParams& p, dim3 grid, hipStream_t s) {
   nia_launch((prefill_dma_kernel<D, PAGED, false, false, false, false, false, true, true>),
              dim3(grid.x, (unsigned)p.splits), dim3(kPrefillThreads), s, p);
-  nia_launch((prefill_merge_kernel<D, PAGED>), dim3(grid.x, kBlockM / kMergeRows),
-             dim3(kPrefillThreads), s, p);
+  constexpr int kStep = kPrefillThreads / kMergeLanes;
+  if (p.splits <= kMergeFew)
+    nia_launch((prefill_merge_kernel<D, PAGED, 4>), dim3(grid.x, kBlockM / (4 * kStep)),
+               dim3(kPrefillThreads), s, p);
+  else
+    nia_launch((prefill_merge_kernel<D, PAGED, 1>), dim3(grid.x, kBlockM / kStep),
+               dim3(kPrefillThreads), s, p);
 }
 
 template <bool PAGED, bool BIAS = false>

@@ -32,8 +32,9 @@
 // every 115-128 cycles (probe; 64 at the nominal rate), so a
 // 16 x 32 tile is ~10k cycles, 4.3 us, and a second wave on the SIMD adds nothing.
 // v_mfma_f64_4x4x4 issues every 16.6 (1.7 times the rate), but with its keys broadcast over
-// the four blocks it reads and widens every K element four times: measured 427 us for the
-// four prompts of 1000.
+// the four blocks it reads and widens every K element four times (427 us for the four
+// prompts of 1000), and with the dims over the blocks and a reduce-scatter of the shares its
+// 32 accumulators spill 18 registers (363 us, bit-identical).
 // Both 16x16x4
 // MFMAs take A[l % 16][l / 16] and B[l / 16][l % 16] from lane l and give it column
 // l % 16 of the 16x16 result; register i holds row 4 (l / 16) + i for fp32 and row
