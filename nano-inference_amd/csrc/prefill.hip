@@ -78,7 +78,7 @@ struct PrefillParams {
   int32_t group;
   // Rows of an m-block: row r of a (sequence, head index) item is query token r / pack, head
   // pack * index + r % pack: a KV head's whole group (pack = group, map_group = 1 head index
-  // per KV head) or one head (pack = 1, map_group = group); set_rows says when.
+  // per KV head) or one head (pack = 1, map_group = group); pack_uncut says when.
   int32_t pack;
   uint32_t pack_magic;  // r / pack = key_block(r, ...) for pack > 1
   int32_t pack_shift;
@@ -1302,20 +1302,33 @@ size_t split_bytes(int64_t nwg, int32_t splits, int head_dim) {
   return splits > 1 ? (size_t)nwg * splits * kBlockM * ((size_t)head_dim + 2) * sizeof(float) : 0;
 }
 
-// Rows per item and m-blocks.  A KV head's query heads are packed into the rows where that
-// takes fewer 128-row blocks than a block of its own for each head's remainder: a 40-row
-// chunk of 4 heads is 2 blocks instead of 4.  Where the count is the same the heads keep
-// their own blocks (packed, a prompt of 1531 tokens ran 34.9 instead of 34.2 us: each lane
-// divides its rows).
-void set_rows(PrefillParams& p, int max_q_len, bool packable) {
-  const int64_t per_head = ((int64_t)max_q_len + kBlockM - 1) / kBlockM;
-  const int64_t all = ((int64_t)max_q_len * p.group + kBlockM - 1) / kBlockM;
-  const bool packed = packable && all < per_head * p.group &&
-                      (int64_t)max_q_len * p.group <= INT32_MAX;
+// Rows per item and m-blocks: the query heads of a KV head packed into the rows (p.pack =
+// group), or one head an item.
+void set_rows(PrefillParams& p, int max_q_len, bool packed) {
   p.pack = packed ? p.group : 1;
   p.map_group = packed ? 1 : p.group;
-  p.num_m_blocks = (int32_t)(packed ? all : per_head);
+  p.num_m_blocks = (int32_t)(((int64_t)max_q_len * p.pack + kBlockM - 1) / kBlockM);
   block_divisor(p.pack, p.pack_magic, p.pack_shift);
+}
+
+// Blocks of 128 rows of a KV head's query heads: packed, and each head on its own.
+int64_t packed_blocks(const PrefillParams& p, int max_q_len) {
+  return ((int64_t)max_q_len * p.group + kBlockM - 1) / kBlockM;
+}
+int64_t head_blocks(const PrefillParams& p, int max_q_len) {
+  return ((int64_t)max_q_len + kBlockM - 1) / kBlockM * p.group;
+}
+
+// Whether an uncut call packs: where the heads' own blocks need more than one round of the
+// chip (two workgroups a CU) and packing saves a sixteenth of them.  Five prompts of 60-500
+// tokens (28 and 4 heads) 22.6 -> 20.3 us, eight of 100-800 (16 and 8) 26.7 -> 24.8; with
+// less to save, or a grid that fits the chip, the rows' divisions cost more than they bring
+// (one prompt of 900 tokens 20.6 -> 21.1 us, six 60-row chunks 9.9 -> 10.7).  A call that is cut
+// into key ranges packs whenever that saves a block: its blocks are what the ranges multiply.
+bool pack_uncut(const PrefillParams& p, int max_q_len) {
+  const int64_t own = head_blocks(p, max_q_len);
+  return packed_blocks(p, max_q_len) * 16 <= own * 15 &&
+         own * p.num_seqs * p.num_kv_heads > 512;
 }
 
 // The workgroups of a packed or unpacked grid.
@@ -1360,15 +1373,14 @@ int launch_prefill(PrefillParams& p, int head_dim, int max_q_len, hipStream_t s,
   if (BIAS && !dma_ok) return NIA_ERR_UNSUPPORTED;
   // packed rows: the lane offsets must fit 32 bits and not be negative
   const bool plain = !BIAS && dma_ok && (!PAGED || (p.bs % 16 == 0 && (p.bs & (p.bs - 1)) == 0));
-  set_rows(p, max_q_len,
-           plain && p.q_head >= 0 && p.q_head < kMaxRowStride &&
-               q_span_bytes(p, p.group, head_dim) <= INT32_MAX);
-  p.q_span = (int32_t)q_span_bytes(p, p.pack, head_dim);
-  const int64_t nwg = grid_size(p);
-  if (nwg >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
-  const dim3 grid((unsigned)nwg);
+  const bool packable = plain && p.q_head >= 0 && p.q_head < kMaxRowStride &&
+                        q_span_bytes(p, p.group, head_dim) <= INT32_MAX &&
+                        (int64_t)max_q_len * p.group <= INT32_MAX;
   p.splits = 1;
+  int64_t nwg = 0;
   if (sp.ws && plain) {
+    set_rows(p, max_q_len, packable && packed_blocks(p, max_q_len) < head_blocks(p, max_q_len));
+    nwg = grid_size(p);
     const int32_t n = split_count(nwg, (sp.max_k_len + kBlockN - 1) / kBlockN, p.causal);
     if (n > 1 && split_bytes(nwg, n, head_dim) <= sp.bytes) {
       p.splits = n;
@@ -1376,6 +1388,13 @@ int launch_prefill(PrefillParams& p, int head_dim, int max_q_len, hipStream_t s,
       p.part_ml = p.part_o + (size_t)nwg * n * kBlockM * head_dim;
     }
   }
+  if (p.splits == 1) {
+    set_rows(p, max_q_len, packable && pack_uncut(p, max_q_len));
+    nwg = grid_size(p);
+  }
+  p.q_span = (int32_t)q_span_bytes(p, p.pack, head_dim);
+  if (nwg >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
+  const dim3 grid((unsigned)nwg);
   switch (head_dim) {
 #define NIA_PREFILL_CASE(DD)                                                                 \
   case DD:                                                                                   \
@@ -1731,7 +1750,8 @@ extern "C" size_t nia_prefill_split_workspace_size(int32_t num_seqs, int32_t max
   if (dtype != NIA_DTYPE_BF16) return 0;
   PrefillParams p{};
   p.group = num_heads / num_kv_heads;
-  set_rows(p, max_q_len, true);
+  if ((int64_t)max_q_len * p.group > INT32_MAX) return 0;
+  set_rows(p, max_q_len, packed_blocks(p, max_q_len) < head_blocks(p, max_q_len));
   p.groups_per_xcd = (int32_t)(((int64_t)num_seqs * num_kv_heads + kXcds - 1) / kXcds);
   p.order_by_len = causal != NIA_CAUSAL_TOP_LEFT && num_seqs <= kOrderMaxSeqs;
   const int64_t nwg = grid_size(p);
