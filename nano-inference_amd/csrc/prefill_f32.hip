@@ -505,7 +505,9 @@ void launch_f32_split(const PrefillF32Params& p, dim3 grid, hipStream_t s) {
 size_t prefill_f32_split_bytes(int32_t num_seqs, int64_t max_q_len, int64_t max_k_len,
                                int32_t num_heads, int32_t num_kv_heads, int head_dim) {
   int32_t a, b, c;
-  const int64_t nwg = f32_grid(num_seqs, num_kv_heads, max_q_len * (num_heads / num_kv_heads), a, b, c);
+  int64_t rows = max_q_len * (num_heads / num_kv_heads);
+  if (rows > INT32_MAX) rows = INT32_MAX;
+  const int64_t nwg = f32_grid(num_seqs, num_kv_heads, rows, a, b, c);
   return f32_split_bytes(nwg, f32_split_count(nwg, max_k_len), head_dim);
 }
 
@@ -517,8 +519,9 @@ int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int nu
     return NIA_ERR_UNSUPPORTED;
   if (elem == kElemFp8 && (head_dim != 128 || !p.k_scale || !p.v_scale))
     return NIA_ERR_UNSUPPORTED;
-  const int64_t rows = (int64_t)(p.decode ? 1 : max_q_len) * p.group;
-  if (rows > INT32_MAX) return NIA_ERR_UNSUPPORTED;
+  // row numbers are ints: a longer bound than any call can fill sizes the grid for them all
+  int64_t rows = (int64_t)(p.decode ? 1 : max_q_len) * p.group;
+  if (rows > INT32_MAX) rows = INT32_MAX;
   p.num_seqs = num_seqs;
   block_divisor(p.group, p.group_magic, p.group_shift);
   const int64_t nwg = f32_grid(num_seqs, p.num_kv_heads, rows, p.num_m_blocks, p.level_run,
