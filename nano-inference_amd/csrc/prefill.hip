@@ -1231,16 +1231,18 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillP
         if (s0 + i >= ranges) st[i][j] = make_float2(-INFINITY, 0.f);
         mn = fmaxf(mn, st[i][j].x);
       }
-      if (mn == -INFINITY) continue;  // no visible key so far
       const float corr = m[j] == -INFINITY ? 0.f : fast_exp2(m[j] - mn);
       l[j] *= corr;
       acc[j] *= corr;
       m[j] = mn;
 #pragma unroll
       for (int i = 0; i < kAhead; ++i) {
-        const float w = st[i][j].x == -INFINITY ? 0.f : fast_exp2(st[i][j].x - mn);
+        // a range without a visible key has m = -inf, l = 0; NaN scores leave m and make l NaN,
+        // and a NaN in o stays one at any weight, as in an uncut call
+        const bool any = st[i][j].x != -INFINITY;
+        const float w = any ? fast_exp2(st[i][j].x - mn) : 0.f;
         l[j] = fmaf(st[i][j].y, w, l[j]);
-        if (w > 0.f) acc[j] += o[i][j] * w;
+        if (any) acc[j] += o[i][j] * w;
       }
     }
   }
@@ -1248,7 +1250,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillP
   for (int j = 0; j < ROWS; ++j) {
     const int r = r0 + j * kStep;
     if (r > last) break;
-    const float inv = l[j] > 0.f ? 1.f / l[j] : 0.f;
+    const float inv = l[j] != 0.f ? 1.f / l[j] : 0.f;
     const int tok = tok_of(m0 + r);
     bf16_t* op = p.o + (qstart + tok) * p.o_tok + (int64_t)(h * pack + m0 + r - tok * pack) * p.o_head + d;
     *reinterpret_cast<uint2*>(op) = make_uint2(pack_bf16x2(acc[j][0] * inv, acc[j][1] * inv),

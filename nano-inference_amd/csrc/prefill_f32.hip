@@ -29,14 +29,12 @@
 // Against one head a block, tiles loaded behind a barrier each and the shortest blocks
 // first: four prompts of 128-1024 tokens (16 and 8 heads, D 128) 268 -> 186 us, one of 1000
 // 192 -> 114, four of 1000 551 -> 280.  The fp64 products bound it: v_mfma_f64_16x16x4 issues
-// every 115-128 cycles (probe; 64 at the nominal rate), so a
-// 16 x 32 tile is ~10k cycles, 4.3 us, and a second wave on the SIMD adds nothing.
-// v_mfma_f64_4x4x4 issues every 16.6 (1.7 times the rate), but with its keys broadcast over
+// every 115-128 cycles (probe; 64 at the nominal rate), so a 16 x 32 tile is ~10k cycles,
+// 4.3 us, and a second wave on the SIMD adds nothing.  v_mfma_f64_4x4x4 issues every 16.6 (1.7 times the rate), but with its keys broadcast over
 // the four blocks it reads and widens every K element four times (427 us for the four
 // prompts of 1000), and with the dims over the blocks and a reduce-scatter of the shares its
 // 32 accumulators spill 18 registers (363 us, bit-identical).
-// Both 16x16x4
-// MFMAs take A[l % 16][l / 16] and B[l / 16][l % 16] from lane l and give it column
+// Both 16x16x4 MFMAs take A[l % 16][l / 16] and B[l / 16][l % 16] from lane l and give it column
 // l % 16 of the 16x16 result; register i holds row 4 (l / 16) + i for fp32 and row
 // 4 i + l / 16 for fp64 (pinned on the device by an in-bounds probe):
 //   S^T = K Q^T (fp64): rows are keys, columns the wave's 16 queries; k step (c, i) of
@@ -460,11 +458,14 @@ __global__ __launch_bounds__(kF32Threads) void prefill_f32_merge_kernel(PrefillF
     const int64_t pr = s * step + prow;
     const double ms = p.part_m[pr];
     const f32x4_t o = *reinterpret_cast<const f32x4_t*>(p.part_o + pr * D + d);
-    const float w = ms == -INFINITY ? 0.f : fast_exp2((float)(ms - m));
+    // no visible key: m = -inf, l = 0; NaN scores leave m and make l NaN, and a NaN in o stays
+    // one at any weight, as in an uncut call
+    const bool any = ms != -INFINITY;
+    const float w = any ? fast_exp2((float)(ms - m)) : 0.f;
     l = fmaf(p.part_l[pr], w, l);
-    if (w > 0.f) acc += o * w;
+    if (any) acc += o * w;
   }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const float inv = l != 0.f ? 1.f / l : 0.f;
   const int tok = f32_tok(p, m0 + rr);
   float* o = static_cast<float*>(p.o) + (p.q_start[seq] + (int64_t)tok) * p.o_tok +
              (int64_t)(hk * p.group + m0 + rr - tok * p.group) * p.o_head + d;

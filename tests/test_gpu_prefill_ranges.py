@@ -133,6 +133,36 @@ def test_workspace_decides_and_never_fails():
     assert np.array_equal(outs[2][24:], outs[0][24:])  # the short sequence is never cut
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_nan_and_infinity_come_through_the_merge(dtype):
+    """A NaN query, a NaN value under a vanishing weight and an infinite key poison the rows
+    that an uncut call (no workspace) poisons, and no others."""
+    c = workloads.chunked_qwen3_8b("cuda", dtype=dtype, seed=96, n=1, chunk=24, prior=[3000],
+                                   num_heads=8, num_kv_heads=2)
+    c.q[3, 1] = float("nan")
+    c.q[:, 4:] *= 40  # the second KV head's group: weights that underflow
+    c.v_cache[c.tables_list[0][2], 1, 3, 5] = float("nan")
+    c.k_cache[c.tables_list[0][100], 0, 0] = float("inf")
+    lib, mb = _lib.load(), c.block_tables.shape[1]
+    code = ops._DTYPES[dtype]
+    need = lib.nia_prefill_split_workspace_size(1, 24, mb * 16, 8, 2, 128, ops.CAUSAL_BOTTOM_RIGHT,
+                                                code)
+    assert need > 0
+    ws, outs = torch.empty(need, dtype=torch.uint8, device="cuda"), []
+    for nbytes in (0, need):
+        out = torch.empty_like(c.q)
+        st = lib.nia_prefill_paged_split(
+            out.data_ptr(), out.stride(0), out.stride(1), c.q.data_ptr(), c.q.stride(0),
+            c.q.stride(1), c.k_cache.data_ptr(), c.v_cache.data_ptr(), c.block_tables.data_ptr(),
+            mb, mb, c.q_start.data_ptr(), c.q_len.data_ptr(), c.context_lens.data_ptr(), 1, 24, 8,
+            2, 128, 16, c.k_cache.shape[0], 1.0 / math.sqrt(128), ops.CAUSAL_BOTTOM_RIGHT, code,
+            ws.data_ptr() if nbytes else None, nbytes, torch.cuda.current_stream().cuda_stream)
+        assert st == _lib.OK
+        outs.append(out.float().cpu())
+    assert torch.isnan(outs[0][3, 1]).all() and torch.isnan(outs[0][:, 4:, 5]).any()
+    assert torch.equal(torch.isnan(outs[0]), torch.isnan(outs[1]))
+
+
 def test_captured_call_replays():
     """A cut call under HIP graph capture, replayed with eager calls in between."""
     c = workloads.chunked_qwen3_8b("cuda", seed=97, n=1, chunk=24, prior=[3000], num_heads=8,
