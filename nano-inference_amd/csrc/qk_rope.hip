@@ -141,11 +141,13 @@ NIA_DEVICE void store_codes(uint8_t* p, const Vec8<T>& x, float scale) {
   }
 }
 
+// Largest magnitude of a row's elements; NaN elements are left out, but a row of nothing else
+// keeps NaN (starting from 0 would turn it into a row of zeros).
 template <typename T>
 NIA_DEVICE float octet_amax(const Vec8<T>& a, const Vec8<T>& b) {
-  float m = 0.f;
+  float m = fmaxf(fabsf(Num<T>::f(a[0])), fabsf(Num<T>::f(b[0])));
 #pragma unroll
-  for (int i = 0; i < kHalf; ++i)
+  for (int i = 1; i < kHalf; ++i)
     m = fmaxf(m, fmaxf(fabsf(Num<T>::f(a[i])), fabsf(Num<T>::f(b[i]))));
   return octet_max(m);
 }

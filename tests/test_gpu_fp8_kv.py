@@ -308,3 +308,40 @@ def test_paged_layer_with_fp8_cache_matches_reference_pipeline():
         out, exp = step([meta.Query(L, t, meta.DECODE, blocks[i], bs)
                          for i, L in enumerate(prompts)], xd, False)
         close(out, exp, f"fp8 decode step {t}")
+
+
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_nan_rows_stay_nan(dtype, norm):
+    """A K or V row that is all NaN keeps a NaN scale (and zero codes), in the separate and in
+    the fused write; a lone NaN shows in its own element, or behind the norm in its whole row."""
+    g = torch.Generator().manual_seed(15)
+    n, hkv, nb, nan = 20, 4, 4, float("nan")
+    q = torch.randn(n, 8, 128, generator=g).to(dtype)
+    k, v = (torch.randn(n, hkv, 128, generator=g).to(dtype) for _ in range(2))
+    k[1, 0] = nan
+    v[2, 1] = nan
+    k[3, 2, 5] = nan
+    v[4, 3, 100] = nan
+    v[5] = nan
+    w = (torch.randn(128, generator=g) * 0.3 + 1).to(dtype).cuda() if norm else None
+    slots = torch.randperm(nb * 16, generator=g)[:n].cuda()
+    qg, kg, vg = q.cuda(), k.cuda(), v.cuda()
+    fused, apart = fp8_pool(nb, hkv), fp8_pool(nb, hkv)
+    ops.qk_norm_rope_kv_write(qg, kg, vg, w, w, 1e-6, torch.arange(n).cuda(),
+                              O.inv_freq(128, 1e6).cuda(), None, *fused[:2], slots, *fused[2:])
+    ops.kv_write(kg, vg, *apart[:2], slots, *apart[2:])
+    rows = [t.view(nb, hkv, 16, 128).transpose(1, 2).reshape(nb * 16, hkv, 128)[slots].cpu()
+            for t in fused[:2] + apart[:2]]
+    scales = [t.transpose(1, 2).reshape(nb * 16, hkv)[slots].cpu() for t in fused[2:] + apart[2:]]
+    for src, i in ((kg.cpu(), 0), (v, 1)):
+        code, scale = F.quantize_rows(src)
+        nans = torch.isnan(src.float())
+        whole = nans.all(-1)
+        assert whole.any() and torch.isnan(scale[whole]).all()
+        for c, s in ((rows[i], scales[i]), (rows[i + 2], scales[i + 2])):
+            assert torch.isnan(s[whole]).all() and not torch.isnan(s[~whole]).any()
+            assert torch.equal(c[whole], code[whole])
+            clean = ~nans.any(-1)
+            assert torch.equal(c[clean], code[clean]) and torch.equal(s[clean], scale[clean])
+            assert torch.equal(torch.isnan(F.dequantize_rows(c, s)), nans)
