@@ -670,15 +670,9 @@ __global__ __launch_bounds__(kDecodeThreads, 2) void decode_split_kernel(DecodeP
   const int64_t vw = (int64_t)blockIdx.x * wph + slice;
   const int64_t wt = Split::weight_before((int64_t)p.grid * wph, p.first_wgs, wl);
   int64_t ustart, uend;
-  // Few units (at most two per workgroup that has a CU to itself): one or two to a range, and
-  // only as many ranges as that takes.  Spread over every resident wave, a sequence's units
-  // would lie between empty ranges, which the merge walks as well: one sequence of 1023 keys
-  // (16 query, 8 KV heads) had 256 ranges to merge, 39.8 us; with one unit a range 10.3 us (two:
-  // 12.4, four: 16.4).  One sequence of 8192 keys (32 and 8 heads) 45.7 us before, 17.2 with one
-  // unit a range (two workgroups per CU), 15.3 with two, 17.7 with four.
   const int64_t alone = (int64_t)p.first_wgs * wph;
-  if (total <= 2 * alone) {
-    const int64_t per = total <= alone ? 1 : 2;
+  if (few_units(total, alone)) {
+    const int64_t per = few_units_a_range(total, alone);
     ustart = vw * per < total ? vw * per : total;
     uend = ustart + per < total ? ustart + per : total;
   } else {

@@ -44,8 +44,6 @@
 
 namespace {
 
-constexpr int kBlockM = 128;
-constexpr int kBlockN = 64;
 constexpr int kPrefillWaves = 4;
 constexpr int kPrefillThreads = kPrefillWaves * kWave;
 constexpr float kLazyRescaleP = 8.0f;
@@ -102,94 +100,8 @@ struct PrefillParams {
   float* part_ml;
 };
 
-// Key tiles of an m-block of `tiles` tiles are cut into this many ranges (kSplitMinTiles each
-// at least); range s takes tiles [tiles s / n, tiles (s + 1) / n).
-constexpr int kSplitMinTiles = 4;
-NIA_DEVICE int key_ranges(int tiles, int splits) {
-  return max(1, min(splits, tiles / kSplitMinTiles));
-}
-
-// Workgroup -> (sequence, head, m-block) mapping of the 1-D prefill grid.
-//
-// The hardware hands workgroups to the 8 XCDs round-robin (id % 8), and each
-// XCD has its own L2.  A (sequence, KV head) "group" owns the K/V rows that all
-// its m-blocks and its G query heads read, so every group is pinned to one XCD
-// (group % 8 == id % 8) and its K/V is fetched into one L2 only.  Inside an XCD
-// the workgroups go out m-block-major from the bottom of the causal triangle,
-// so the longest rows of every group start first and the short ones fill the
-// tail.  Ids that map past the real work (ragged sequences, uneven groups per
-// XCD) return false.
-// The hardware hands an XCD's workgroups to its shader engines in turn, whatever each still
-// has to do, so workgroups that follow each other must do about the same work: consecutive
-// ones are the heads of one group and level, or where a KV head's heads are packed into the
-// rows, kLevelRun adjacent levels of one group.  One level of every group in turn put each
-// sequence on one engine: causal prefill of eight sequences of 256-4096 tokens 585 us
-// instead of 320-335.
-constexpr int kXcds = 8;
-constexpr int kLevelRun = 4;
-
-NIA_DEVICE bool prefill_map(const PrefillParams& p, int& seq, int& h, int& mb) {
-  const int id = blockIdx.x;
-  const int x = id % kXcds;
-  const int t = id / kXcds;
-  // `run` workgroups of one group follow each other: its heads of one level, or (one head
-  // index per KV head) kLevelRun levels of it
-  const bool heads = p.map_group > 1;
-  const int run = heads ? p.map_group : kLevelRun;
-  const int per_z = p.groups_per_xcd * run;
-  const int z0 = t / per_z;
-  const int rem = t - z0 * per_z;
-  const int j = rem / run;
-  const int g = rem - j * run;
-  const int gid = x + kXcds * j;
-  const int z = heads ? z0 : z0 * kLevelRun + g;
-  if (z >= p.num_m_blocks || gid >= p.num_seqs * p.num_kv_heads) return false;
-  seq = gid / p.num_kv_heads;
-  h = (gid - seq * p.num_kv_heads) * p.map_group + (heads ? g : 0);
-  mb = p.num_m_blocks - 1 - z;
-  return true;
-}
-
-// Paired-head grids (one query head per KV head, short unmasked sequences): all head pairs
-// of a sequence on one XCD (sequence % 8), so the cache lines that two neighbouring pairs'
-// rows share (a D = 80 row is 160 bytes) are fetched into one L2 once.
-NIA_DEVICE bool pair_map(const PrefillParams& p, int& seq, int& h, int& mb) {
-  const int id = blockIdx.x;
-  const int x = id % kXcds;
-  const int t = id / kXcds;
-  const int j = t / p.num_kv_heads;
-  seq = x + kXcds * j;
-  h = t - j * p.num_kv_heads;
-  mb = 0;
-  return seq < p.num_seqs;
-}
-
-// Rank-major variant, for grids whose workgroups of one sequence all do about the same
-// work (non-causal calls, and chunks after a cached context): sequences are ranked by
-// key length (longest first), the groups of rank r go out before those of rank r + 1
-// on every XCD (a group still lives on one XCD), and a group's m-blocks go out longest
-// first.  Issuing the longest work first keeps a long sequence's workgroups out of the
-// last round of the grid.  s_order[r] is the sequence of rank r.
-constexpr int kOrderMaxSeqs = kPrefillThreads;  // one sequence per thread
-
-NIA_DEVICE bool prefill_map_ranked(const PrefillParams& p, const int* s_order, int& seq, int& h,
-                                   int& mb) {
-  const int id = blockIdx.x;
-  const int x = id % kXcds;
-  const int t = id / kXcds;
-  const int per_j = p.num_m_blocks * p.map_group;
-  const int j = t / per_j;
-  const int rem = t - j * per_j;
-  const int z = rem / p.map_group;
-  const int g = rem - z * p.map_group;
-  const int gid = x + kXcds * j;
-  if (j >= p.groups_per_xcd || gid >= p.num_seqs * p.num_kv_heads) return false;
-  const int r = gid / p.num_kv_heads;
-  seq = s_order[r];
-  h = (gid - r * p.num_kv_heads) * p.map_group + g;
-  mb = p.num_m_blocks - 1 - z;
-  return true;
-}
+// The maps of work_map.h; the ranked one takes one sequence per thread.
+constexpr int kOrderMaxSeqs = kPrefillThreads;
 
 // Sequences by descending key length (ties by index) into s_order[0 .. num_seqs), for
 // num_seqs <= kOrderMaxSeqs; every thread of the workgroup takes part.
@@ -228,9 +140,9 @@ NIA_DEVICE bool map_workgroup(const PrefillParams& p, int& seq, int& h, int& mb)
     __shared__ int s_key[kOrderMaxSeqs];
     __shared__ int s_order[kOrderMaxSeqs];
     rank_sequences<PAGED>(p, s_key, s_order);
-    return prefill_map_ranked(p, s_order, seq, h, mb);
+    return prefill_map_ranked(p, blockIdx.x, s_order, seq, h, mb);
   }
-  return prefill_map(p, seq, h, mb);
+  return prefill_map(p, blockIdx.x, seq, h, mb);
 }
 
 // XOR swizzle of the 4-key groups inside a transposed-V row (row = head dim d).
@@ -603,7 +515,7 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
   if constexpr (PAIR) asm volatile("" ::"s"(p.q_start), "s"(p.q_len), "s"(p.k_start), "s"(p.k_len));
   int seq, h, mb;
   if constexpr (PAIR) {
-    if (!pair_map(p, seq, h, mb)) return;
+    if (!pair_map(p, blockIdx.x, seq, h, mb)) return;
   } else {
     if (!map_workgroup<PAGED>(p, seq, h, mb)) return;
   }
@@ -665,8 +577,8 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
     ranges = key_ranges(tiles, p.splits);
     const int s = blockIdx.y;
     if (s >= ranges) return;
-    n_begin = tiles * s / ranges * kBlockN;
-    n_stop = min(n_end, tiles * (s + 1) / ranges * kBlockN);
+    n_begin = range_tile(tiles, s, ranges) * kBlockN;
+    n_stop = min(n_end, range_tile(tiles, s + 1, ranges) * kBlockN);
   }
 
   const int r0 = m0 + wrow * 32;
@@ -1270,78 +1182,6 @@ void launch_staged(const PrefillParams& p, dim3 grid, hipStream_t s) {
     nia_launch((prefill_kernel<D, PAGED>), grid, dim3(kPrefillThreads), s, p);
 }
 
-// Bytes that 16 consecutive packed rows of q span from the first one's token, head 0 of the
-// group: at most 15 / pack + 1 tokens further (one token's rows may straddle two groups).
-int64_t q_span_bytes(const PrefillParams& p, int32_t pack, int head_dim) {
-  const int64_t toks = pack == 1 ? 15 : 15 / pack + 1;
-  return 2 * (toks * p.q_tok + (pack - 1) * p.q_head + head_dim);
-}
-
-// Key ranges per m-block for a grid of nwg workgroups whose m-blocks have at most `tiles` key
-// tiles.  A lone workgroup takes about 1.1 us a tile, and the fp32 partials of a full chip's
-// 512 workgroups about 13.6 us to write and read back, so n ranges cost 1.1 tiles / n +
-// 13.6 n nwg / 512 us: least at n = sqrt(41 tiles / nwg).  At most what the chip holds at
-// once (two workgroups a CU), and none where fewer than kSplitGain tiles are saved (the
-// second launch).  A 64-row chunk after 8000 keys (32 and 8 heads) 145 us uncut, 30 in 31
-// ranges, 26 in 15; 24 rows after 16000 keys 279 -> 26; eight 40-row chunks after 500-8192
-// keys 139 -> 75; 1024 rows after 12000 keys 242 -> 216.  Top-left causal calls stay uncut:
-// their m-blocks average half the longest one's tiles, and a prompt of 2000 tokens (16 and 8
-// heads) in two ranges ran 42-44 us, uncut 38.
-constexpr int kSplitSlots = 512;
-constexpr int kSplitMax = 32;
-constexpr int kSplitGain = 12;
-
-int32_t split_count(int64_t nwg, int64_t tiles, int32_t causal) {
-  if (causal == NIA_CAUSAL_TOP_LEFT) return 1;
-  int64_t n = kSplitSlots / nwg;
-  if (n > kSplitMax) n = kSplitMax;
-  if (n > tiles / kSplitMinTiles) n = tiles / kSplitMinTiles;
-  while (n > 1 && n * n * nwg > 41 * tiles) --n;
-  return n < 2 || tiles * (n - 1) < kSplitGain * n ? 1 : (int32_t)n;
-}
-
-size_t split_bytes(int64_t nwg, int32_t splits, int head_dim) {
-  return splits > 1 ? (size_t)nwg * splits * kBlockM * ((size_t)head_dim + 2) * sizeof(float) : 0;
-}
-
-// Rows per item and m-blocks: the query heads of a KV head packed into the rows (p.pack =
-// group), or one head an item.
-void set_rows(PrefillParams& p, int max_q_len, bool packed) {
-  p.pack = packed ? p.group : 1;
-  p.map_group = packed ? 1 : p.group;
-  p.num_m_blocks = (int32_t)(((int64_t)max_q_len * p.pack + kBlockM - 1) / kBlockM);
-  block_divisor(p.pack, p.pack_magic, p.pack_shift);
-}
-
-// Blocks of 128 rows of a KV head's query heads: packed, and each head on its own.
-int64_t packed_blocks(const PrefillParams& p, int max_q_len) {
-  return ((int64_t)max_q_len * p.group + kBlockM - 1) / kBlockM;
-}
-int64_t head_blocks(const PrefillParams& p, int max_q_len) {
-  return ((int64_t)max_q_len + kBlockM - 1) / kBlockM * p.group;
-}
-
-// Whether an uncut call packs: where the heads' own blocks need more than one round of the
-// chip (two workgroups a CU) and packing saves a sixteenth of them.  Five prompts of 60-500
-// tokens (28 and 4 heads) 22.6 -> 20.3 us, eight of 100-800 (16 and 8) 26.7 -> 24.8; with
-// less to save, or a grid that fits the chip, the rows' divisions cost more than they bring
-// (one prompt of 900 tokens 20.6 -> 21.1 us, six 60-row chunks 9.9 -> 10.7).  A call that is cut
-// into key ranges packs whenever that saves a block: its blocks are what the ranges multiply.
-bool pack_uncut(const PrefillParams& p, int max_q_len) {
-  const int64_t own = head_blocks(p, max_q_len);
-  return packed_blocks(p, max_q_len) * 16 <= own * 15 &&
-         own * p.num_seqs * p.num_kv_heads > 512;
-}
-
-// The workgroups of a packed or unpacked grid.
-int64_t grid_size(const PrefillParams& p) {
-  const int64_t levels =
-      p.map_group > 1 || p.order_by_len
-          ? p.num_m_blocks
-          : ((int64_t)p.num_m_blocks + kLevelRun - 1) / kLevelRun * kLevelRun;
-  return (int64_t)kXcds * p.groups_per_xcd * p.map_group * levels;
-}
-
 // Caller memory for the key ranges' partials, and the longest key run (a bound).
 struct SplitArgs {
   void* ws = nullptr;
@@ -1376,14 +1216,15 @@ int launch_prefill(PrefillParams& p, int head_dim, int max_q_len, hipStream_t s,
   // packed rows: the lane offsets must fit 32 bits and not be negative
   const bool plain = !BIAS && dma_ok && (!PAGED || (p.bs % 16 == 0 && (p.bs & (p.bs - 1)) == 0));
   const bool packable = plain && p.q_head >= 0 && p.q_head < kMaxRowStride &&
-                        q_span_bytes(p, p.group, head_dim) <= INT32_MAX &&
+                        q_span_bytes(p.q_tok, p.q_head, p.group, head_dim) <= INT32_MAX &&
                         (int64_t)max_q_len * p.group <= INT32_MAX;
   p.splits = 1;
   int64_t nwg = 0;
   if (sp.ws && plain) {
-    set_rows(p, max_q_len, packable && packed_blocks(p, max_q_len) < head_blocks(p, max_q_len));
+    set_rows(p, max_q_len, packable && packed_blocks(p.group, max_q_len) < head_blocks(p.group, max_q_len));
     nwg = grid_size(p);
-    const int32_t n = split_count(nwg, (sp.max_k_len + kBlockN - 1) / kBlockN, p.causal);
+    const int32_t n = split_count(nwg, (sp.max_k_len + kBlockN - 1) / kBlockN,
+                                  p.causal == NIA_CAUSAL_TOP_LEFT);
     if (n > 1 && split_bytes(nwg, n, head_dim) <= sp.bytes) {
       p.splits = n;
       p.part_o = (float*)sp.ws;
@@ -1394,7 +1235,7 @@ int launch_prefill(PrefillParams& p, int head_dim, int max_q_len, hipStream_t s,
     set_rows(p, max_q_len, packable && pack_uncut(p, max_q_len));
     nwg = grid_size(p);
   }
-  p.q_span = (int32_t)q_span_bytes(p, p.pack, head_dim);
+  p.q_span = (int32_t)q_span_bytes(p.q_tok, p.q_head, p.pack, head_dim);
   if (nwg >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)nwg);
   switch (head_dim) {
@@ -1753,11 +1594,13 @@ extern "C" size_t nia_prefill_split_workspace_size(int32_t num_seqs, int32_t max
   PrefillParams p{};
   p.group = num_heads / num_kv_heads;
   if ((int64_t)max_q_len * p.group > INT32_MAX) return 0;
-  set_rows(p, max_q_len, packed_blocks(p, max_q_len) < head_blocks(p, max_q_len));
+  set_rows(p, max_q_len, packed_blocks(p.group, max_q_len) < head_blocks(p.group, max_q_len));
   p.groups_per_xcd = (int32_t)(((int64_t)num_seqs * num_kv_heads + kXcds - 1) / kXcds);
   p.order_by_len = causal != NIA_CAUSAL_TOP_LEFT && num_seqs <= kOrderMaxSeqs;
   const int64_t nwg = grid_size(p);
-  return split_bytes(nwg, split_count(nwg, (max_k_len + kBlockN - 1) / kBlockN, causal), head_dim);
+  return split_bytes(nwg, split_count(nwg, (max_k_len + kBlockN - 1) / kBlockN,
+                                      causal == NIA_CAUSAL_TOP_LEFT),
+                     head_dim);
 }
 
 extern "C" int32_t nia_prefill_split(

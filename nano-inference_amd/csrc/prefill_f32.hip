@@ -56,50 +56,18 @@ namespace {
 
 constexpr int kF32Waves = 4;
 constexpr int kF32Threads = kF32Waves * kWave;
-constexpr int kF32BlockM = 16 * kF32Waves;  // query rows per workgroup
-constexpr int kF32BlockN = 32;              // keys per LDS tile
-constexpr int kF32Xcds = 8;
+static_assert(kF32BlockM == 16 * kF32Waves, "16 rows a wave");
 
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
-
-// Element kinds: fp32 rows, bf16 rows, or a paged fp8 cache (e4m3 codes with one fp32
-// scale per cache row; q and o in bf16).  Every element is widened to fp32 in LDS (fp8 as
-// code * row scale in fp32, the rows the fp8 format stands for), so one kernel serves the
-// cache layouts the bf16 and fp8 kernels do not take: any block size, any group.
-// Key ranges of about kF32RangeTiles tiles, so that no workgroup is left behind on a long row
-// block (a tile takes 4.3 us and every workgroup's SIMDs are busy): four prompts of 128-1024
-// tokens 217 us uncut, 183-186 in ranges of 5, 8 or 12 tiles; one of 500 77 us, 51 / 47 / 64.
-// The caller leaves out calls whose blocks fill the chip (ops.py); the partials stay below
-// kF32MaxParts x 33 KB (135 MB).
-constexpr int kF32RangeTiles = 8;
-constexpr int kF32SplitTiles = 12;   // fewer at most: uncut (the merge is a second launch)
-constexpr int64_t kF32MaxParts = 4096;
-
-NIA_DEVICE int f32_ranges(int tiles, int splits) {
-  return max(1, min(splits, (tiles + kF32RangeTiles - 1) / kF32RangeTiles));
-}
-
-// The workgroup's (sequence, KV head, row block); false past the real work.
-NIA_DEVICE bool f32_map(const PrefillF32Params& p, int& seq, int& hk, int& m0) {
-  const int x = blockIdx.x % kF32Xcds;
-  const int wt = blockIdx.x / kF32Xcds;
-  const int per_level = p.groups_per_xcd * p.level_run;
-  const int lv = wt / per_level;
-  const int wrem = wt - lv * per_level;
-  const int gj = wrem / p.level_run;
-  const int gid = x + kF32Xcds * gj;
-  const int z = lv * p.level_run + (wrem - gj * p.level_run);
-  if (z >= p.num_m_blocks || gid >= p.num_seqs * p.num_kv_heads) return false;
-  seq = gid / p.num_kv_heads;
-  hk = gid - seq * p.num_kv_heads;
-  m0 = (p.num_m_blocks - 1 - z) * kF32BlockM;
-  return true;
-}
 
 NIA_DEVICE int f32_tok(const PrefillF32Params& p, int r) {
   return p.group == 1 ? r : key_block(r, p.group_magic, p.group_shift);
 }
 
+// Element kinds: fp32 rows, bf16 rows, or a paged fp8 cache (e4m3 codes with one fp32
+// scale per cache row; q and o in bf16).  Every element is widened to fp32 in LDS (fp8 as
+// code * row scale in fp32, the rows the fp8 format stands for), so one kernel serves the
+// cache layouts the bf16 and fp8 kernels do not take: any block size, any group.
 template <int D, bool PAGED, int E>
 __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32Params p) {
   static_assert(D % 16 == 0 && D <= 128, "head_dim a multiple of 16, at most 128");
@@ -115,7 +83,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
   __shared__ int sok[2][kF32BlockN];  // key of the tile lies in a valid block
 
   int seq, hk, m0;
-  if (!f32_map(p, seq, hk, m0)) return;
+  if (!f32_map(p, blockIdx.x, seq, hk, m0)) return;
   const int G = p.group;
   const int qlen = p.decode ? 1 : p.q_len[seq];
   const int64_t qstart = p.decode ? seq : p.q_start[seq];
@@ -141,8 +109,8 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
   const int tiles = (n_end + kF32BlockN - 1) / kF32BlockN;
   const int ranges = f32_ranges(tiles, p.splits);
   if ((int)blockIdx.y >= ranges) return;
-  const int n_begin = tiles * (int)blockIdx.y / ranges * kF32BlockN;
-  const int n_stop = min(n_end, tiles * ((int)blockIdx.y + 1) / ranges * kF32BlockN);
+  const int n_begin = range_tile(tiles, blockIdx.y, ranges) * kF32BlockN;
+  const int n_stop = min(n_end, range_tile(tiles, blockIdx.y + 1, ranges) * kF32BlockN);
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -428,7 +396,7 @@ template <int D, bool PAGED>
 __global__ __launch_bounds__(kF32Threads) void prefill_f32_merge_kernel(PrefillF32Params p) {
   constexpr int kLanes = 32;
   int seq, hk, m0;
-  if (!f32_map(p, seq, hk, m0)) return;
+  if (!f32_map(p, blockIdx.x, seq, hk, m0)) return;
   const int qlen = p.q_len[seq];
   const int rows = qlen * p.group;
   const int rr = blockIdx.y * (kF32Threads / kLanes) + threadIdx.x / kLanes;  // of the block
@@ -470,27 +438,6 @@ __global__ __launch_bounds__(kF32Threads) void prefill_f32_merge_kernel(PrefillF
   float* o = static_cast<float*>(p.o) + (p.q_start[seq] + (int64_t)tok) * p.o_tok +
              (int64_t)(hk * p.group + m0 + rr - tok * p.group) * p.o_head + d;
   *reinterpret_cast<float4*>(o) = make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
-}
-
-// The grid of a call's row blocks.
-int64_t f32_grid(int64_t num_seqs, int64_t num_kv_heads, int64_t rows, int32_t& m_blocks,
-                 int32_t& run, int32_t& groups_per_xcd) {
-  m_blocks = (int32_t)((rows + kF32BlockM - 1) / kF32BlockM);
-  run = m_blocks >= 4 ? 4 : 1;
-  groups_per_xcd = (int32_t)((num_seqs * num_kv_heads + kF32Xcds - 1) / kF32Xcds);
-  return (int64_t)kF32Xcds * groups_per_xcd * (((int64_t)m_blocks + run - 1) / run * run);
-}
-
-int32_t f32_split_count(int64_t nwg, int64_t max_k_len) {
-  const int64_t tiles = (max_k_len + kF32BlockN - 1) / kF32BlockN;
-  if (tiles < kF32SplitTiles) return 1;
-  int64_t n = (tiles + kF32RangeTiles - 1) / kF32RangeTiles;
-  if (n > kF32MaxParts / nwg) n = kF32MaxParts / nwg;
-  return n < 2 ? 1 : (int32_t)n;
-}
-
-size_t f32_split_bytes(int64_t nwg, int32_t n, int head_dim) {
-  return n > 1 ? (size_t)nwg * n * kF32BlockM * (sizeof(double) + (1 + head_dim) * sizeof(float)) : 0;
 }
 
 template <int D, bool PAGED>

@@ -1,0 +1,283 @@
+// Which work a workgroup takes: the row blocks, grids and key ranges of the prefill kernels and
+// the short unit ranges of the split decode.  Plain integer code for the device and for the
+// host (the launchers; tests compile this file with the host's compiler).  The maps are
+// templates over the kernels' parameter structs, whose fields they name.
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#ifdef __HIP__
+#define NIA_BOTH __host__ __device__ __forceinline__
+#else
+#define NIA_BOTH inline
+#endif
+
+template <typename T>
+NIA_BOTH T at_least(T x, T lo) { return x > lo ? x : lo; }
+template <typename T>
+NIA_BOTH T at_most(T x, T hi) { return x < hi ? x : hi; }
+
+// ---- division by a run-time constant --------------------------------------------------------
+
+// Division of 0 <= x < 2^31 by d >= 1 (a block size, a group) as mulhi(x, m) >> s: with
+// l = ceil(log2 d) and m = ceil(2^(31 + l) / d) (< 2^32 since d > 2^(l - 1)), m d - 2^(31 + l)
+// < d <= 2^l, so floor(x m / 2^(31 + l)) = floor(x / d) for every x < 2^31 (the round-up
+// method of Granlund and Montgomery, "Division by invariant integers using
+// multiplication", 1994).  For d = 2^k it is m = 2^31, s = k - 1: the shift by k.
+inline void block_divisor(int32_t d, uint32_t& m, int32_t& s) {
+  if (d <= 1) {  // no 32-bit m divides by 1: every key maps to block 0 (the kernels that
+    m = 0;        // use this take block sizes >= 4; block size 1 is routed elsewhere)
+    s = 0;
+    return;
+  }
+  int l = 1;
+  while ((int64_t)1 << l < d) ++l;
+  m = (uint32_t)((((uint64_t)1 << (31 + l)) + (uint64_t)d - 1) / (uint64_t)d);
+  s = l - 1;
+}
+
+// x / d under the divisor (m, s) of block_divisor.
+NIA_BOTH int key_block(int x, uint32_t m, int s) {
+  return (int)((uint32_t)((uint64_t)(uint32_t)x * m >> 32) >> s);
+}
+
+// ---- bf16 prefill ------------------------------------------------------------------------------
+
+constexpr int kBlockM = 128;  // query rows per workgroup
+constexpr int kBlockN = 64;   // keys per tile
+constexpr int kXcds = 8;
+constexpr int kLevelRun = 4;
+
+// Key tiles of an m-block of `tiles` tiles are cut into this many ranges (kSplitMinTiles each
+// at least); range s takes tiles [tiles s / n, tiles (s + 1) / n).
+constexpr int kSplitMinTiles = 4;
+NIA_BOTH int key_ranges(int tiles, int splits) {
+  return at_least(at_most(splits, tiles / kSplitMinTiles), 1);
+}
+
+// Workgroup -> (sequence, head, m-block) mapping of the 1-D prefill grid.
+//
+// The hardware hands workgroups to the 8 XCDs round-robin (id % 8), and each
+// XCD has its own L2.  A (sequence, KV head) "group" owns the K/V rows that all
+// its m-blocks and its G query heads read, so every group is pinned to one XCD
+// (group % 8 == id % 8) and its K/V is fetched into one L2 only.  Inside an XCD
+// the workgroups go out m-block-major from the bottom of the causal triangle,
+// so the longest rows of every group start first and the short ones fill the
+// tail.  Ids that map past the real work (ragged sequences, uneven groups per
+// XCD) return false.
+// The hardware hands an XCD's workgroups to its shader engines in turn, whatever each still
+// has to do, so workgroups that follow each other must do about the same work: consecutive
+// ones are the heads of one group and level, or where a KV head's heads are packed into the
+// rows, kLevelRun adjacent levels of one group.  One level of every group in turn put each
+// sequence on one engine: causal prefill of eight sequences of 256-4096 tokens 585 us
+// instead of 320-335.
+template <typename P>
+NIA_BOTH bool prefill_map(const P& p, int id, int& seq, int& h, int& mb) {
+  const int x = id % kXcds;
+  const int t = id / kXcds;
+  // `run` workgroups of one group follow each other: its heads of one level, or (one head
+  // index per KV head) kLevelRun levels of it
+  const bool heads = p.map_group > 1;
+  const int run = heads ? p.map_group : kLevelRun;
+  const int per_z = p.groups_per_xcd * run;
+  const int z0 = t / per_z;
+  const int rem = t - z0 * per_z;
+  const int j = rem / run;
+  const int g = rem - j * run;
+  const int gid = x + kXcds * j;
+  const int z = heads ? z0 : z0 * kLevelRun + g;
+  if (z >= p.num_m_blocks || gid >= p.num_seqs * p.num_kv_heads) return false;
+  seq = gid / p.num_kv_heads;
+  h = (gid - seq * p.num_kv_heads) * p.map_group + (heads ? g : 0);
+  mb = p.num_m_blocks - 1 - z;
+  return true;
+}
+
+// Paired-head grids (one query head per KV head, short unmasked sequences): all head pairs
+// of a sequence on one XCD (sequence % 8), so the cache lines that two neighbouring pairs'
+// rows share (a D = 80 row is 160 bytes) are fetched into one L2 once.
+template <typename P>
+NIA_BOTH bool pair_map(const P& p, int id, int& seq, int& h, int& mb) {
+  const int x = id % kXcds;
+  const int t = id / kXcds;
+  const int j = t / p.num_kv_heads;
+  seq = x + kXcds * j;
+  h = t - j * p.num_kv_heads;
+  mb = 0;
+  return seq < p.num_seqs;
+}
+
+// Rank-major variant, for grids whose workgroups of one sequence all do about the same
+// work (non-causal calls, and chunks after a cached context): sequences are ranked by
+// key length (longest first), the groups of rank r go out before those of rank r + 1
+// on every XCD (a group still lives on one XCD), and a group's m-blocks go out longest
+// first.  Issuing the longest work first keeps a long sequence's workgroups out of the
+// last round of the grid.  s_order[r] is the sequence of rank r.
+template <typename P>
+NIA_BOTH bool prefill_map_ranked(const P& p, int id, const int* s_order, int& seq, int& h,
+                                 int& mb) {
+  const int x = id % kXcds;
+  const int t = id / kXcds;
+  const int per_j = p.num_m_blocks * p.map_group;
+  const int j = t / per_j;
+  const int rem = t - j * per_j;
+  const int z = rem / p.map_group;
+  const int g = rem - z * p.map_group;
+  const int gid = x + kXcds * j;
+  if (j >= p.groups_per_xcd || gid >= p.num_seqs * p.num_kv_heads) return false;
+  const int r = gid / p.num_kv_heads;
+  seq = s_order[r];
+  h = (gid - r * p.num_kv_heads) * p.map_group + g;
+  mb = p.num_m_blocks - 1 - z;
+  return true;
+}
+
+// Bytes that 16 consecutive packed rows of q span from the first one's token, head 0 of the
+// group: at most 15 / pack + 1 tokens further (one token's rows may straddle two groups).
+inline int64_t q_span_bytes(int64_t q_tok, int64_t q_head, int32_t pack, int head_dim) {
+  const int64_t toks = pack == 1 ? 15 : 15 / pack + 1;
+  return 2 * (toks * q_tok + (pack - 1) * q_head + head_dim);
+}
+
+// Key ranges per m-block for a grid of nwg workgroups whose m-blocks have at most `tiles` key
+// tiles.  A lone workgroup takes about 1.1 us a tile, and the fp32 partials of a full chip's
+// 512 workgroups about 13.6 us to write and read back, so n ranges cost 1.1 tiles / n +
+// 13.6 n nwg / 512 us: least at n = sqrt(41 tiles / nwg).  At most what the chip holds at
+// once (two workgroups a CU), and none where fewer than kSplitGain tiles are saved (the
+// second launch).  A 64-row chunk after 8000 keys (32 and 8 heads) 145 us uncut, 30 in 31
+// ranges, 26 in 15; 24 rows after 16000 keys 279 -> 26; eight 40-row chunks after 500-8192
+// keys 139 -> 75; 1024 rows after 12000 keys 242 -> 216.  Top-left causal calls (`top_left`)
+// stay uncut: their m-blocks average half the longest one's tiles, and a prompt of 2000 tokens
+// (16 and 8 heads) in two ranges ran 42-44 us, uncut 38.
+constexpr int kSplitSlots = 512;
+constexpr int kSplitMax = 32;
+constexpr int kSplitGain = 12;
+
+inline int32_t split_count(int64_t nwg, int64_t tiles, bool top_left) {
+  if (top_left) return 1;
+  int64_t n = kSplitSlots / nwg;
+  if (n > kSplitMax) n = kSplitMax;
+  if (n > tiles / kSplitMinTiles) n = tiles / kSplitMinTiles;
+  while (n > 1 && n * n * nwg > 41 * tiles) --n;
+  return n < 2 || tiles * (n - 1) < kSplitGain * n ? 1 : (int32_t)n;
+}
+
+inline size_t split_bytes(int64_t nwg, int32_t splits, int head_dim) {
+  return splits > 1 ? (size_t)nwg * splits * kBlockM * ((size_t)head_dim + 2) * sizeof(float) : 0;
+}
+
+// Rows per item and m-blocks: the query heads of a KV head packed into the rows (p.pack =
+// group), or one head an item.
+template <typename P>
+void set_rows(P& p, int max_q_len, bool packed) {
+  p.pack = packed ? p.group : 1;
+  p.map_group = packed ? 1 : p.group;
+  p.num_m_blocks = (int32_t)(((int64_t)max_q_len * p.pack + kBlockM - 1) / kBlockM);
+  block_divisor(p.pack, p.pack_magic, p.pack_shift);
+}
+
+// Blocks of 128 rows of a KV head's query heads: packed, and each head on its own.
+inline int64_t packed_blocks(int32_t group, int max_q_len) {
+  return ((int64_t)max_q_len * group + kBlockM - 1) / kBlockM;
+}
+inline int64_t head_blocks(int32_t group, int max_q_len) {
+  return ((int64_t)max_q_len + kBlockM - 1) / kBlockM * group;
+}
+
+// Whether an uncut call packs: where the heads' own blocks need more than one round of the
+// chip (two workgroups a CU) and packing saves a sixteenth of them.  Five prompts of 60-500
+// tokens (28 and 4 heads) 22.6 -> 20.3 us, eight of 100-800 (16 and 8) 26.7 -> 24.8; with
+// less to save, or a grid that fits the chip, the rows' divisions cost more than they bring
+// (one prompt of 900 tokens 20.6 -> 21.1 us, six 60-row chunks 9.9 -> 10.7).  A call that is cut
+// into key ranges packs whenever that saves a block: its blocks are what the ranges multiply.
+template <typename P>
+bool pack_uncut(const P& p, int max_q_len) {
+  const int64_t own = head_blocks(p.group, max_q_len);
+  return packed_blocks(p.group, max_q_len) * 16 <= own * 15 &&
+         own * p.num_seqs * p.num_kv_heads > 512;
+}
+
+// The workgroups of a packed or unpacked grid.
+template <typename P>
+int64_t grid_size(const P& p) {
+  const int64_t levels =
+      p.map_group > 1 || p.order_by_len
+          ? p.num_m_blocks
+          : ((int64_t)p.num_m_blocks + kLevelRun - 1) / kLevelRun * kLevelRun;
+  return (int64_t)kXcds * p.groups_per_xcd * p.map_group * levels;
+}
+
+// ---- fp32 prefill ------------------------------------------------------------------------------
+
+constexpr int kF32BlockM = 64;  // packed rows (query token, head of the group) per workgroup
+constexpr int kF32BlockN = 32;  // keys per LDS tile
+
+// Key ranges of about kF32RangeTiles tiles, so that no workgroup is left behind on a long row
+// block (a tile takes 4.3 us and every workgroup's SIMDs are busy): four prompts of 128-1024
+// tokens 217 us uncut, 183-186 in ranges of 5, 8 or 12 tiles; one of 500 77 us, 51 / 47 / 64.
+// The caller leaves out calls whose blocks fill the chip (ops.py); the partials stay below
+// kF32MaxParts x 33 KB (135 MB).
+constexpr int kF32RangeTiles = 8;
+constexpr int kF32SplitTiles = 12;   // fewer at most: uncut (the merge is a second launch)
+constexpr int64_t kF32MaxParts = 4096;
+
+NIA_BOTH int f32_ranges(int tiles, int splits) {
+  return at_least(at_most(splits, (tiles + kF32RangeTiles - 1) / kF32RangeTiles), 1);
+}
+
+// The workgroup's (sequence, KV head, row block); false past the real work.
+template <typename P>
+NIA_BOTH bool f32_map(const P& p, uint32_t id, int& seq, int& hk, int& m0) {
+  const int x = id % kXcds;
+  const int wt = id / kXcds;
+  const int per_level = p.groups_per_xcd * p.level_run;
+  const int lv = wt / per_level;
+  const int wrem = wt - lv * per_level;
+  const int gj = wrem / p.level_run;
+  const int gid = x + kXcds * gj;
+  const int z = lv * p.level_run + (wrem - gj * p.level_run);
+  if (z >= p.num_m_blocks || gid >= p.num_seqs * p.num_kv_heads) return false;
+  seq = gid / p.num_kv_heads;
+  hk = gid - seq * p.num_kv_heads;
+  m0 = (p.num_m_blocks - 1 - z) * kF32BlockM;
+  return true;
+}
+
+// The grid of a call's row blocks.
+inline int64_t f32_grid(int64_t num_seqs, int64_t num_kv_heads, int64_t rows, int32_t& m_blocks,
+                        int32_t& run, int32_t& groups_per_xcd) {
+  m_blocks = (int32_t)((rows + kF32BlockM - 1) / kF32BlockM);
+  run = m_blocks >= 4 ? 4 : 1;
+  groups_per_xcd = (int32_t)((num_seqs * num_kv_heads + kXcds - 1) / kXcds);
+  return (int64_t)kXcds * groups_per_xcd * (((int64_t)m_blocks + run - 1) / run * run);
+}
+
+inline int32_t f32_split_count(int64_t nwg, int64_t max_k_len) {
+  const int64_t tiles = (max_k_len + kF32BlockN - 1) / kF32BlockN;
+  if (tiles < kF32SplitTiles) return 1;
+  int64_t n = (tiles + kF32RangeTiles - 1) / kF32RangeTiles;
+  if (n > kF32MaxParts / nwg) n = kF32MaxParts / nwg;
+  return n < 2 ? 1 : (int32_t)n;
+}
+
+inline size_t f32_split_bytes(int64_t nwg, int32_t n, int head_dim) {
+  return n > 1 ? (size_t)nwg * n * kF32BlockM * (sizeof(double) + (1 + head_dim) * sizeof(float)) : 0;
+}
+
+// ---- key tiles of a range (both kernels) ---------------------------------------------------------
+
+// First tile of range s of n, for `tiles` tiles.
+NIA_BOTH int range_tile(int tiles, int s, int n) { return tiles * s / n; }
+
+// ---- split decode: few units ---------------------------------------------------------------------
+
+// Few units (at most two per workgroup that has a CU to itself, `alone` ranges): one or two to a
+// range, and only as many ranges as that takes.  Spread over every resident wave, a sequence's units would lie between empty ranges,
+// which the merge walks as well: one sequence of 1023 keys (16 query, 8 KV heads) had 256 ranges
+// to merge, 39.8 us; with one unit a range 10.3 us (two: 12.4, four: 16.4).  One sequence of 8192
+// keys (32 and 8 heads) 45.7 us before, 17.2 with one unit a range (two workgroups per CU), 15.3
+// with two, 17.7 with four.
+NIA_BOTH bool few_units(int64_t total, int64_t alone) { return total <= 2 * alone; }
+
+NIA_BOTH int64_t few_units_a_range(int64_t total, int64_t alone) { return total <= alone ? 1 : 2; }
