@@ -119,9 +119,11 @@ def source_digest(paths) -> str:
     return h.hexdigest()
 
 
-DECODE_SOURCES = ("nano-inference_amd/csrc/paged_decode.hip", "nano-inference_amd/csrc/common.h")
-KV_WRITE_SOURCES = ("nano-inference_amd/csrc/kv_write.hip", "nano-inference_amd/csrc/common.h")
-PREFILL_SOURCES = ("nano-inference_amd/csrc/prefill.hip", "nano-inference_amd/csrc/common.h")
+_COMMON = ("nano-inference_amd/csrc/common.h", "nano-inference_amd/csrc/key_units.h")
+DECODE_SOURCES = ("nano-inference_amd/csrc/paged_decode.hip", *_COMMON)
+KV_WRITE_SOURCES = ("nano-inference_amd/csrc/kv_write.hip", *_COMMON)
+PREFILL_SOURCES = ("nano-inference_amd/csrc/prefill.hip", *_COMMON,
+                   "nano-inference_amd/csrc/work_map.h")
 
 
 def read_traffic(workload: str, sources=DECODE_SOURCES):

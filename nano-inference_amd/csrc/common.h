@@ -8,7 +8,7 @@
 #include <stdint.h>
 
 #include "../../include/nia_attn.h"
-#include "work_map.h"
+#include "key_units.h"
 
 typedef __bf16 bf16_t;
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));

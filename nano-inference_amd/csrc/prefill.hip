@@ -41,6 +41,7 @@
 
 #include "common.h"
 #include "prefill_f32.h"
+#include "work_map.h"
 
 namespace {
 

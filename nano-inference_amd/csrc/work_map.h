@@ -1,46 +1,17 @@
-// Which work a workgroup takes: the row blocks, grids and key ranges of the prefill kernels and
-// the short unit ranges of the split decode.  Plain integer code for the device and for the
-// host (the launchers; tests compile this file with the host's compiler).  The maps are
-// templates over the kernels' parameter structs, whose fields they name.
+// Which work a workgroup takes: the row blocks, grids and key ranges of the prefill kernels.
+// Plain integer code for the device and for the host, as key_units.h.  The maps are templates
+// over the kernels' parameter structs, whose fields they name.
 #pragma once
 
 #include <stddef.h>
 #include <stdint.h>
 
-#ifdef __HIP__
-#define NIA_BOTH __host__ __device__ __forceinline__
-#else
-#define NIA_BOTH inline
-#endif
+#include "key_units.h"
 
 template <typename T>
 NIA_BOTH T at_least(T x, T lo) { return x > lo ? x : lo; }
 template <typename T>
 NIA_BOTH T at_most(T x, T hi) { return x < hi ? x : hi; }
-
-// ---- division by a run-time constant --------------------------------------------------------
-
-// Division of 0 <= x < 2^31 by d >= 1 (a block size, a group) as mulhi(x, m) >> s: with
-// l = ceil(log2 d) and m = ceil(2^(31 + l) / d) (< 2^32 since d > 2^(l - 1)), m d - 2^(31 + l)
-// < d <= 2^l, so floor(x m / 2^(31 + l)) = floor(x / d) for every x < 2^31 (the round-up
-// method of Granlund and Montgomery, "Division by invariant integers using
-// multiplication", 1994).  For d = 2^k it is m = 2^31, s = k - 1: the shift by k.
-inline void block_divisor(int32_t d, uint32_t& m, int32_t& s) {
-  if (d <= 1) {  // no 32-bit m divides by 1: every key maps to block 0 (the kernels that
-    m = 0;        // use this take block sizes >= 4; block size 1 is routed elsewhere)
-    s = 0;
-    return;
-  }
-  int l = 1;
-  while ((int64_t)1 << l < d) ++l;
-  m = (uint32_t)((((uint64_t)1 << (31 + l)) + (uint64_t)d - 1) / (uint64_t)d);
-  s = l - 1;
-}
-
-// x / d under the divisor (m, s) of block_divisor.
-NIA_BOTH int key_block(int x, uint32_t m, int s) {
-  return (int)((uint32_t)((uint64_t)(uint32_t)x * m >> 32) >> s);
-}
 
 // ---- bf16 prefill ------------------------------------------------------------------------------
 
@@ -269,15 +240,3 @@ inline size_t f32_split_bytes(int64_t nwg, int32_t n, int head_dim) {
 
 // First tile of range s of n, for `tiles` tiles.
 NIA_BOTH int range_tile(int tiles, int s, int n) { return tiles * s / n; }
-
-// ---- split decode: few units ---------------------------------------------------------------------
-
-// Few units (at most two per workgroup that has a CU to itself, `alone` ranges): one or two to a
-// range, and only as many ranges as that takes.  Spread over every resident wave, a sequence's units would lie between empty ranges,
-// which the merge walks as well: one sequence of 1023 keys (16 query, 8 KV heads) had 256 ranges
-// to merge, 39.8 us; with one unit a range 10.3 us (two: 12.4, four: 16.4).  One sequence of 8192
-// keys (32 and 8 heads) 45.7 us before, 17.2 with one unit a range (two workgroups per CU), 15.3
-// with two, 17.7 with four.
-NIA_BOTH bool few_units(int64_t total, int64_t alone) { return total <= 2 * alone; }
-
-NIA_BOTH int64_t few_units_a_range(int64_t total, int64_t alone) { return total <= alone ? 1 : 2; }

@@ -1,9 +1,10 @@
-"""How the kernels divide their work, by the functions they run (csrc/work_map.h, compiled for
-the host): every (sequence, head, row block) is some workgroup's exactly once under each map,
-whatever remainder the groups and levels leave; the multiply-shift division that splits packed
-rows into (token, head) agrees with the true one; a DMA group of 16 packed rows stays within
-the span its buffer resource covers; ranges tile the key tiles in order and none is empty; and
-few decode units take no more ranges than there are workgroups alone on a CU."""
+"""How the kernels divide their work, by the functions they run (csrc/work_map.h and
+key_units.h, compiled for the host): every (sequence, head, row block) is some workgroup's
+exactly once under each map, whatever remainder the groups and levels leave; the
+multiply-shift division that splits packed rows into (token, head) agrees with the true one;
+a DMA group of 16 packed rows stays within the span its buffer resource covers; ranges tile
+the key tiles in order and none is empty; and few decode units take no more ranges than there
+are workgroups alone on a CU."""
 import ctypes
 import itertools
 import random

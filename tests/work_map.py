@@ -1,4 +1,4 @@
-"""nano-inference_amd/csrc/work_map.h compiled for the host: the functions by which the kernels
+"""nano-inference_amd/csrc/work_map.h (and key_units.h) compiled for the host: the functions by which the kernels
 and their launchers divide the work, callable from tests."""
 from __future__ import annotations
 
