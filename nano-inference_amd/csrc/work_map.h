@@ -35,8 +35,10 @@ NIA_BOTH int key_ranges(int tiles, int splits) {
 // (group % 8 == id % 8) and its K/V is fetched into one L2 only.  Inside an XCD
 // the workgroups go out m-block-major from the bottom of the causal triangle,
 // so the longest rows of every group start first and the short ones fill the
-// tail.  Ids that map past the real work (ragged sequences, uneven groups per
-// XCD) return false.
+// tail.  Ids that map past the real work (uneven groups per XCD) return false.
+// The grid holds no others: rounded up to whole runs of levels, three quarters of the packed
+// grid of 100 prompts of 60 tokens (16 and 8 heads) were empty workgroups, about 10 ns each: 44
+// us instead of 23, 300 of 20 tokens 94 instead of 29.
 // The hardware hands an XCD's workgroups to its shader engines in turn, whatever each still
 // has to do, so workgroups that follow each other must do about the same work: consecutive
 // ones are the heads of one group and level, or where a KV head's heads are packed into the
@@ -48,17 +50,18 @@ NIA_BOTH bool prefill_map(const P& p, int id, int& seq, int& h, int& mb) {
   const int x = id % kXcds;
   const int t = id / kXcds;
   // `run` workgroups of one group follow each other: its heads of one level, or (one head
-  // index per KV head) kLevelRun levels of it
+  // index per KV head) kLevelRun levels of it, fewer where the levels end
   const bool heads = p.map_group > 1;
   const int run = heads ? p.map_group : kLevelRun;
   const int per_z = p.groups_per_xcd * run;
   const int z0 = t / per_z;
   const int rem = t - z0 * per_z;
-  const int j = rem / run;
-  const int g = rem - j * run;
+  const int len = heads ? run : at_most(run, p.num_m_blocks - z0 * run);
+  const int j = rem / len;
+  const int g = rem - j * len;
   const int gid = x + kXcds * j;
   const int z = heads ? z0 : z0 * kLevelRun + g;
-  if (z >= p.num_m_blocks || gid >= p.num_seqs * p.num_kv_heads) return false;
+  if (gid >= p.num_seqs * p.num_kv_heads) return false;
   seq = gid / p.num_kv_heads;
   h = (gid - seq * p.num_kv_heads) * p.map_group + (heads ? g : 0);
   mb = p.num_m_blocks - 1 - z;
@@ -172,11 +175,7 @@ bool pack_uncut(const P& p, int max_q_len) {
 // The workgroups of a packed or unpacked grid.
 template <typename P>
 int64_t grid_size(const P& p) {
-  const int64_t levels =
-      p.map_group > 1 || p.order_by_len
-          ? p.num_m_blocks
-          : ((int64_t)p.num_m_blocks + kLevelRun - 1) / kLevelRun * kLevelRun;
-  return (int64_t)kXcds * p.groups_per_xcd * p.map_group * levels;
+  return (int64_t)kXcds * p.groups_per_xcd * p.map_group * p.num_m_blocks;
 }
 
 // ---- fp32 prefill ------------------------------------------------------------------------------
@@ -205,10 +204,11 @@ NIA_BOTH bool f32_map(const P& p, uint32_t id, int& seq, int& hk, int& m0) {
   const int per_level = p.groups_per_xcd * p.level_run;
   const int lv = wt / per_level;
   const int wrem = wt - lv * per_level;
-  const int gj = wrem / p.level_run;
+  const int len = at_most(p.level_run, p.num_m_blocks - lv * p.level_run);
+  const int gj = wrem / len;
   const int gid = x + kXcds * gj;
-  const int z = lv * p.level_run + (wrem - gj * p.level_run);
-  if (z >= p.num_m_blocks || gid >= p.num_seqs * p.num_kv_heads) return false;
+  const int z = lv * p.level_run + (wrem - gj * len);
+  if (gid >= p.num_seqs * p.num_kv_heads) return false;
   seq = gid / p.num_kv_heads;
   hk = gid - seq * p.num_kv_heads;
   m0 = (p.num_m_blocks - 1 - z) * kF32BlockM;
@@ -221,7 +221,7 @@ inline int64_t f32_grid(int64_t num_seqs, int64_t num_kv_heads, int64_t rows, in
   m_blocks = (int32_t)((rows + kF32BlockM - 1) / kF32BlockM);
   run = m_blocks >= 4 ? 4 : 1;
   groups_per_xcd = (int32_t)((num_seqs * num_kv_heads + kXcds - 1) / kXcds);
-  return (int64_t)kXcds * groups_per_xcd * (((int64_t)m_blocks + run - 1) / run * run);
+  return (int64_t)kXcds * groups_per_xcd * m_blocks;
 }
 
 inline int32_t f32_split_count(int64_t nwg, int64_t max_k_len) {

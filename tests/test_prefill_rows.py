@@ -32,6 +32,8 @@ def test_maps_cover_the_work_once(seqs, hkv, group, rows, packed, ranked):
     order = random.Random(rows).sample(range(seqs), seqs)
     got = wm.mapped(g, "ranked" if ranked else "dense", n, order)
     heads = hkv if packed else hkv * group
+    # no workgroup goes out for a level that no call has (an empty one costs what a short one does)
+    assert n == 8 * cdiv(seqs * hkv, 8) * (heads // hkv) * cdiv(rows * g.pack, 128)
     assert_covers(got, range(seqs), range(heads), range(cdiv(rows * (group if packed else 1), 128)))
 
 
@@ -40,6 +42,7 @@ def test_maps_cover_the_work_once(seqs, hkv, group, rows, packed, ranked):
 def test_other_maps_cover_the_work_once(seqs, hkv, blocks):
     g = wm.Grid(num_seqs=seqs, num_kv_heads=hkv)
     n = wm.lib().t_f32_grid(ctypes.byref(g), 64 * blocks - 3)
+    assert n == 8 * cdiv(seqs * hkv, 8) * blocks
     assert_covers([(s, h, m // 64) for s, h, m in wm.mapped(g, "f32", n)],
                   range(seqs), range(hkv), range(blocks))
     assert_covers(wm.mapped(g, "pair", 8 * cdiv(seqs, 8) * hkv), range(seqs), range(hkv), range(1))
