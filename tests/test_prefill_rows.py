@@ -37,6 +37,16 @@ def test_maps_cover_the_work_once(seqs, hkv, group, rows, packed, ranked):
     assert_covers(got, range(seqs), range(heads), range(cdiv(rows * (group if packed else 1), 128)))
 
 
+@pytest.mark.parametrize("seqs,hkv,group", [(3, 2, 4), (5, 4, 1), (9, 16, 1)])
+def test_longest_levels_go_out_first(seqs, hkv, group):
+    """Unpacked causal grids: a group's heads together, then the next shorter level of every
+    group.  Runs of levels of one group are for packed heads only: with one head per KV head
+    too they put long levels of the last groups behind short ones of the first."""
+    g, n = wm.grid(seqs, hkv, group, 1100, False)
+    levels = [m for _, _, m in wm.mapped(g, "dense", n)]
+    assert levels == sorted(levels, reverse=True)
+
+
 @pytest.mark.parametrize("seqs,hkv", [(1, 1), (3, 2), (9, 8), (17, 5)])
 @pytest.mark.parametrize("blocks", [1, 3, 4, 5, 9])
 def test_other_maps_cover_the_work_once(seqs, hkv, blocks):
