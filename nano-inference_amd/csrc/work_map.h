@@ -240,5 +240,9 @@ inline size_t f32_split_bytes(int64_t nwg, int32_t n, int head_dim) {
 
 // ---- key tiles of a range (both kernels) ---------------------------------------------------------
 
-// First tile of range s of n, for `tiles` tiles.
-NIA_BOTH int range_tile(int tiles, int s, int n) { return tiles * s / n; }
+// First tile of range s of n, floor(tiles s / n), for `tiles` tiles: the product itself does not
+// fit an int (2^26 tiles of 32 keys in up to 512 ranges; n is at most kF32MaxParts).
+NIA_BOTH int range_tile(int tiles, int s, int n) {
+  const int q = tiles / n;
+  return q * s + (tiles - q * n) * s / n;
+}

@@ -94,6 +94,10 @@ def test_ranges_tile_the_keys():
             assert cut[0] == 0 and cut[-1] == tiles
             least = 1 if f32 else 3
             assert n == 1 or all(b - a >= least for a, b in zip(cut, cut[1:]))
+    for tiles in (4194305, (1 << 26) - 1, 1 << 26):  # 2^31 keys in tiles of 32
+        for n in (32, 511, 512, 4096):
+            assert [lib.t_range_tile(tiles, s, n) for s in (0, 1, n // 2, n - 1, n)] == \
+                [tiles * s // n for s in (0, 1, n // 2, n - 1, n)]
 
 
 @pytest.mark.parametrize("alone", [256, 1024, 17])
