@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
   __shared__ int sok[2][kF32BlockN];  // key of the tile lies in a valid block
 
   int seq, hk, m0;
-  if (!f32_map(p, blockIdx.x, seq, hk, m0)) return;
+  if (!f32_map(p, blockIdx.x, blockIdx.y, blockIdx.z, seq, hk, m0)) return;
   const int G = p.group;
   const int qlen = p.decode ? 1 : p.q_len[seq];
   const int64_t qstart = p.decode ? seq : p.q_start[seq];
@@ -109,9 +109,10 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
   // keys [n_begin, n_stop) are this workgroup's
   const int tiles = (n_end + kF32BlockN - 1) / kF32BlockN;
   const int ranges = f32_ranges(tiles, p.splits);
-  if ((int)blockIdx.y >= ranges) return;
-  const int n_begin = range_tile(tiles, blockIdx.y, ranges) * kF32BlockN;
-  const int n_stop = min(n_end, range_tile(tiles, blockIdx.y + 1, ranges) * kF32BlockN);
+  const int range = p.splits > 1 ? (int)blockIdx.y : 0;  // uncut: y may be a KV head
+  if (range >= ranges) return;
+  const int n_begin = range_tile(tiles, range, ranges) * kF32BlockN;
+  const int n_stop = min(n_end, range_tile(tiles, range + 1, ranges) * kF32BlockN);
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -352,7 +353,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
   if (!row_ok) return;
   if (ranges > 1) {  // un-normalised, for prefill_f32_merge_kernel
     const int64_t prow =
-        ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kF32BlockM + (r - m0);
+        ((int64_t)range * gridDim.x + blockIdx.x) * kF32BlockM + (r - m0);
     if (slot == 0) {
       p.part_m[prow] = m_run;
       p.part_l[prow] = l_run;
@@ -397,7 +398,7 @@ template <int D, bool PAGED>
 __global__ __launch_bounds__(kF32Threads) void prefill_f32_merge_kernel(PrefillF32Params p) {
   constexpr int kLanes = 32;
   int seq, hk, m0;
-  if (!f32_map(p, blockIdx.x, seq, hk, m0)) return;
+  if (!f32_map(p, blockIdx.x, blockIdx.y, blockIdx.z, seq, hk, m0)) return;
   const int qlen = p.q_len[seq];
   const int rows = qlen * p.group;
   const int rr = blockIdx.y * (kF32Threads / kLanes) + threadIdx.x / kLanes;  // of the block
@@ -468,14 +469,13 @@ int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int nu
     return NIA_ERR_UNSUPPORTED;
   if (elem == kElemFp8 && (head_dim != 128 || !p.k_scale || !p.v_scale))
     return NIA_ERR_UNSUPPORTED;
-  // row numbers are ints: a longer bound than any call can fill sizes the grid for them all
+  // row numbers are ints
   int64_t rows = (int64_t)(p.decode ? 1 : max_q_len) * p.group;
   if (rows > INT32_MAX) rows = INT32_MAX;
   p.num_seqs = num_seqs;
   block_divisor(p.group, p.group_magic, p.group_shift);
   const int64_t nwg = f32_grid(num_seqs, p.num_kv_heads, rows, p.num_m_blocks, p.level_run,
                                p.groups_per_xcd);
-  if (nwg >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
   p.splits = 1;
   if (ws && elem == kElemF32 && !p.decode) {
     const int32_t n = f32_split_count(nwg, max_k_len);
@@ -487,7 +487,9 @@ int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int nu
       p.part_l = p.part_o + parts * head_dim;
     }
   }
-  const dim3 grid((unsigned)nwg);
+  const dim3 grid = p.level_run ? dim3((unsigned)nwg)
+                                : dim3((unsigned)p.num_m_blocks, (unsigned)p.num_kv_heads,
+                                       (unsigned)num_seqs);
   if (elem == kElemFp8) {
     nia_launch((prefill_f32_kernel<128, true, kElemFp8>), grid, dim3(kF32Threads), stream, p);
     return hipGetLastError() == hipSuccess ? NIA_OK : NIA_ERR_LAUNCH;

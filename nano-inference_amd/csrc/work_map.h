@@ -198,9 +198,17 @@ NIA_BOTH int f32_ranges(int tiles, int splits) {
   return at_least(at_most(splits, (tiles + kF32RangeTiles - 1) / kF32RangeTiles), 1);
 }
 
-// The workgroup's (sequence, KV head, row block); false past the real work.
+// The workgroup's (sequence, KV head, row block); false past the real work.  `id`: its number in
+// the 1-D grid, or x in a 3-D one (level_run 0) of row blocks, KV heads and sequences.
 template <typename P>
-NIA_BOTH bool f32_map(const P& p, uint32_t id, int& seq, int& hk, int& m0) {
+NIA_BOTH bool f32_map(const P& p, uint32_t id, uint32_t y, uint32_t z3, int& seq, int& hk,
+                      int& m0) {
+  if (p.level_run == 0) {
+    seq = (int)z3;
+    hk = (int)y;
+    m0 = (p.num_m_blocks - 1 - (int)id) * kF32BlockM;
+    return true;
+  }
   const int x = id % kXcds;
   const int wt = id / kXcds;
   const int per_level = p.groups_per_xcd * p.level_run;
@@ -217,13 +225,16 @@ NIA_BOTH bool f32_map(const P& p, uint32_t id, int& seq, int& hk, int& m0) {
   return true;
 }
 
-// The grid of a call's row blocks.
+// The row blocks of a call of at most `rows` packed rows a group, and their grid: 1-D, or 3-D
+// (run 0) where one dimension does not hold it (a loose row bound over very many sequences).
+// A sequence of more rows than a dimension holds blocks for would be a q of 2^30 rows.
 inline int64_t f32_grid(int64_t num_seqs, int64_t num_kv_heads, int64_t rows, int32_t& m_blocks,
                         int32_t& run, int32_t& groups_per_xcd) {
-  m_blocks = (int32_t)((rows + kF32BlockM - 1) / kF32BlockM);
-  run = m_blocks >= 4 ? 4 : 1;
+  m_blocks = (int32_t)at_most((rows + kF32BlockM - 1) / kF32BlockM, kMaxGroups);
   groups_per_xcd = (int32_t)((num_seqs * num_kv_heads + kXcds - 1) / kXcds);
-  return (int64_t)kXcds * groups_per_xcd * m_blocks;
+  const int64_t nwg = (int64_t)kXcds * groups_per_xcd * m_blocks;
+  run = nwg > kMaxGroups ? 0 : (m_blocks >= 4 ? 4 : 1);
+  return nwg;
 }
 
 inline int32_t f32_split_count(int64_t nwg, int64_t max_k_len) {

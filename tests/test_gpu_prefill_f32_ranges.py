@@ -73,3 +73,35 @@ def test_additive_mask_over_packed_heads():
     kd, vd = (x.repeat_interleave(h // hkv, 1) for x in (kd, vd))
     ref = torch.softmax(qd @ kd.transpose(2, 3) / math.sqrt(d) + mask.double(), -1) @ vd
     assert_attn_close(out.numpy(), ref.transpose(1, 2).reshape(b * s, h, d).numpy(), torch.float32)
+
+
+@pytest.mark.parametrize("paged", [False, True])
+def test_many_sequences_under_a_loose_row_bound(paged):
+    """2^24 row blocks of 256 threads: one grid dimension does not hold them."""
+    n, h, d, bound = 1024, 8, 64, 131072
+    g = torch.Generator().manual_seed(62)
+    ql = [1 + i % 3 if i % 100 == 7 else 0 for i in range(n)]
+    ql[n - 1] = 2
+    q, k, v = (torch.randn(sum(ql), h, d, generator=g) for _ in range(3))
+    at = torch.tensor([0] + ql[:-1]).cumsum(0).to(torch.int32)
+    lens = torch.tensor(ql, dtype=torch.int32)
+    if paged:
+        tables = torch.zeros(n, 1, dtype=torch.int32)
+        used = [s for s in range(n) if ql[s]]
+        cache = torch.zeros(2, len(used), h, 4, d)
+        for b, s in enumerate(used):
+            tables[s] = b
+            for i, x in enumerate((k, v)):
+                cache[i, b, :, :ql[s]] = x[at[s]:at[s] + ql[s]].transpose(0, 1)
+        kc, vc = cache.cuda()
+        out = ops.prefill_paged(q.cuda(), kc, vc, tables.cuda(), at.cuda(), lens.cuda(),
+                                lens.to(torch.int64).cuda(), bound, ops.CAUSAL_BOTTOM_RIGHT)
+    else:
+        out = ops.prefill(q.cuda(), k.cuda(), v.cuda(), at.cuda(), lens.cuda(), at.cuda(),
+                          lens.cuda(), bound, ops.CAUSAL_TOP_LEFT)
+    o = out.double().cpu().numpy()
+    res = tb.varlen(q.double().numpy(), k.double().numpy(), v.double().numpy(), at.numpy(), ql,
+                    at.numpy(), ql, 1.0 / math.sqrt(d), "top_left")
+    for s, (idx, ref) in res.items():
+        if ql[s]:
+            assert_attn_close(o[int(at[s]) + idx], ref, torch.float32, f"seq {s}")

@@ -58,6 +58,16 @@ def test_other_maps_cover_the_work_once(seqs, hkv, blocks):
     assert_covers(wm.mapped(g, "pair", 8 * cdiv(seqs, 8) * hkv), range(seqs), range(hkv), range(1))
 
 
+def test_fp32_grid_takes_three_dimensions_past_one():
+    """A dimension holds 2^24 - 1 workgroups of 256 threads."""
+    for seqs, rows, run in ((1023, 131072, 4), (1024, 131072, 0), (65535, 1 << 20, 0),
+                            (1, (1 << 31) - 1, 0), (8, (1 << 24) - 64 * 9, 4)):
+        g = wm.Grid(num_seqs=seqs, num_kv_heads=8)
+        n = wm.lib().t_f32_grid(ctypes.byref(g), rows)
+        assert g.level_run == run and g.num_m_blocks == min(cdiv(rows, 64), (1 << 24) - 1)
+        assert (n < 1 << 24) == (run > 0)
+
+
 def test_division_by_the_group():
     div = wm.lib().t_div
     rng = random.Random(5)

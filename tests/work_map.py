@@ -37,7 +37,7 @@ void t_map(const Grid* p, int kind, int n, const int* order, int* out) {
     const bool ok = kind == 0   ? prefill_map(*p, id, s, h, m)
                     : kind == 1 ? prefill_map_ranked(*p, id, order, s, h, m)
                     : kind == 2 ? pair_map(*p, id, s, h, m)
-                                : f32_map(*p, id, s, h, m);
+                                : f32_map(*p, id, 0, 0, s, h, m);
     out[0] = ok ? s : -1;
     out[1] = ok ? h : -1;
     out[2] = ok ? m : -1;
