@@ -10,10 +10,6 @@
 #define NIA_BOTH inline
 #endif
 
-// Workgroups of 256 threads along one dimension of a grid: HIP counts a dimension's threads in 32
-// bits, refuses 2^32 and wraps beyond (a grid of 2^24 + 3 workgroups ran three of them).
-constexpr int64_t kMaxGroups = ((int64_t)1 << 24) - 1;
-
 // Division of 0 <= x < 2^31 by d >= 1 (a block size, a group) as mulhi(x, m) >> s: with
 // l = ceil(log2 d) and m = ceil(2^(31 + l) / d) (< 2^32 since d > 2^(l - 1)), m d - 2^(31 + l)
 // < d <= 2^l, so floor(x m / 2^(31 + l)) = floor(x / d) for every x < 2^31 (the round-up

@@ -13,6 +13,10 @@ NIA_BOTH T at_least(T x, T lo) { return x > lo ? x : lo; }
 template <typename T>
 NIA_BOTH T at_most(T x, T hi) { return x < hi ? x : hi; }
 
+// Workgroups of 256 threads along one dimension of a grid: HIP counts a dimension's threads in 32
+// bits, refuses 2^32 and wraps beyond (a grid of 2^24 + 3 workgroups ran three of them).
+constexpr int64_t kMaxGroups = ((int64_t)1 << 24) - 1;
+
 // ---- bf16 prefill ------------------------------------------------------------------------------
 
 constexpr int kBlockM = 128;  // query rows per workgroup
