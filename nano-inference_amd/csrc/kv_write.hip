@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "work_map.h"
 
 namespace {
 
@@ -168,7 +169,7 @@ extern "C" int32_t nia_kv_write_fp8(const void* k, int64_t k_tok_stride, int64_t
   if (!aligned(k_cache, 2) || !aligned(v_cache, 2)) return NIA_ERR_MISALIGNED;
   const int64_t rows = 2 * (int64_t)num_tokens * num_kv_heads;
   const int64_t groups = (rows + kFp8Rows - 1) / kFp8Rows;
-  if (groups >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
+  if (groups > kMaxGroups) return NIA_ERR_UNSUPPORTED;
   const int64_t num_slots = num_blocks * block_size;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == NIA_DTYPE_BF16)
@@ -227,12 +228,13 @@ template <bool VEC>
 __global__ __launch_bounds__(kGatherThreads) void dequant_gather_fp8_kernel(GatherParams p) {
   constexpr int D = 128;
   const int s = blockIdx.y;
-  const int jb = blockIdx.x / p.parts;
-  const int part = blockIdx.x - jb * p.parts;
+  const uint32_t id = blockIdx.z * gridDim.x + blockIdx.x;  // past the table: past the context
+  const uint32_t jb = id / (uint32_t)p.parts;
+  const int part = (int)(id - jb * (uint32_t)p.parts);
   int64_t ctx = p.context_lens[s];
   const int64_t cap = (int64_t)p.max_blocks * p.block_size;
   ctx = ctx < 0 ? 0 : (ctx > cap ? cap : ctx);
-  if (p.k_start && blockIdx.x == 0 && threadIdx.x == 0) {
+  if (p.k_start && id == 0 && threadIdx.x == 0) {
     p.k_start[s] = (int32_t)(s * p.start);
     p.k_len[s] = (int32_t)ctx;
   }
@@ -309,9 +311,11 @@ int32_t launch_gather(GatherParams& p, int32_t batch, hipStream_t stream) {
   p.parts = (int32_t)((pieces + kGatherItems - 1) / kGatherItems);
   const int64_t groups = (int64_t)p.max_blocks * p.parts;
   if (groups >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
+  // a table too wide for one dimension: over two
+  const int64_t z = (groups + kMaxGroups - 1) / kMaxGroups;
   const bool vec = aligned(p.k_cache, 16) && aligned(p.v_cache, 16) && aligned(p.out_k, 16) &&
                    aligned(p.out_v, 16);
-  const dim3 grid((unsigned)groups, (unsigned)batch);
+  const dim3 grid((unsigned)((groups + z - 1) / z), (unsigned)batch, (unsigned)z);
   if (vec)
     nia_launch(dequant_gather_fp8_kernel<true>, grid, dim3(kGatherThreads), stream, p);
   else

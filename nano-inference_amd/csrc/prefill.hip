@@ -1237,7 +1237,7 @@ int launch_prefill(PrefillParams& p, int head_dim, int max_q_len, hipStream_t s,
     nwg = grid_size(p);
   }
   p.q_span = (int32_t)q_span_bytes(p.q_tok, p.q_head, p.pack, head_dim);
-  if (nwg >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
+  if (nwg > kMaxGroups) return NIA_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)nwg);
   switch (head_dim) {
 #define NIA_PREFILL_CASE(DD)                                                                 \
@@ -1395,7 +1395,7 @@ int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride
     p.num_m_blocks = 1;
     p.pack = 1;
     const int64_t nwg = (int64_t)kXcds * ((num_seqs + kXcds - 1) / kXcds) * p.num_kv_heads;
-    if (nwg >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
+    if (nwg > kMaxGroups) return NIA_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     switch (head_dim) {
 #define NIA_PAIR_CASE(DD)                                                                       \

@@ -30,6 +30,7 @@
 // With fp8 caches the rotated k row and the v row are stored as e4m3 codes with one
 // fp32 scale per row (max |x| / 448), as nia_kv_write_fp8 stores them.
 #include "common.h"
+#include "work_map.h"
 
 namespace {
 
@@ -330,7 +331,6 @@ int32_t launch_qk_norm_rope(
   if (head_dim != 128 || (dtype != NIA_DTYPE_BF16 && dtype != NIA_DTYPE_F32))
     return NIA_ERR_UNSUPPORTED;
   const int64_t rows = (int64_t)num_heads + num_kv_heads;
-  if (((int64_t)num_tokens * rows + 3) / 4 >= ((int64_t)1 << 31)) return NIA_ERR_UNSUPPORTED;
   RopeParams p{};
   p.q = q;
   p.q_tok = q_tok_stride;
@@ -369,6 +369,7 @@ int32_t launch_qk_norm_rope(
   p.parts = (int32_t)parts;
   p.part_rows = (int32_t)(per_part * kRowGroup);
   const int64_t wgs = ((int64_t)num_tokens * parts + kRopeWaves - 1) / kRopeWaves;
+  if (wgs > kMaxGroups) return NIA_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)wgs);
   const bool bf16 = dtype == NIA_DTYPE_BF16;

@@ -92,6 +92,23 @@ def test_validation_returns_codes_without_launching():
                                  10, 0.1, 2, 0, None) == _lib.ERR_UNSUPPORTED
 
 
+def test_grids_past_one_dimension_are_refused_without_launching():
+    """HIP wraps a grid of more than 2^32 threads along one dimension and runs what is left."""
+    lib = _lib.load()
+    p, n = ctypes.c_void_p(16), 1 << 18  # never dereferenced
+    for heads, hkv, causal, max_q in ((8, 8, 1, 1024), (16, 8, 1, 1024), (128, 128, 0, 64)):
+        for seqs, ok in ((n, False), (0, True)):
+            assert lib.nia_prefill(p, 8, 8, p, 8, 8, p, 8, 8, p, 8, 8, p, p, p, p, seqs, max_q,
+                                   heads, hkv, 128, 0.1, causal, 0, None) == \
+                (_lib.OK if ok else _lib.ERR_UNSUPPORTED)
+    assert lib.nia_kv_write_fp8(p, 8, 8, p, 8, 8, p, p, p, p, p, 1 << 25, 1, 128, 16, 10, 0,
+                                None) == _lib.ERR_UNSUPPORTED
+    # the fused write: four waves a workgroup, one token or more each
+    assert lib.nia_qk_norm_rope_kv_write(p, 1024, 128, p, 512, 128, p, 512, 128, None, None, 1e-6,
+                                         p, 8, 1, p, 0, 0, None, None, None, 1 << 26, 8, 4, 128,
+                                         16, 10, 0, None) == _lib.ERR_UNSUPPORTED
+
+
 def test_noalloc_decode_refuses_sizes_beyond_its_scratch_without_launching():
     lib = _lib.load()
     p = ctypes.c_void_p(16)  # never dereferenced: the size check comes first

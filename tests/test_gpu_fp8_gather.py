@@ -51,3 +51,25 @@ def test_gather(bs, hkv, lens, shift):
                 exp[i, t] = 0.0 if b < 0 else rows[b, :, t % bs]
         assert torch.equal(o.cpu().view(torch.int16),
                            exp.view(n * stride, hkv, d).view(torch.int16))
+
+
+def test_wide_table_of_single_rows():
+    """More table entries than one grid dimension has workgroups of 256 threads (2^24): a key a
+    block and one KV head."""
+    d, mb, length = 128, (1 << 24) + 3, 7
+    g = torch.Generator().manual_seed(9)
+    codes = torch.randint(0, 120, (8, 1, 1, d), generator=g).to(torch.uint8)
+    scale = torch.rand((8, 1, 1), generator=g) + 0.01
+    table = torch.zeros(mb, dtype=torch.int32)
+    table[:length] = torch.randperm(8, generator=g)[:length]
+    tb, cg, sg = table.cuda(), codes.cuda(), scale.cuda()
+    out = [torch.full((length, 1, d), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    ctx = torch.tensor([length], dtype=torch.int64, device="cuda")  # no row past it is written
+    st = _lib.load().nia_dequant_gather_fp8(
+        cg.data_ptr(), cg.data_ptr(), sg.data_ptr(), sg.data_ptr(), tb.data_ptr(), mb, mb,
+        ctx.data_ptr(), 1, 1, d, 1, 8, out[0].data_ptr(), out[1].data_ptr(), mb,
+        torch.cuda.current_stream().cuda_stream)
+    assert st == _lib.OK
+    rows = (codes.view(torch.float8_e4m3fn).float() * scale.unsqueeze(-1)).to(torch.bfloat16)
+    exp = rows[table[:length].long(), 0]
+    assert all(torch.equal(o.cpu(), exp) for o in out)
