@@ -389,7 +389,9 @@ int32_t nia_dequant_gather_fp8(const void* k_cache, const void* v_cache, const f
  * gathered and dequantised into the workspace (as nia_dequant_gather_fp8 does, keys in
  * blocks outside [0, num_blocks) as zero rows), then attended by nia_prefill.  `workspace`:
  * 256-byte aligned device memory of at least nia_prefill_paged_fp8_workspace_size(...)
- * bytes; nothing in it needs initialising.
+ * bytes; nothing in it needs initialising.  Arguments are checked before the gather is
+ * launched; a table without blocks (max_blocks_per_seq 0) is an invalid argument, a call
+ * without query rows returns NIA_OK at once.
  */
 size_t nia_prefill_paged_fp8_workspace_size(int32_t num_seqs, int32_t max_q_len,
                                             int32_t num_heads, int32_t num_kv_heads,

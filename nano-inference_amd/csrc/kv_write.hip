@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "prefill_args.h"
 #include "work_map.h"
 
 namespace {
@@ -412,46 +413,52 @@ extern "C" int32_t nia_prefill_paged_fp8(
     const int64_t* context_lens, int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
     int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int64_t num_blocks, float scale,
     int32_t causal, void* workspace, size_t workspace_bytes, void* stream) {
-  if (num_seqs < 0 || num_kv_heads <= 0 || max_blocks_per_seq < 0 ||
-      bt_stride < max_blocks_per_seq || block_size <= 0 || num_blocks < 0)
+  if (max_blocks_per_seq < 0 || bt_stride < max_blocks_per_seq || block_size <= 0 ||
+      num_blocks < 0)
     return NIA_ERR_INVALID_ARGUMENT;
   if (head_dim != 128) return NIA_ERR_UNSUPPORTED;
   const int64_t rows = (int64_t)max_blocks_per_seq * block_size;  // of a sequence
   const int64_t tok = (int64_t)num_kv_heads * head_dim;
+  // All that the attention refuses is refused before the gather is launched.  Its key rows and
+  // their index lie in the workspace: 256 stands for an aligned address in it.
+  const void* in_ws = (const void*)256;
+  bool empty = false;
+  int32_t st = check_prefill_args(
+      out, out_tok_stride, out_head_stride, q, q_tok_stride, q_head_stride, in_ws, tok, head_dim,
+      in_ws, tok, head_dim, q_start, q_len, (const int32_t*)in_ws, (const int32_t*)in_ws, num_seqs,
+      max_q_len, num_heads, num_kv_heads, head_dim, scale, causal, NIA_DTYPE_BF16, nullptr, 0, 0,
+      0, empty);
+  if (st != NIA_OK || empty) return st;
+  // a table without blocks leaves no key rows to attend
+  if (max_blocks_per_seq == 0) return NIA_ERR_INVALID_ARGUMENT;
   // the sequences' first rows are int32
   if (num_seqs > 65535 || rows > INT32_MAX || rows * num_seqs > INT32_MAX)
     return NIA_ERR_UNSUPPORTED;
   uint8_t* ws = (uint8_t*)workspace;
-  int32_t *k_start = nullptr, *k_len = nullptr;
-  uint8_t *keys = nullptr, *vals = nullptr, *split = nullptr;
-  size_t split_bytes = 0;
-  if (num_seqs > 0 && max_blocks_per_seq > 0) {
-    const size_t half =
-        (size_t)num_seqs * rows * num_kv_heads * head_dim * sizeof(bf16_t);
-    if (!ws || workspace_bytes < fp8_index_bytes(num_seqs) + 2 * half) return NIA_ERR_WORKSPACE;
-    if (!aligned(ws, 256)) return NIA_ERR_MISALIGNED;
-    k_start = (int32_t*)ws;
-    k_len = k_start + num_seqs;
-    keys = ws + fp8_index_bytes(num_seqs);
-    vals = keys + half;
-    split = vals + half;
-    split_bytes = workspace_bytes - (size_t)(split - ws);
-    GatherParams p{};
-    int32_t st = gather_params(p, k_cache, v_cache, k_scale, v_scale, block_tables, bt_stride,
-                               max_blocks_per_seq, context_lens, num_kv_heads, block_size,
-                               num_blocks, keys, vals);
-    if (st != NIA_OK) return st;
-    p.tok = tok;
-    p.head = head_dim;
-    p.seq = tok * rows;
-    p.k_start = k_start;
-    p.k_len = k_len;
-    p.start = rows;
-    st = launch_gather(p, num_seqs, (hipStream_t)stream);
-    if (st != NIA_OK) return st;
-  }
-  return nia_prefill_split(out, out_tok_stride, out_head_stride, q, q_tok_stride, q_head_stride, keys, tok,
-                     head_dim, vals, tok, head_dim, q_start, q_len, k_start, k_len, num_seqs,
-                     max_q_len, num_heads, num_kv_heads, head_dim, scale, causal, NIA_DTYPE_BF16,
-                     rows, split, split_bytes, stream);
+  const size_t half = (size_t)num_seqs * rows * num_kv_heads * head_dim * sizeof(bf16_t);
+  if (!ws || workspace_bytes < fp8_index_bytes(num_seqs) + 2 * half) return NIA_ERR_WORKSPACE;
+  if (!aligned(ws, 256)) return NIA_ERR_MISALIGNED;
+  int32_t* k_start = (int32_t*)ws;
+  int32_t* k_len = k_start + num_seqs;
+  uint8_t* keys = ws + fp8_index_bytes(num_seqs);
+  uint8_t* vals = keys + half;
+  uint8_t* split = vals + half;
+  const size_t split_bytes = workspace_bytes - (size_t)(split - ws);
+  GatherParams p{};
+  st = gather_params(p, k_cache, v_cache, k_scale, v_scale, block_tables, bt_stride,
+                     max_blocks_per_seq, context_lens, num_kv_heads, block_size, num_blocks, keys,
+                     vals);
+  if (st != NIA_OK) return st;
+  p.tok = tok;
+  p.head = head_dim;
+  p.seq = tok * rows;
+  p.k_start = k_start;
+  p.k_len = k_len;
+  p.start = rows;
+  st = launch_gather(p, num_seqs, (hipStream_t)stream);
+  if (st != NIA_OK) return st;
+  return nia_prefill_split(out, out_tok_stride, out_head_stride, q, q_tok_stride, q_head_stride,
+                           keys, tok, head_dim, vals, tok, head_dim, q_start, q_len, k_start, k_len,
+                           num_seqs, max_q_len, num_heads, num_kv_heads, head_dim, scale, causal,
+                           NIA_DTYPE_BF16, rows, split, split_bytes, stream);
 }

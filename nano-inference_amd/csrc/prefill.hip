@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "prefill_args.h"
 #include "prefill_f32.h"
 #include "work_map.h"
 
@@ -1285,6 +1286,43 @@ bool vec_ok_f32(const void* ptr, int64_t a, int64_t b) {
 
 }  // namespace
 
+int32_t check_prefill_args(const void* out, int64_t out_tok_stride, int64_t out_head_stride,
+                           const void* q, int64_t q_tok_stride, int64_t q_head_stride,
+                           const void* k, int64_t k_tok_stride, int64_t k_head_stride,
+                           const void* v, int64_t v_tok_stride, int64_t v_head_stride,
+                           const int32_t* q_start, const int32_t* q_len, const int32_t* k_start,
+                           const int32_t* k_len, int32_t num_seqs, int32_t max_q_len,
+                           int32_t num_heads, int32_t num_kv_heads, int32_t head_dim, float scale,
+                           int32_t causal, int32_t dtype, const float* mask,
+                           int64_t mask_seq_stride, int64_t mask_head_stride,
+                           int64_t mask_q_stride, bool& empty) {
+  empty = false;
+  if (num_seqs < 0 || max_q_len < 0 || num_heads <= 0 || num_kv_heads <= 0 ||
+      num_heads % num_kv_heads != 0)
+    return NIA_ERR_INVALID_ARGUMENT;
+  if (causal < NIA_CAUSAL_NONE || causal > NIA_CAUSAL_BOTTOM_RIGHT || !(scale > 0.f) ||
+      scale == INFINITY)
+    return NIA_ERR_INVALID_ARGUMENT;
+  if (num_seqs == 0 || max_q_len == 0) {
+    empty = true;
+    return NIA_OK;
+  }
+  if (!out || !q || !k || !v || !q_start || !q_len || !k_start || !k_len)
+    return NIA_ERR_INVALID_ARGUMENT;
+  if (!supported_head_dim(head_dim)) return NIA_ERR_UNSUPPORTED;
+  // the mask is read four keys (16 bytes) at a time
+  if (mask && ((uintptr_t)mask % 16 || mask_seq_stride % 4 || mask_head_stride % 4 ||
+               mask_q_stride % 4 || mask_seq_stride < 0 || mask_head_stride < 0 ||
+               mask_q_stride < 0))
+    return NIA_ERR_MISALIGNED;
+  if (dtype != NIA_DTYPE_F32 && dtype != NIA_DTYPE_BF16) return NIA_ERR_UNSUPPORTED;
+  const auto ok = dtype == NIA_DTYPE_F32 ? vec_ok_f32 : vec_ok;
+  if (!ok(q, q_tok_stride, q_head_stride) || !ok(k, k_tok_stride, k_head_stride) ||
+      !ok(v, v_tok_stride, v_head_stride) || !ok(out, out_tok_stride, out_head_stride))
+    return NIA_ERR_MISALIGNED;
+  return NIA_OK;
+}
+
 namespace {
 
 int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride, const void* q,
@@ -1297,26 +1335,14 @@ int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride
                       int32_t dtype, const float* mask, int64_t mask_seq_stride,
                       int64_t mask_head_stride, int64_t mask_q_stride, void* stream,
                       const SplitArgs& split = SplitArgs()) {
-  if (num_seqs < 0 || max_q_len < 0 || num_heads <= 0 || num_kv_heads <= 0 ||
-      num_heads % num_kv_heads != 0)
-    return NIA_ERR_INVALID_ARGUMENT;
-  if (causal < NIA_CAUSAL_NONE || causal > NIA_CAUSAL_BOTTOM_RIGHT || !(scale > 0.f) ||
-      scale == INFINITY)
-    return NIA_ERR_INVALID_ARGUMENT;
-  if (num_seqs == 0 || max_q_len == 0) return NIA_OK;
-  if (!out || !q || !k || !v || !q_start || !q_len || !k_start || !k_len)
-    return NIA_ERR_INVALID_ARGUMENT;
-  if (!supported_head_dim(head_dim)) return NIA_ERR_UNSUPPORTED;
-  // the mask is read four keys (16 bytes) at a time
-  if (mask && ((uintptr_t)mask % 16 || mask_seq_stride % 4 || mask_head_stride % 4 ||
-               mask_q_stride % 4 || mask_seq_stride < 0 || mask_head_stride < 0 ||
-               mask_q_stride < 0))
-    return NIA_ERR_MISALIGNED;
+  bool empty = false;
+  const int32_t st = check_prefill_args(
+      out, out_tok_stride, out_head_stride, q, q_tok_stride, q_head_stride, k, k_tok_stride,
+      k_head_stride, v, v_tok_stride, v_head_stride, q_start, q_len, k_start, k_len, num_seqs,
+      max_q_len, num_heads, num_kv_heads, head_dim, scale, causal, dtype, mask, mask_seq_stride,
+      mask_head_stride, mask_q_stride, empty);
+  if (st != NIA_OK || empty) return st;
   if (dtype == NIA_DTYPE_F32) {
-    if (!vec_ok_f32(q, q_tok_stride, q_head_stride) || !vec_ok_f32(k, k_tok_stride, k_head_stride) ||
-        !vec_ok_f32(v, v_tok_stride, v_head_stride) ||
-        !vec_ok_f32(out, out_tok_stride, out_head_stride))
-      return NIA_ERR_MISALIGNED;
     PrefillF32Params f{};
     f.o = (float*)out;
     f.o_tok = out_tok_stride;
@@ -1346,10 +1372,6 @@ int32_t prefill_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride
     return launch_prefill_f32(f, false, head_dim, num_seqs, max_q_len, (hipStream_t)stream,
                               kElemF32, split.ws, split.bytes, split.max_k_len);
   }
-  if (dtype != NIA_DTYPE_BF16) return NIA_ERR_UNSUPPORTED;
-  if (!vec_ok(q, q_tok_stride, q_head_stride) || !vec_ok(k, k_tok_stride, k_head_stride) ||
-      !vec_ok(v, v_tok_stride, v_head_stride) || !vec_ok(out, out_tok_stride, out_head_stride))
-    return NIA_ERR_MISALIGNED;
   PrefillParams p{};
   p.o = (bf16_t*)out;
   p.o_tok = out_tok_stride;

@@ -109,6 +109,37 @@ def test_grids_past_one_dimension_are_refused_without_launching():
                                          16, 10, 0, None) == _lib.ERR_UNSUPPORTED
 
 
+def test_fp8_prefill_refuses_before_it_gathers():
+    """Every argument is checked before the gather is launched (without a GPU a launch would
+    return ERR_LAUNCH); an empty call gathers nothing."""
+    lib = _lib.load()
+    p, ws = ctypes.c_void_p(16), ctypes.c_void_p(4096)  # never dereferenced
+    names = ("out ot oh q qt qh kc vc ks vs bt bts mb qs ql ctx n mq h hkv d bs nb scale causal ws "
+             "bytes st").split()
+    base = dict(zip(names, [p, 1024, 128, p, 1024, 128, p, p, p, p, p, 4, 4, p, p, p, 2, 8, 8, 4,
+                            128, 16, 10, 0.1, 2, ws, 1 << 30, None]))
+
+    def call(**kw):
+        return lib.nia_prefill_paged_fp8(*dict(base, **kw).values())
+
+    odd = ctypes.c_void_p(24)
+    for kw in (dict(mq=-1), dict(n=-1), dict(h=6), dict(h=0), dict(hkv=0), dict(causal=3),
+               dict(causal=-1), dict(scale=0.0), dict(scale=float("inf")),
+               dict(scale=float("nan")), dict(out=None), dict(q=None), dict(qs=None),
+               dict(ql=None), dict(ctx=None), dict(bt=None), dict(kc=None), dict(vs=None),
+               dict(bts=3), dict(bs=0), dict(nb=-1), dict(mb=0, bts=0)):
+        assert call(**kw) == _lib.ERR_INVALID_ARGUMENT, kw
+    for kw in (dict(q=odd), dict(out=odd), dict(qt=1020), dict(oh=4), dict(ws=odd),
+               dict(kc=ctypes.c_void_p(17))):
+        assert call(**kw) == _lib.ERR_MISALIGNED, kw
+    for kw in (dict(d=64), dict(n=65536), dict(mb=1 << 27, bts=1 << 27)):
+        assert call(**kw) == _lib.ERR_UNSUPPORTED, kw
+    for kw in (dict(ws=None), dict(bytes=4096)):
+        assert call(**kw) == _lib.ERR_WORKSPACE, kw
+    for kw in (dict(mq=0), dict(n=0)):
+        assert call(ws=None, **kw) == _lib.OK, kw
+
+
 def test_noalloc_decode_refuses_sizes_beyond_its_scratch_without_launching():
     lib = _lib.load()
     p = ctypes.c_void_p(16)  # never dereferenced: the size check comes first
