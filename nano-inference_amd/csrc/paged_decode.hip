@@ -336,7 +336,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void paged_decode_f32_kernel(Decode
     }
     const int h = hk * G + g;
     if (nparts == 1) {
-      ob[(int64_t)g * p.out_h + d] = lt > 0.f ? ot / lt : 0.f;
+      ob[(int64_t)g * p.out_h + d] = lt != 0.f ? ot / lt : 0.f;  // NaN stays NaN
     } else {
       const int64_t at = ((int64_t)b * p.num_heads + h) * p.max_parts + part;
       p.ws_o[at * D + d] = ot;
@@ -1162,17 +1162,18 @@ decode_split_combine_kernel(DecodeParams p, int batch) {
     float cm = m_run;
 #pragma unroll
     for (int i = 0; i < kCombineRows; ++i) cm = fmaxf(cm, ml[i].x);
-    if (cm == -INFINITY) continue;  // no keys so far
     const float corr = m_run == -INFINITY ? 0.f : fast_exp2(m_run - cm);
     l_run *= corr;
     acc.x *= corr;
     acc.y *= corr;
 #pragma unroll
     for (int i = 0; i < kCombineRows; ++i) {
-      // a range that saw no key has m = -inf and weight 0; its o is not read into the sum
-      const float w = ml[i].x == -INFINITY ? 0.f : fast_exp2(ml[i].x - cm);
+      // a range that saw no key has m = -inf, l = 0; its o is not read into the sum.  NaN scores
+      // leave m and make l NaN, and a NaN in o stays one at any weight, as in an uncut sequence
+      const bool any = ml[i].x != -INFINITY;
+      const float w = any ? fast_exp2(ml[i].x - cm) : 0.f;
       l_run = fmaf(ml[i].y, w, l_run);
-      if (w > 0.f) {
+      if (any) {
         acc.x = fmaf(o[i].x, w, acc.x);
         acc.y = fmaf(o[i].y, w, acc.y);
       }
@@ -1199,7 +1200,7 @@ decode_split_combine_kernel(DecodeParams p, int batch) {
       }
     }
   }
-  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+  const float inv = l_run != 0.f ? 1.f / l_run : 0.f;  // NaN stays NaN
   if (has_dims) *reinterpret_cast<uint32_t*>(out + d0) = pack_bf16x2(acc.x * inv, acc.y * inv);
 }
 
