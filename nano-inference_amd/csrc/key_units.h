@@ -41,3 +41,18 @@ NIA_BOTH int key_block(int x, uint32_t m, int s) {
 NIA_BOTH bool few_units(int64_t total, int64_t alone) { return total <= 2 * alone; }
 
 NIA_BOTH int64_t few_units_a_range(int64_t total, int64_t alone) { return total <= alone ? 1 : 2; }
+
+constexpr int kCombineRows = 16;  // partial rows a wave of the decode's merge takes at a time
+
+// Waves per (sequence, head) pair in the merge of a decode whose `ranges` hold `sequences`
+// (sequence, KV head group) pairs.  Few pairs (a small batch, whose sequences lie in many ranges)
+// leave the chip to it: with at most 256 pairs 16 waves each, at most 1024 four, i.e. at most
+// 4096 waves (half of what the chip holds): a sequence of 8000 keys among 23 of 100 (32 and 8
+// heads) 35 us with one wave a pair, 22 with four.  Four only where there are eight ranges a
+// sequence or more: with fewer the other three waves find nothing to do and cost their launch
+// (59 sequences of up to 238 keys, 16 and 8 heads, 13.7 us instead of 12.8).  The 2048 pairs of
+// 64 sequences of 32 heads, each in few ranges, keep one wave (190 us either way).
+inline int merge_waves(int64_t pairs, int64_t ranges, int64_t sequences) {
+  if (pairs <= 256) return 16;
+  return pairs <= 1024 && ranges >= 8 * sequences ? 4 : 1;
+}

@@ -1094,14 +1094,8 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_prefix_kernel(DecodePar
 // and the lane's two dims) and are merged online (running max, rescaled sums).  An empty
 // range inside a sequence wrote m = -inf there and adds nothing.  Pairs of empty
 // sequences get zeros; pairs finished by the split kernel are left alone.
-// WAVES > 1: a workgroup of that many waves per pair, wave w taking rows 16 w .. + 15 of
-// every 16 WAVES, merged through LDS; a pair of at most 16 rows is wave 0's alone.  Few
-// pairs (a small batch, whose sequences lie in many ranges) leave the chip to it: with at
-// most kCombineWide pairs 16 waves each, at most kCombineMid 4, i.e. at most 4096 waves
-// (half of what the chip holds).  32 sequences of 28 heads 53.1 -> 52.5 us; the 2048 pairs of
-// 64 sequences of 32 heads, each in few ranges, keep one wave (190 us either way).
-constexpr int kCombineRows = 16;
-constexpr int kCombineWide = 256, kCombineMid = 1024;
+// WAVES > 1 (merge_waves): a workgroup of that many waves per pair, wave w taking rows 16 w ..
+// + 15 of every 16 WAVES, merged through LDS; a pair of at most 16 rows is wave 0's alone.
 
 template <int D, int WAVES>
 __global__ __launch_bounds__(WAVES == 1 ? kCombineThreads : WAVES * kWave) void
@@ -1299,10 +1293,11 @@ int launch_split(DecodeParams& p, int batch, hipStream_t s) {
              batch);
   constexpr int kPairsPerGroup = kCombineThreads / kWave;
   const int64_t pairs = (int64_t)batch * p.num_heads;
-  if (pairs <= kCombineWide)
+  const int waves = merge_waves(pairs, (int64_t)grid * p.wph, (int64_t)batch * p.nhg);
+  if (waves == 16)
     nia_launch((decode_split_combine_kernel<D, 16>), dim3((unsigned)pairs), dim3(16 * kWave), s, p,
                batch);
-  else if (pairs <= kCombineMid)
+  else if (waves == 4)
     nia_launch((decode_split_combine_kernel<D, 4>), dim3((unsigned)pairs), dim3(4 * kWave), s, p,
                batch);
   else

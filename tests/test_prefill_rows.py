@@ -117,3 +117,11 @@ def test_few_decode_units_fill_no_more_ranges_than_stand_alone(alone):
         assert lib.t_few(total, alone)
         assert cdiv(total, lib.t_few_per(total, alone)) <= alone
     assert not lib.t_few(2 * alone + 1, alone)
+
+
+def test_decode_merge_takes_more_waves_only_for_many_ranges_a_sequence():
+    waves = wm.lib().t_merge_waves
+    assert waves(16, 512, 2) == waves(256, 512, 32) == 16
+    assert waves(28 * 36, 512, 36) == waves(32 * 32, 512, 2 * 32) == 4  # 14 and 8 ranges each
+    assert waves(16 * 59, 512, 2 * 59) == waves(9 * 90, 2048, 3 * 90) == 1  # 4 and 7
+    assert waves(32 * 64, 512, 64) == 1

@@ -65,6 +65,9 @@ int t_split_count(int64_t nwg, int64_t tiles, int top_left) {
 }
 int t_f32_split_count(int64_t nwg, int64_t keys) { return f32_split_count(nwg, keys); }
 int t_few(int64_t total, int64_t alone) { return few_units(total, alone); }
+int t_merge_waves(int64_t pairs, int64_t ranges, int64_t sequences) {
+  return merge_waves(pairs, ranges, sequences);
+}
 int64_t t_few_per(int64_t total, int64_t alone) { return few_units_a_range(total, alone); }
 }
 """
@@ -92,6 +95,7 @@ def lib():
     so.t_span.argtypes = [i64, i64, ctypes.c_int, ctypes.c_int]
     so.t_split_count.argtypes = [i64, i64, ctypes.c_int]
     so.t_f32_split_count.argtypes = [i64, i64]
+    so.t_merge_waves.argtypes = [i64, i64, i64]
     so.t_few.argtypes = [i64, i64]
     so.t_few_per.argtypes = [i64, i64]
     return so
