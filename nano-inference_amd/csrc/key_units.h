@@ -32,6 +32,8 @@ NIA_BOTH int key_block(int x, uint32_t m, int s) {
   return (int)((uint32_t)((uint64_t)(uint32_t)x * m >> 32) >> s);
 }
 
+constexpr int kCombineRows = 16;  // partial rows a wave of the decode's merge takes at a time
+
 // Few units (at most two per workgroup that has a CU to itself, `alone` ranges): one or two to a
 // range, and only as many ranges as that takes.  Spread over every resident wave, a sequence's
 // units would lie between empty ranges, which the merge walks as well: one sequence of 1023 keys
@@ -40,9 +42,13 @@ NIA_BOTH int key_block(int x, uint32_t m, int s) {
 // unit a range (two workgroups per CU), 15.3 with two, 17.7 with four.
 NIA_BOTH bool few_units(int64_t total, int64_t alone) { return total <= 2 * alone; }
 
-NIA_BOTH int64_t few_units_a_range(int64_t total, int64_t alone) { return total <= alone ? 1 : 2; }
-
-constexpr int kCombineRows = 16;  // partial rows a wave of the decode's merge takes at a time
+// Units a range, of `ranges` in all: two past `alone` (the merge is what they save), one where
+// the `sequences` (sequence, KV head group) pairs are short enough for a merge in one round
+// either way: 130 sequences of up to 141 keys (32 and 4 heads) 16.6 us with two, 15.3 with one.
+NIA_BOTH int64_t few_units_a_range(int64_t total, int64_t alone, int64_t ranges,
+                                   int64_t sequences) {
+  return total <= alone || (total <= ranges && total <= kCombineRows * sequences) ? 1 : 2;
+}
 
 // Waves per (sequence, head) pair in the merge of a decode whose `ranges` hold `sequences`
 // (sequence, KV head group) pairs.  Few pairs (a small batch, whose sequences lie in many ranges)

@@ -672,7 +672,8 @@ __global__ __launch_bounds__(kDecodeThreads, 2) void decode_split_kernel(DecodeP
   int64_t ustart, uend;
   const int64_t alone = (int64_t)p.first_wgs * wph;
   if (few_units(total, alone)) {
-    const int64_t per = few_units_a_range(total, alone);
+    const int64_t per =
+        few_units_a_range(total, alone, (int64_t)p.grid * wph, (int64_t)batch * p.nhg);
     ustart = vw * per < total ? vw * per : total;
     uend = ustart + per < total ? ustart + per : total;
   } else {

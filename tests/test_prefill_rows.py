@@ -4,7 +4,7 @@ exactly once under each map, whatever remainder the groups and levels leave; the
 multiply-shift division that splits packed rows into (token, head) agrees with the true one;
 a DMA group of 16 packed rows stays within the span its buffer resource covers; ranges tile
 the key tiles in order and none is empty; and few decode units take no more ranges than there
-are workgroups alone on a CU."""
+are, two to a range where that spares the merge a round."""
 import ctypes
 import itertools
 import random
@@ -111,11 +111,16 @@ def test_ranges_tile_the_keys():
 
 
 @pytest.mark.parametrize("alone", [256, 1024, 17])
-def test_few_decode_units_fill_no_more_ranges_than_stand_alone(alone):
+@pytest.mark.parametrize("resident", [1, 2])
+@pytest.mark.parametrize("sequences", [1, 7, 130])
+def test_few_decode_units_fit_the_ranges(alone, resident, sequences):
     lib = wm.lib()
     for total in {0, 1, 2, alone - 1, alone, alone + 1, 2 * alone - 1, 2 * alone}:
         assert lib.t_few(total, alone)
-        assert cdiv(total, lib.t_few_per(total, alone)) <= alone
+        per = lib.t_few_per(total, alone, resident * alone, sequences)
+        assert cdiv(total, per) <= resident * alone
+        # two units a range only where that spares the merge of a sequence a round
+        assert (per == 2) == (total > alone and (resident == 1 or total > 16 * sequences))
     assert not lib.t_few(2 * alone + 1, alone)
 
 

@@ -68,7 +68,9 @@ int t_few(int64_t total, int64_t alone) { return few_units(total, alone); }
 int t_merge_waves(int64_t pairs, int64_t ranges, int64_t sequences) {
   return merge_waves(pairs, ranges, sequences);
 }
-int64_t t_few_per(int64_t total, int64_t alone) { return few_units_a_range(total, alone); }
+int64_t t_few_per(int64_t total, int64_t alone, int64_t ranges, int64_t sequences) {
+  return few_units_a_range(total, alone, ranges, sequences);
+}
 }
 """
 
@@ -97,6 +99,7 @@ def lib():
     so.t_f32_split_count.argtypes = [i64, i64]
     so.t_merge_waves.argtypes = [i64, i64, i64]
     so.t_few.argtypes = [i64, i64]
+    so.t_few_per.argtypes = [i64, i64, i64, i64]
     so.t_few_per.argtypes = [i64, i64]
     return so
 
