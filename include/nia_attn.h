@@ -234,7 +234,8 @@ int32_t nia_prefill_paged(void* out, int64_t out_tok_stride, int64_t out_head_st
  * nia_prefill and nia_prefill_paged with caller memory: a call whose workgroups leave the
  * chip idle (few query rows over long keys) cuts each row block's keys into ranges that run
  * side by side and merges their fp32 partials from the workspace in a second launch.
- * `max_k_len`: a bound of the sequences' key counts (paged calls: the table width).
+ * `max_k_len`: the longest sequence's key count, or an estimate of it (paged calls take the
+ * table width): it chooses how many ranges there are, whatever the sequences then hold.
  * `workspace`: 256-byte aligned device memory; nia_prefill_split_workspace_size gives the
  * bytes that a call can use, 0 where it would not cut (enough rows, short keys).  A
  * null, unaligned or smaller workspace runs the call uncut.  Nothing in it needs

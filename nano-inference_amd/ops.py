@@ -476,9 +476,10 @@ _SPLIT_MAX_ROWS_F32 = 640 * 64
 
 
 def _split_workspace(n, max_q_len, keys, h, hkv, d, causal, dt, dev) -> Optional[torch.Tensor]:
-    """Memory for the key ranges of a prefill call with few query rows over long keys (the
-    callers ask _SPLIT_MIN_KEYS and _SPLIT_MAX_ROWS first), or None when the call runs uncut.  Allocated per call: the caching allocator then orders
-    its reuse by stream, under graph capture too."""
+    """Memory for the key ranges of a prefill call with few query rows over sequences of about
+    ``keys`` keys (the callers ask _SPLIT_MIN_KEYS and _SPLIT_MAX_ROWS first), or None when the
+    call runs uncut.  Allocated per call: the caching allocator then orders its reuse by stream,
+    under graph capture too."""
     nbytes = _lib.load().nia_prefill_split_workspace_size(n, max_q_len, keys, h, hkv, d, causal,
                                                           dt)
     return torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
@@ -561,13 +562,20 @@ def prefill(
         )
         _lib.check("nia_prefill_masked", st)
         return out
+    # The keys of a sequence choose its ranges: the lengths are on the device, so the longest
+    # query run where there are as many keys as queries, else the mean.  For the sum of 16
+    # sequences of 1000 keys, 32 rows each, the call was cut: 24.9 us instead of 22.2.
+    if keys == rows:
+        keys = max_q_len
+    elif n > 1:
+        keys = -(-keys // n)
     ws = None
     if dt != _lib.DTYPE_BF16:
         if rows * h <= _SPLIT_MAX_ROWS_F32:
             if causal == CAUSAL_TOP_LEFT:  # its rows see no key past their own position
                 keys = min(keys, max_q_len)
             ws = _split_workspace(n, max_q_len, keys, h, hkv, d, causal, dt, q.device)
-    elif causal != CAUSAL_TOP_LEFT and keys >= n * _SPLIT_MIN_KEYS and \
+    elif causal != CAUSAL_TOP_LEFT and keys >= _SPLIT_MIN_KEYS and \
             n * h * max_q_len <= _SPLIT_MAX_ROWS:
         ws = _split_workspace(n, max_q_len, keys, h, hkv, d, causal, dt, q.device)
     if ws is not None:

@@ -179,3 +179,19 @@ def test_captured_call_replays():
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
         assert torch.equal(ops.prefill_paged(*args), eager)
+
+
+@pytest.mark.parametrize("dtype,ql,kl,cut", [
+    (torch.bfloat16, [32] * 16, [1000] * 16, False), (torch.bfloat16, [64], [8000], True),
+    (torch.float32, [8] * 20, [100] * 20, False), (torch.float32, [200], [900], True),
+    (torch.float32, [30, 400, 10], [30, 400, 10], True), (torch.float32, [30] * 14, [30] * 14, False)])
+def test_ranges_are_chosen_for_one_sequence_not_for_the_sum(monkeypatch, dtype, ql, kl, cut):
+    """Many short sequences are not cut for the sum of their keys."""
+    seen, ask = [], ops._split_workspace
+    monkeypatch.setattr(ops, "_split_workspace", lambda *a: seen.append(ask(*a)) or seen[-1])
+    h, hkv, d = 16, 8, 128
+    q, k, v = (_randn((sum(n), m, d), 5).to(dtype).cuda() for n, m in ((ql, h), (kl, hkv), (kl, hkv)))
+    starts = [torch.tensor([0] + x[:-1]).cumsum(0).to(torch.int32).cuda() for x in (ql, kl)]
+    lens = [torch.tensor(x, dtype=torch.int32).cuda() for x in (ql, kl)]
+    ops.prefill(q, k, v, starts[0], lens[0], starts[1], lens[1], max(ql), ops.CAUSAL_NONE)
+    assert any(x is not None for x in seen) == cut
