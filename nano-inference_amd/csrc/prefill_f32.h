@@ -37,10 +37,9 @@ struct PrefillF32Params {
   int32_t decode;  // one query row per sequence: row s of q / o (q_start, q_len unused)
   double scale_log2;
   // set by launch_prefill_f32: r / group = key_block(r, magic, shift) for group > 1, the grid
-  int32_t num_seqs;
   uint32_t group_magic;
   int32_t group_shift;
-  int32_t num_m_blocks, level_run, groups_per_xcd;
+  int32_t num_m_blocks, level_run, groups;
   // key ranges per row block at most (grid y) and their partials, per (range, workgroup, row)
   int32_t splits;
   double* part_m;

@@ -25,9 +25,9 @@
 // other of two LDS stages (fp32, 512-byte rows, 16-byte chunk c of row r at c ^ (r & 15):
 // the K reads take one chunk of 16 rows, the V reads 16 chunks of one row, both without
 // bank conflicts).  Row blocks go out longest first, four levels of one (sequence, KV head)
-// after another (see prefill.hip on the shader engines) and every group on one XCD.
+// after another over all XCDs (f32_map).
 // Against one head a block, tiles loaded behind a barrier each and the shortest blocks
-// first: four prompts of 128-1024 tokens (16 and 8 heads, D 128) 268 -> 186 us, one of 1000
+// first: four prompts of 128-1024 tokens (16 and 8 heads, D 128) 268 -> 182 us, one of 1000
 // 192 -> 114, four of 1000 551 -> 280.  The fp64 products bound it: v_mfma_f64_16x16x4 issues
 // every 115-128 cycles (probe; 64 at the nominal rate), so a 16 x 32 tile is ~10k cycles,
 // 4.3 us, and a second wave on the SIMD adds nothing.  v_mfma_f64_4x4x4 issues every 16.6 (1.7 times the rate), but with its keys broadcast over
@@ -84,7 +84,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
   __shared__ int sok[2][kF32BlockN];  // key of the tile lies in a valid block
 
   int seq, hk, m0;
-  if (!f32_map(p, blockIdx.x, blockIdx.y, blockIdx.z, seq, hk, m0)) return;
+  f32_map(p, blockIdx.x, blockIdx.y, blockIdx.z, seq, hk, m0);
   const int G = p.group;
   const int qlen = p.decode ? 1 : p.q_len[seq];
   const int64_t qstart = p.decode ? seq : p.q_start[seq];
@@ -398,7 +398,7 @@ template <int D, bool PAGED>
 __global__ __launch_bounds__(kF32Threads) void prefill_f32_merge_kernel(PrefillF32Params p) {
   constexpr int kLanes = 32;
   int seq, hk, m0;
-  if (!f32_map(p, blockIdx.x, blockIdx.y, blockIdx.z, seq, hk, m0)) return;
+  f32_map(p, blockIdx.x, blockIdx.y, blockIdx.z, seq, hk, m0);
   const int qlen = p.q_len[seq];
   const int rows = qlen * p.group;
   const int rr = blockIdx.y * (kF32Threads / kLanes) + threadIdx.x / kLanes;  // of the block
@@ -454,10 +454,10 @@ void launch_f32_split(const PrefillF32Params& p, dim3 grid, hipStream_t s) {
 
 size_t prefill_f32_split_bytes(int32_t num_seqs, int64_t max_q_len, int64_t max_k_len,
                                int32_t num_heads, int32_t num_kv_heads, int head_dim) {
-  int32_t a, b, c;
+  int32_t a, b;
   int64_t rows = max_q_len * (num_heads / num_kv_heads);
   if (rows > INT32_MAX) rows = INT32_MAX;
-  const int64_t nwg = f32_grid(num_seqs, num_kv_heads, rows, a, b, c);
+  const int64_t nwg = f32_grid((int64_t)num_seqs * num_kv_heads, rows, a, b);
   return f32_split_bytes(nwg, f32_split_count(nwg, max_k_len), head_dim);
 }
 
@@ -472,10 +472,10 @@ int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int nu
   // row numbers are ints
   int64_t rows = (int64_t)(p.decode ? 1 : max_q_len) * p.group;
   if (rows > INT32_MAX) rows = INT32_MAX;
-  p.num_seqs = num_seqs;
   block_divisor(p.group, p.group_magic, p.group_shift);
-  const int64_t nwg = f32_grid(num_seqs, p.num_kv_heads, rows, p.num_m_blocks, p.level_run,
-                               p.groups_per_xcd);
+  const int64_t groups = (int64_t)num_seqs * p.num_kv_heads;
+  const int64_t nwg = f32_grid(groups, rows, p.num_m_blocks, p.level_run);
+  p.groups = (int32_t)at_most(groups, kMaxGroups);  // 1-D: no more than its workgroups
   p.splits = 1;
   if (ws && elem == kElemF32 && !p.decode) {
     const int32_t n = f32_split_count(nwg, max_k_len);

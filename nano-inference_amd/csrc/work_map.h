@@ -202,41 +202,41 @@ NIA_BOTH int f32_ranges(int tiles, int splits) {
   return at_least(at_most(splits, (tiles + kF32RangeTiles - 1) / kF32RangeTiles), 1);
 }
 
-// The workgroup's (sequence, KV head, row block); false past the real work.  `id`: its number in
-// the 1-D grid, or x in a 3-D one (level_run 0) of row blocks, KV heads and sequences.
+// The workgroup's (sequence, KV head, row block).  `id`: its number in the 1-D grid, or x in a
+// 3-D one (level_run 0) of row blocks, KV heads and sequences.  Runs of adjacent levels of one
+// (sequence, KV head) group follow each other, for the shader engines as in prefill_map; the
+// groups lie over all XCDs, since the matrix cores bound the tiles and not their loads: with
+// every group on one XCD, four groups left half the chip idle (690 rows of 28 and 4 heads, D 96,
+// 131 us instead of 73) and one XCD had the longest sequence to itself (seven of up to 775 rows of
+// 8 heads and one 298 instead of 187); four prompts of 128-1024 tokens (16 and 8 heads) 186 and
+// 182.
 template <typename P>
-NIA_BOTH bool f32_map(const P& p, uint32_t id, uint32_t y, uint32_t z3, int& seq, int& hk,
+NIA_BOTH void f32_map(const P& p, uint32_t id, uint32_t y, uint32_t z3, int& seq, int& hk,
                       int& m0) {
+  int z;
   if (p.level_run == 0) {
     seq = (int)z3;
     hk = (int)y;
-    m0 = (p.num_m_blocks - 1 - (int)id) * kF32BlockM;
-    return true;
+    z = (int)id;
+  } else {
+    const int per_level = p.groups * p.level_run;
+    const int lv = (int)id / per_level;
+    const int rem = (int)id - lv * per_level;
+    const int len = at_most(p.level_run, p.num_m_blocks - lv * p.level_run);
+    const int gid = rem / len;
+    z = lv * p.level_run + (rem - gid * len);
+    seq = gid / p.num_kv_heads;
+    hk = gid - seq * p.num_kv_heads;
   }
-  const int x = id % kXcds;
-  const int wt = id / kXcds;
-  const int per_level = p.groups_per_xcd * p.level_run;
-  const int lv = wt / per_level;
-  const int wrem = wt - lv * per_level;
-  const int len = at_most(p.level_run, p.num_m_blocks - lv * p.level_run);
-  const int gj = wrem / len;
-  const int gid = x + kXcds * gj;
-  const int z = lv * p.level_run + (wrem - gj * len);
-  if (gid >= p.num_seqs * p.num_kv_heads) return false;
-  seq = gid / p.num_kv_heads;
-  hk = gid - seq * p.num_kv_heads;
   m0 = (p.num_m_blocks - 1 - z) * kF32BlockM;
-  return true;
 }
 
 // The row blocks of a call of at most `rows` packed rows a group, and their grid: 1-D, or 3-D
 // (run 0) where one dimension does not hold it (a loose row bound over very many sequences).
 // A sequence of more rows than a dimension holds blocks for would be a q of 2^30 rows.
-inline int64_t f32_grid(int64_t num_seqs, int64_t num_kv_heads, int64_t rows, int32_t& m_blocks,
-                        int32_t& run, int32_t& groups_per_xcd) {
+inline int64_t f32_grid(int64_t groups, int64_t rows, int32_t& m_blocks, int32_t& run) {
   m_blocks = (int32_t)at_most((rows + kF32BlockM - 1) / kF32BlockM, kMaxGroups);
-  groups_per_xcd = (int32_t)((num_seqs * num_kv_heads + kXcds - 1) / kXcds);
-  const int64_t nwg = (int64_t)kXcds * groups_per_xcd * m_blocks;
+  const int64_t nwg = groups * m_blocks;
   run = nwg > kMaxGroups ? 0 : (m_blocks >= 4 ? 4 : 1);
   return nwg;
 }

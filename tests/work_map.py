@@ -17,7 +17,7 @@ SHIM = r"""
 #include "work_map.h"
 struct Grid {
   int32_t num_seqs, num_kv_heads, group, map_group, num_m_blocks, groups_per_xcd, order_by_len;
-  int32_t pack, pack_shift, level_run;
+  int32_t pack, pack_shift, level_run, groups;
   uint32_t pack_magic;
 };
 extern "C" {
@@ -27,8 +27,8 @@ int64_t t_grid(Grid* p, int max_q_len, int packed) {
   return grid_size(*p);
 }
 int64_t t_f32_grid(Grid* p, int64_t rows) {
-  return f32_grid(p->num_seqs, p->num_kv_heads, rows, p->num_m_blocks, p->level_run,
-                  p->groups_per_xcd);
+  p->groups = p->num_seqs * p->num_kv_heads;
+  return f32_grid(p->groups, rows, p->num_m_blocks, p->level_run);
 }
 // kind 0: prefill_map, 1: ranked, 2: pair, 3: fp32; out[id] = seq, head, block or -1s
 void t_map(const Grid* p, int kind, int n, const int* order, int* out) {
@@ -37,7 +37,7 @@ void t_map(const Grid* p, int kind, int n, const int* order, int* out) {
     const bool ok = kind == 0   ? prefill_map(*p, id, s, h, m)
                     : kind == 1 ? prefill_map_ranked(*p, id, order, s, h, m)
                     : kind == 2 ? pair_map(*p, id, s, h, m)
-                                : f32_map(*p, id, 0, 0, s, h, m);
+                                : (f32_map(*p, id, 0, 0, s, h, m), true);
     out[0] = ok ? s : -1;
     out[1] = ok ? h : -1;
     out[2] = ok ? m : -1;
@@ -78,7 +78,7 @@ int64_t t_few_per(int64_t total, int64_t alone, int64_t ranges, int64_t sequence
 class Grid(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int32) for n in (
         "num_seqs", "num_kv_heads", "group", "map_group", "num_m_blocks", "groups_per_xcd",
-        "order_by_len", "pack", "pack_shift", "level_run")] + [("pack_magic", ctypes.c_uint32)]
+        "order_by_len", "pack", "pack_shift", "level_run", "groups")] + [("pack_magic", ctypes.c_uint32)]
 
 
 @functools.lru_cache(maxsize=None)
