@@ -20,20 +20,23 @@
 // and 2 D in fp32 (157), 4096 + 2048 cycles of a SIMD for a wave's 16 x 32 tile at D = 128.
 // Tiling: a workgroup of 4 waves owns 64 packed rows (16 per wave): row r is query token
 // r / G, head r % G of a KV head's G query heads, so the heads of a group share their K/V
-// tiles and a decode's G heads fill one wave's columns.  Key tiles of 32 rows are loaded
-// into registers one tile ahead, while the tile before is computed on, and written to the
-// other of two LDS stages (fp32, 512-byte rows, 16-byte chunk c of row r at c ^ (r & 15):
-// the K reads take one chunk of 16 rows, the V reads 16 chunks of one row, both without
-// bank conflicts).  Row blocks go out longest first, four levels of one (sequence, KV head)
-// after another over all XCDs (f32_map).
+// tiles and a decode's G heads fill one wave's columns.  Key tiles of 32 rows are staged in LDS
+// (fp32, 16-byte chunks permuted within a row: swz).  D 128, whose registers leave two
+// workgroups a CU: a tile is loaded into registers while the one before is computed on, and
+// written to the other of two stages; operands are read from LDS a step ahead.  Smaller D: one
+// stage and no read-ahead, which leaves room for three workgroups a CU (D 64: four) that hide
+// each other's loads: four images of 784-3072 rows (16 heads of 80) 1633 us with two stages and
+// two workgroups, 1528 so, 114 windows of 16-64 rows 61.5 and 52.0 (54 with 512-byte rows left
+// out but two stages kept), 109 decodes of up to 40 keys (16 heads of 64) 27.7 and 18.1.
 // Against one head a block, tiles loaded behind a barrier each and the shortest blocks
 // first: four prompts of 128-1024 tokens (16 and 8 heads, D 128) 268 -> 182 us, one of 1000
 // 192 -> 114, four of 1000 551 -> 280.  The fp64 products bound it: v_mfma_f64_16x16x4 issues
 // every 115-128 cycles (probe; 64 at the nominal rate), so a 16 x 32 tile is ~10k cycles,
-// 4.3 us, and a second wave on the SIMD adds nothing.  v_mfma_f64_4x4x4 issues every 16.6 (1.7 times the rate), but with its keys broadcast over
-// the four blocks it reads and widens every K element four times (427 us for the four
-// prompts of 1000), and with the dims over the blocks and a reduce-scatter of the shares its
-// 32 accumulators spill 18 registers (363 us, bit-identical).
+// 4.3 us, and a second wave on the SIMD adds nothing.  v_mfma_f64_4x4x4 issues every 16.6 (1.7
+// times the rate), but with its keys broadcast over the four blocks it reads and widens every
+// K element four times (427 us for the four prompts of 1000), and with the dims over the blocks
+// and a reduce-scatter of the shares its 32 accumulators spill 18 registers (363 us,
+// bit-identical).
 // Both 16x16x4 MFMAs take A[l % 16][l / 16] and B[l / 16][l % 16] from lane l and give it column
 // l % 16 of the 16x16 result; register i holds row 4 (l / 16) + i for fp32 and row
 // 4 i + l / 16 for fp64 (pinned on the device by an in-bounds probe):
@@ -65,23 +68,29 @@ NIA_DEVICE int f32_tok(const PrefillF32Params& p, int r) {
   return p.group == 1 ? r : key_block(r, p.group_magic, p.group_shift);
 }
 
+template <int D>
+constexpr int kF32PerSimd = D == 64 ? 4 : D < 128 ? 3 : 2;  // waves a SIMD: workgroups a CU
+
 // Element kinds: fp32 rows, bf16 rows, or a paged fp8 cache (e4m3 codes with one fp32
 // scale per cache row; q and o in bf16).  Every element is widened to fp32 in LDS (fp8 as
 // code * row scale in fp32, the rows the fp8 format stands for), so one kernel serves the
 // cache layouts the bf16 and fp8 kernels do not take: any block size, any group.
 template <int D, bool PAGED, int E>
-__global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32Params p) {
+__global__ __launch_bounds__(kF32Threads, kF32PerSimd<D>) void prefill_f32_kernel(
+    PrefillF32Params p) {
   static_assert(D % 16 == 0 && D <= 128, "head_dim a multiple of 16, at most 128");
   static_assert(E == kElemF32 || PAGED, "bf16 and fp8 elements come from a paged cache");
-  constexpr int kRow = 128;        // LDS row stride in floats, whatever D is
+  constexpr int kRow = D;          // LDS row stride in floats
   constexpr int kC4 = D / 4;       // 16-byte chunks per row
   constexpr int kTiles = D / 16;   // output tiles
   constexpr int kQuads = D / 64;   // groups of four tiles read by 16-byte chunks
   constexpr int kChunks = kF32BlockN * kC4;  // per operand
   constexpr int kItems = (kChunks + kF32Threads - 1) / kF32Threads;  // of a thread
-  __shared__ __attribute__((aligned(16))) float sk[2][kF32BlockN * kRow];
-  __shared__ __attribute__((aligned(16))) float sv[2][kF32BlockN * kRow];
-  __shared__ int sok[2][kF32BlockN];  // key of the tile lies in a valid block
+  constexpr int kAhead = D == 128;  // operands read from LDS a step ahead
+  constexpr int kStages = D == 128 ? 2 : 1;  // of LDS
+  __shared__ __attribute__((aligned(16))) float sk[kStages][kF32BlockN * kRow];
+  __shared__ __attribute__((aligned(16))) float sv[kStages][kF32BlockN * kRow];
+  __shared__ int sok[kStages][kF32BlockN];  // key of the tile lies in a valid block
 
   int seq, hk, m0;
   f32_map(p, blockIdx.x, blockIdx.y, blockIdx.z, seq, hk, m0);
@@ -157,6 +166,12 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
   double m_run = -INFINITY;  // the query's running max, log2 units
   float l_run = 0.f;         // this lane's share of the query's sum
 
+  // Row r's 16-byte chunk c lies at c ^ swz(r): the same chunk of 16 rows, and 16 adjacent chunks
+  // of one row, then fall on all 64 banks, and the chunk stays inside its row of D / 4 chunks
+  // (16 or 32, 24 in groups of 8, 20 in groups of 4).
+  auto swz = [](int r) __attribute__((always_inline)) -> int {
+    return D % 64 == 0 ? r & 15 : (D % 32 == 0 ? (r >> 1) & 7 : (r >> 2) & 3);
+  };
   const int32_t* bt = PAGED ? p.block_tables + (int64_t)seq * p.bt_stride : nullptr;
   const float* bias_row = p.bias ? p.bias + (int64_t)seq * p.bias_seq + (int64_t)h * p.bias_head +
                                        (int64_t)tok * p.bias_q
@@ -222,7 +237,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
       const int idx = tid + i * kF32Threads;
       const int key = idx / kC4;
       const int c4 = idx - key * kC4;
-      const int at = key * kRow + 4 * (c4 ^ (key & 15));
+      const int at = key * kRow + 4 * (c4 ^ swz(key));
       if (kChunks % kF32Threads != 0 && idx >= kChunks) break;
       *reinterpret_cast<float4*>(sk[stage] + at) = widen(kr[i], ksr[i]);
       *reinterpret_cast<float4*>(sv[stage] + at) = widen(vr[i], vsr[i]);
@@ -238,17 +253,17 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
     // the operands of step c + 1 are read while the products of step c run, and the two
     // tiles' chains alternate
     auto k_read = [&](int c, float4 (&a)[2]) __attribute__((always_inline)) {
-      const int at = 4 * ((4 * c + slot) ^ col);
+      const int at = 4 * ((4 * c + slot) ^ swz(col));
       a[0] = *reinterpret_cast<const float4*>(ks + at);
       a[1] = *reinterpret_cast<const float4*>(ks + 16 * kRow + at);
     };
-    float4 ka[2][2];
-    k_read(0, ka[0]);
+    float4 ka[kAhead + 1][2];
+    if constexpr (kAhead) k_read(0, ka[0]);
 #pragma unroll
     for (int c = 0; c < D / 16; ++c) {
-      if (c + 1 < D / 16) k_read(c + 1, ka[(c + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);
-      const float4(&a)[2] = ka[c & 1];
+      if (!kAhead || c + 1 < D / 16) k_read(c + kAhead, ka[(c + kAhead) & kAhead]);
+      if constexpr (kAhead) __builtin_amdgcn_sched_barrier(0);
+      const float4(&a)[2] = ka[c & kAhead];
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
         s[kt] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[kt].x, qd[4 * c + 0], s[kt], 0, 0, 0);
@@ -301,7 +316,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
     };
     auto v_read = [&](int u, VRow& a) __attribute__((always_inline)) {  // keys 4 u + slot
       const float* vrow = sv[stage] + (4 * u + slot) * kRow;
-      const int sw = (4 * u + slot) & 15;
+      const int sw = swz(4 * u + slot);
 #pragma unroll
       for (int g = 0; g < kQuads; ++g)
         a.q[g] = *reinterpret_cast<const float4*>(vrow + 4 * ((16 * g + col) ^ sw));
@@ -311,13 +326,13 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
         a.t[t - 4 * kQuads] = vrow[4 * ((d >> 2) ^ sw) + (d & 3)];
       }
     };
-    VRow va[2];
-    v_read(0, va[0]);
+    VRow va[kAhead + 1];
+    if constexpr (kAhead) v_read(0, va[0]);
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      if (u < 7) v_read(u + 1, va[(u + 1) & 1]);
-      __builtin_amdgcn_sched_barrier(0);
-      const VRow& a = va[u & 1];
+      if (!kAhead || u < 7) v_read(u + kAhead, va[(u + kAhead) & kAhead]);
+      if constexpr (kAhead) __builtin_amdgcn_sched_barrier(0);
+      const VRow& a = va[u & kAhead];
       const float pu = pr[u >> 2][u & 3];
 #pragma unroll
       for (int g = 0; g < kQuads; ++g) {
@@ -332,7 +347,15 @@ __global__ __launch_bounds__(kF32Threads, 2) void prefill_f32_kernel(PrefillF32P
     }
   };
 
-  if (n_begin < n_stop) {
+  if constexpr (kStages == 1) {
+    for (int n0 = n_begin; n0 < n_stop; n0 += kF32BlockN) {
+      __syncthreads();
+      load_tile(n0);
+      store_tile(0);
+      __syncthreads();
+      if (wave_any(n0 < kb)) compute(n0, 0);
+    }
+  } else if (n_begin < n_stop) {
     load_tile(n_begin);
     store_tile(0);
     __syncthreads();
