@@ -477,10 +477,10 @@ void launch_f32_split(const PrefillF32Params& p, dim3 grid, hipStream_t s) {
 
 size_t prefill_f32_split_bytes(int32_t num_seqs, int64_t max_q_len, int64_t max_k_len,
                                int32_t num_heads, int32_t num_kv_heads, int head_dim) {
-  int32_t a, b;
+  int32_t blocks;
   int64_t rows = max_q_len * (num_heads / num_kv_heads);
   if (rows > INT32_MAX) rows = INT32_MAX;
-  const int64_t nwg = f32_grid((int64_t)num_seqs * num_kv_heads, rows, a, b);
+  const int64_t nwg = f32_grid((int64_t)num_seqs * num_kv_heads, rows, blocks);
   return f32_split_bytes(nwg, f32_split_count(nwg, max_k_len), head_dim);
 }
 
@@ -497,7 +497,7 @@ int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int nu
   if (rows > INT32_MAX) rows = INT32_MAX;
   block_divisor(p.group, p.group_magic, p.group_shift);
   const int64_t groups = (int64_t)num_seqs * p.num_kv_heads;
-  const int64_t nwg = f32_grid(groups, rows, p.num_m_blocks, p.level_run);
+  const int64_t nwg = f32_grid(groups, rows, p.num_m_blocks);
   p.groups = (int32_t)at_most(groups, kMaxGroups);  // 1-D: no more than its workgroups
   p.splits = 1;
   if (ws && elem == kElemF32 && !p.decode) {
@@ -510,6 +510,7 @@ int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int nu
       p.part_l = p.part_o + parts * head_dim;
     }
   }
+  p.level_run = f32_run(nwg, p.num_m_blocks, p.causal == NIA_CAUSAL_TOP_LEFT, p.splits > 1);
   const dim3 grid = p.level_run ? dim3((unsigned)nwg)
                                 : dim3((unsigned)p.num_m_blocks, (unsigned)p.num_kv_heads,
                                        (unsigned)num_seqs);

@@ -203,13 +203,12 @@ NIA_BOTH int f32_ranges(int tiles, int splits) {
 }
 
 // The workgroup's (sequence, KV head, row block).  `id`: its number in the 1-D grid, or x in a
-// 3-D one (level_run 0) of row blocks, KV heads and sequences.  Runs of adjacent levels of one
-// (sequence, KV head) group follow each other, for the shader engines as in prefill_map; the
-// groups lie over all XCDs, since the matrix cores bound the tiles and not their loads: with
-// every group on one XCD, four groups left half the chip idle (690 rows of 28 and 4 heads, D 96,
-// 131 us instead of 73) and one XCD had the longest sequence to itself (seven of up to 775 rows of
-// 8 heads and one 298 instead of 187); four prompts of 128-1024 tokens (16 and 8 heads) 186 and
-// 182.
+// 3-D one (level_run 0) of row blocks, KV heads and sequences.  Runs of level_run adjacent
+// levels of one (sequence, KV head) group follow each other (f32_run); the groups lie over all
+// XCDs, since the matrix cores bound the tiles and not their loads: with every group on one
+// XCD, four groups left half the chip idle (690 rows of 28 and 4 heads, D 96, 131 us instead of
+// 73) and one XCD had the longest sequence to itself (seven of up to 775 rows of 8 heads and one
+// 298 instead of 187); four prompts of 128-1024 tokens (16 and 8 heads) 186 and 182.
 template <typename P>
 NIA_BOTH void f32_map(const P& p, uint32_t id, uint32_t y, uint32_t z3, int& seq, int& hk,
                       int& m0) {
@@ -231,14 +230,23 @@ NIA_BOTH void f32_map(const P& p, uint32_t id, uint32_t y, uint32_t z3, int& seq
   m0 = (p.num_m_blocks - 1 - z) * kF32BlockM;
 }
 
-// The row blocks of a call of at most `rows` packed rows a group, and their grid: 1-D, or 3-D
-// (run 0) where one dimension does not hold it (a loose row bound over very many sequences).
-// A sequence of more rows than a dimension holds blocks for would be a q of 2^30 rows.
-inline int64_t f32_grid(int64_t groups, int64_t rows, int32_t& m_blocks, int32_t& run) {
+// The row blocks of a call of at most `rows` packed rows a group, and all workgroups.  A sequence
+// of more rows than a grid dimension holds blocks for would be a q of 2^30 rows.
+inline int64_t f32_grid(int64_t groups, int64_t rows, int32_t& m_blocks) {
   m_blocks = (int32_t)at_most((rows + kF32BlockM - 1) / kF32BlockM, kMaxGroups);
-  const int64_t nwg = groups * m_blocks;
-  run = nwg > kMaxGroups ? 0 : (m_blocks >= 4 ? 4 : 1);
-  return nwg;
+  return groups * m_blocks;
+}
+
+// Adjacent levels of a group that follow each other in a grid of nwg workgroups; 0: the 3-D
+// grid.  Top-left causal blocks are as long as their level: four levels of every group in turn,
+// for the shader engines as in prefill_map.  Otherwise a group's blocks are about equally long
+// and go out together, group by group, which the 3-D grid does without a division (ranges take
+// its second dimension): with four levels in turn the last blocks of the longest image ended
+// four images of 784-3072 rows (16 heads of 80) at 1528 us instead of 1293.  The 3-D grid is also
+// for what one dimension does not hold (a loose row bound over very many sequences).
+inline int32_t f32_run(int64_t nwg, int32_t m_blocks, bool top_left, bool cut) {
+  if (!cut && (!top_left || nwg > kMaxGroups)) return 0;
+  return top_left ? (m_blocks >= 4 ? 4 : 1) : m_blocks;
 }
 
 inline int32_t f32_split_count(int64_t nwg, int64_t max_k_len) {

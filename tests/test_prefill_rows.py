@@ -51,10 +51,13 @@ def test_longest_levels_go_out_first(seqs, hkv, group):
 @pytest.mark.parametrize("blocks", [1, 3, 4, 5, 9])
 def test_other_maps_cover_the_work_once(seqs, hkv, blocks):
     g = wm.Grid(num_seqs=seqs, num_kv_heads=hkv)
-    n = wm.lib().t_f32_grid(ctypes.byref(g), 64 * blocks - 3)
-    assert n == seqs * hkv * blocks  # every XCD takes its share, however few the groups
-    assert_covers([(s, h, m // 64) for s, h, m in wm.mapped(g, "f32", n)],
-                  range(seqs), range(hkv), range(blocks))
+    for top_left, cut in itertools.product((0, 1), repeat=2):
+        n = wm.lib().t_f32_grid(ctypes.byref(g), 64 * blocks - 3, top_left, cut)
+        assert n == seqs * hkv * blocks  # every XCD takes its share, however few the groups
+        got = [(s, h, m // 64) for s, h, m in wm.mapped(g, "f32", n)]
+        assert_covers(got, range(seqs), range(hkv), range(blocks))
+        if not top_left:  # a group's blocks together: they are equally long
+            assert [x[:2] for x in got] == sorted(x[:2] for x in got)
     assert_covers(wm.mapped(g, "pair", 8 * cdiv(seqs, 8) * hkv), range(seqs), range(hkv), range(1))
 
 
@@ -63,7 +66,7 @@ def test_fp32_grid_takes_three_dimensions_past_one():
     for seqs, rows, run in ((1023, 131072, 4), (1024, 131072, 0), (65535, 1 << 20, 0),
                             (1, (1 << 31) - 1, 0), (8, (1 << 24) - 64 * 9, 4)):
         g = wm.Grid(num_seqs=seqs, num_kv_heads=8)
-        n = wm.lib().t_f32_grid(ctypes.byref(g), rows)
+        n = wm.lib().t_f32_grid(ctypes.byref(g), rows, 1, 0)
         assert g.level_run == run and g.num_m_blocks == min(cdiv(rows, 64), (1 << 24) - 1)
         assert (n < 1 << 24) == (run > 0)
 

@@ -26,18 +26,25 @@ int64_t t_grid(Grid* p, int max_q_len, int packed) {
   p->groups_per_xcd = (p->num_seqs * p->num_kv_heads + kXcds - 1) / kXcds;
   return grid_size(*p);
 }
-int64_t t_f32_grid(Grid* p, int64_t rows) {
+int64_t t_f32_grid(Grid* p, int64_t rows, int top_left, int cut) {
   p->groups = p->num_seqs * p->num_kv_heads;
-  return f32_grid(p->groups, rows, p->num_m_blocks, p->level_run);
+  const int64_t n = f32_grid(p->groups, rows, p->num_m_blocks);
+  p->level_run = f32_run(n, p->num_m_blocks, top_left, cut);
+  return n;
 }
-// kind 0: prefill_map, 1: ranked, 2: pair, 3: fp32; out[id] = seq, head, block or -1s
+// kind 0: prefill_map, 1: ranked, 2: pair, 3: fp32 (3-D: x, then y, then z); out[id] = seq, head,
+// block or -1s
 void t_map(const Grid* p, int kind, int n, const int* order, int* out) {
   for (int id = 0; id < n; ++id, out += 3) {
     int s = 0, h = 0, m = 0;
     const bool ok = kind == 0   ? prefill_map(*p, id, s, h, m)
                     : kind == 1 ? prefill_map_ranked(*p, id, order, s, h, m)
                     : kind == 2 ? pair_map(*p, id, s, h, m)
-                                : (f32_map(*p, id, 0, 0, s, h, m), true);
+                    : p->level_run
+                        ? (f32_map(*p, id, 0, 0, s, h, m), true)
+                        : (f32_map(*p, id % p->num_m_blocks, id / p->num_m_blocks % p->num_kv_heads,
+                                   id / p->num_m_blocks / p->num_kv_heads, s, h, m),
+                           true);
     out[0] = ok ? s : -1;
     out[1] = ok ? h : -1;
     out[2] = ok ? m : -1;
@@ -93,7 +100,7 @@ def lib():
     for name in ("t_grid", "t_f32_grid", "t_blocks", "t_span", "t_range_tile", "t_few_per"):
         getattr(so, name).restype = ctypes.c_int64
     i64 = ctypes.c_int64
-    so.t_f32_grid.argtypes = [ctypes.c_void_p, i64]
+    so.t_f32_grid.argtypes = [ctypes.c_void_p, i64, ctypes.c_int, ctypes.c_int]
     so.t_span.argtypes = [i64, i64, ctypes.c_int, ctypes.c_int]
     so.t_split_count.argtypes = [i64, i64, ctypes.c_int]
     so.t_f32_split_count.argtypes = [i64, i64]
