@@ -97,13 +97,16 @@ struct DecodeParams {
 };
 
 // ---- fp32 caches: head_dim 128, block size 16, at most 8 query heads per KV head ----------
-// Grid (512-key partition, KV head, sequence); wave w of 8 takes blocks w, w + 8, ... of the
-// partition.  Bound by HBM once the scores are off the vector unit: q . k summed there in fp64
+// Grid (512-key partition, KV head, sequence); wave w of WAVES takes blocks w, w + WAVES, ... of
+// the partition.  Bound by HBM once the scores are off the vector unit: q . k summed there in fp64
 // over 32 lanes (five exchanges a score) took 47 us with the merge for 16 sequences of 339-2304
 // keys (16 and 8 heads, 164 MB), 77 with 32 and 8 heads, 107 for 8 sequences of 28 and 4
 // heads; now 43, 47 and 22 (32 sequences of 4096 keys stream at 5.7 TB/s; the rest is the
 // start, about 8 us, and the merge's launch, 5).  Eight waves, one workgroup a CU: four waves
-// and three workgroups 51 us, two workgroups in 128 registers 45.
+// and three workgroups 51 us, two workgroups in 128 registers 45.  Where one partition of every
+// (sequence, KV head) is more than a workgroup a CU, four waves and three workgroups instead:
+// 100 sequences of 60 keys (16 heads) 29.5 us with eight, 20.2 with four, 80 of 3000 (28 and 4
+// heads) 194 and 183, 64 of 4000 (16 and 8) 344 and 347.
 //   Scores: v_mfma_f64_4x4x4 (16.6 cycles; fp32 inputs widened exactly), four 4 x 4 products
 //   a time: A lane l holds key l % 16 (block (l / 4) % 4 is the keys 4 b .. + 3), dim slot
 //   l / 16; B lane l query head l % 4 of a group of four, the same dim, from LDS in fp64; the
@@ -115,8 +118,7 @@ struct DecodeParams {
 //   they are never read.  Row i of output tile t is dim 64 (t / 4) + 4 i + t % 4, so that one
 //   16-byte load of a V row feeds four tiles.
 //   Each operand of the next block is loaded as soon as this block's has been consumed.
-constexpr int kF32Waves = 8;
-constexpr int kF32Threads = kF32Waves * kWave;
+constexpr int kF32Groups = 256;  // (sequence, KV head) pairs up to which a workgroup has 8 waves
 
 // x of the lane N up the row of 16 (wrapping).
 template <int N>
@@ -127,9 +129,10 @@ NIA_DEVICE float row_up(float x) {
 }
 
 // CG: groups of four query heads (1 or 2).
-template <int CG, int PART_BLOCKS>
-__global__ __launch_bounds__(kF32Threads, 2) void paged_decode_f32_kernel(DecodeParams p) {
-  constexpr int D = 128, BS = 16, kTiles = D / 16;
+template <int CG, int PART_BLOCKS, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave, WAVES == 4 ? 3 : 2) void paged_decode_f32_kernel(
+    DecodeParams p) {
+  constexpr int D = 128, BS = 16, kTiles = D / 16, kThreads = WAVES * kWave;
   constexpr int PART_TOKENS = PART_BLOCKS * BS;
   const int part = blockIdx.x;
   const int hk = blockIdx.y;
@@ -148,7 +151,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void paged_decode_f32_kernel(Decode
     // Whole workgroup leaves together.  A sequence without keys gets zeros from
     // its first partition.
     if (part == 0 && ctx == 0)
-      for (int idx = threadIdx.x; idx < G * D; idx += kF32Threads)
+      for (int idx = threadIdx.x; idx < G * D; idx += kThreads)
         ob[(int64_t)(idx / D) * p.out_h + idx % D] = 0.f;
     return;
   }
@@ -188,7 +191,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void paged_decode_f32_kernel(Decode
 
   // the query heads in fp64, [group][c][e pair][slot][head] pairs of dims 16 c + 4 slot + e
   __shared__ __attribute__((aligned(16))) double s_q[CG * 4 * D];
-  for (int idx = threadIdx.x; idx < CG * 4 * D; idx += kF32Threads) {
+  for (int idx = threadIdx.x; idx < CG * 4 * D; idx += kThreads) {
     const int e = idx & 1, j = (idx >> 1) & 3, k = (idx >> 3) & 3, ep = (idx >> 5) & 1,
               c = (idx >> 6) & 7, g = idx >> 9;
     const int h = 4 * g + j;
@@ -212,7 +215,7 @@ __global__ __launch_bounds__(kF32Threads, 2) void paged_decode_f32_kernel(Decode
   const int my_key = 4 * ((lane >> 2) & 3) + slot;  // of the scores
 
   while (jb < blk_end) {
-    const int64_t nbase = block_base(jb + kF32Waves);
+    const int64_t nbase = block_base(jb + WAVES);
     const bool ok = base >= 0;  // uniform: an invalid block id contributes nothing
     float x[CG];
     if (ok) {
@@ -295,13 +298,13 @@ __global__ __launch_bounds__(kF32Threads, 2) void paged_decode_f32_kernel(Decode
     }
     load_v(nbase);
     base = nbase;
-    jb += kF32Waves;
+    jb += WAVES;
   }
 
   // ---- merge the waves' states: the final output (single-partition sequence) or the
   // partition's partial (m, l, un-normalised o) for the combine kernel ------------------------
-  __shared__ float sm_o[kF32Waves][CG * 4][D];
-  __shared__ float sm_m[kF32Waves][CG * 4], sm_l[kF32Waves][CG * 4];
+  __shared__ float sm_o[WAVES][CG * 4][D];
+  __shared__ float sm_m[WAVES][CG * 4], sm_l[WAVES][CG * 4];
 #pragma unroll
   for (int g = 0; g < CG; ++g) {
 #pragma unroll
@@ -320,15 +323,15 @@ __global__ __launch_bounds__(kF32Threads, 2) void paged_decode_f32_kernel(Decode
             make_float4(oacc[4 * g][i], oacc[4 * g + 1][i], oacc[4 * g + 2][i], oacc[4 * g + 3][i]);
   }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < G * D; idx += kF32Threads) {
+  for (int idx = threadIdx.x; idx < G * D; idx += kThreads) {
     const int g = idx / D;
     const int d = idx - g * D;
     float mt = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < kF32Waves; ++w) mt = fmaxf(mt, sm_m[w][g]);
+    for (int w = 0; w < WAVES; ++w) mt = fmaxf(mt, sm_m[w][g]);
     float lt = 0.f, ot = 0.f;
 #pragma unroll
-    for (int w = 0; w < kF32Waves; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const float mw = sm_m[w][g];
       const float wt = (mw == -INFINITY) ? 0.f : fast_exp2(mw - mt);
       lt = fmaf(sm_l[w][g], wt, lt);
@@ -1311,10 +1314,15 @@ int launch_split(DecodeParams& p, int batch, hipStream_t s) {
 int launch_f32_partitions(const DecodeParams& p, int G, int batch, hipStream_t s) {
   const dim3 grid(p.max_parts, p.num_kv_heads, batch);
   if (G > 8) return NIA_ERR_UNSUPPORTED;
+  const bool wide = (int64_t)batch * p.num_kv_heads <= kF32Groups;
+  const dim3 block((wide ? 8 : 4) * kWave);
+  auto launch = [&](auto kernel) { nia_launch(kernel, grid, block, s, p); };
   if (G <= 4)
-    nia_launch((paged_decode_f32_kernel<1, kPartBlocks>), grid, dim3(kF32Threads), s, p);
+    launch(wide ? paged_decode_f32_kernel<1, kPartBlocks, 8>
+                : paged_decode_f32_kernel<1, kPartBlocks, 4>);
   else
-    nia_launch((paged_decode_f32_kernel<2, kPartBlocks>), grid, dim3(kF32Threads), s, p);
+    launch(wide ? paged_decode_f32_kernel<2, kPartBlocks, 8>
+                : paged_decode_f32_kernel<2, kPartBlocks, 4>);
   if (p.max_parts > 1) {
     constexpr int kPairsPerGroup = kCombineThreads / kWave;
     const int pairs = batch * p.num_heads;

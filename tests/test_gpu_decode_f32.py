@@ -24,6 +24,19 @@ def test_groups_and_edges(g):
     assert_attn_close(out.double().cpu().numpy(), oracle(c), torch.float32)
 
 
+@pytest.mark.parametrize("g", [1, 4, 5, 8])
+@pytest.mark.parametrize("batch", [128, 129])
+def test_many_sequences(batch, g):
+    """Past 256 (sequence, KV head) pairs a workgroup has four waves instead of eight."""
+    edges = [1, 16, 17, 63, 64, 65, 80, 129, 511, 512, 513, 1025]
+    lens = [edges[i % len(edges)] for i in range(batch)]
+    print(f"f32 decode G={g} batch={batch}", flush=True)
+    c = workloads.make_decode(batch, 2 * g, 2, 128, lens, sum(-(-n // 16) for n in lens) + 5, 16,
+                              torch.float32, "cuda", 60 + g)
+    out = ops.paged_decode(c.q, c.k_cache[0], c.v_cache[0], c.block_tables, c.context_lens)
+    assert_attn_close(out.double().cpu().numpy(), oracle(c), torch.float32)
+
+
 def test_block_outside_the_pool_is_skipped():
     c = workloads.make_decode(2, 8, 2, 128, [48, 700], 60, 16, torch.float32, "cuda", 39)
     whole = ops.paged_decode(c.q, c.k_cache[0], c.v_cache[0], c.block_tables, c.context_lens)
