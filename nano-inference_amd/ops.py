@@ -761,9 +761,10 @@ def prefill_paged(
     max_q_len, causal, mb = int(max_q_len), int(causal), bt_shape[1]
     scale = _default_scale(d, scale)
     ws = None
+    # bf16 ranges want blocks of a power of two from 16 on
     if rows * h <= _SPLIT_MAX_ROWS_F32 if dt != _lib.DTYPE_BF16 else (
             mb * bs >= _SPLIT_MIN_KEYS and causal != CAUSAL_TOP_LEFT and
-            n * h * max_q_len <= _SPLIT_MAX_ROWS):
+            n * h * max_q_len <= _SPLIT_MAX_ROWS and bs >= 16 and bs & (bs - 1) == 0):
         ws = _split_workspace(n, max_q_len, mb * bs, h, hkv, d, causal, dt, q.device)
     if ws is not None:
         st = _lib.load().nia_prefill_paged_split(

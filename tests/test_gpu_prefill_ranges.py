@@ -195,3 +195,14 @@ def test_ranges_are_chosen_for_one_sequence_not_for_the_sum(monkeypatch, dtype, 
     lens = [torch.tensor(x, dtype=torch.int32).cuda() for x in (ql, kl)]
     ops.prefill(q, k, v, starts[0], lens[0], starts[1], lens[1], max(ql), ops.CAUSAL_NONE)
     assert any(x is not None for x in seen) == cut
+
+
+@pytest.mark.parametrize("bs,cut", [(16, True), (64, True), (24, False), (12, False), (5, False)])
+def test_block_sizes_that_are_never_cut_ask_for_no_workspace(monkeypatch, bs, cut):
+    seen, ask = [], ops._split_workspace
+    monkeypatch.setattr(ops, "_split_workspace", lambda *a: seen.append(ask(*a)) or seen[-1])
+    c = workloads.chunked_qwen3_8b("cuda", seed=95, n=1, chunk=24, prior=[3000], num_heads=8,
+                                   num_kv_heads=2, block_size=bs)
+    ops.prefill_paged(c.q, c.k_cache, c.v_cache, c.block_tables, c.q_start, c.q_len,
+                      c.context_lens, c.chunk)
+    assert any(x is not None for x in seen) == cut
