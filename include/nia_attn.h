@@ -240,7 +240,11 @@ int32_t nia_prefill_paged(void* out, int64_t out_tok_stride, int64_t out_head_st
  * bytes that a call can use, 0 where it would not cut (enough rows, short keys).  A
  * null, unaligned or smaller workspace runs the call uncut.  Nothing in it needs
  * initialising; calls one after another on a stream may share it.
+ * fp32 calls of more than NIA_PREFILL_F32_SPLIT_MAX_ROWS query rows (all sequences' rows x
+ * num_heads) are faster uncut.  The library knows only max_q_len: it sees that bound for a
+ * single sequence; for several the caller, who knows the rows, passes no workspace past it.
  */
+#define NIA_PREFILL_F32_SPLIT_MAX_ROWS 40960
 size_t nia_prefill_split_workspace_size(int32_t num_seqs, int32_t max_q_len, int64_t max_k_len,
                                         int32_t num_heads, int32_t num_kv_heads,
                                         int32_t head_dim, int32_t causal, int32_t dtype);

@@ -35,6 +35,7 @@ ERR_LAUNCH = 4
 ERR_MISALIGNED = 5
 ERR_SCRATCH_LIMIT = 6
 DECODE_SCRATCH_BYTES = 40 << 20  # NIA_DECODE_SCRATCH_BYTES
+PREFILL_F32_SPLIT_MAX_ROWS = 40960  # NIA_PREFILL_F32_SPLIT_MAX_ROWS
 
 _p = C.c_void_p
 _i32 = C.c_int32

@@ -61,6 +61,7 @@ namespace {
 constexpr int kF32Waves = 4;
 constexpr int kF32Threads = kF32Waves * kWave;
 static_assert(kF32BlockM == 16 * kF32Waves, "16 rows a wave");
+static_assert(kF32SplitMaxRows == NIA_PREFILL_F32_SPLIT_MAX_ROWS, "the header's bound");
 
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
@@ -481,7 +482,8 @@ size_t prefill_f32_split_bytes(int32_t num_seqs, int64_t max_q_len, int64_t max_
   int64_t rows = max_q_len * (num_heads / num_kv_heads);
   if (rows > INT32_MAX) rows = INT32_MAX;
   const int64_t nwg = f32_grid((int64_t)num_seqs * num_kv_heads, rows, blocks);
-  return f32_split_bytes(nwg, f32_split_count(nwg, max_k_len), head_dim);
+  const int64_t sure = num_seqs == 1 ? max_q_len * num_heads : 0;
+  return f32_split_bytes(nwg, f32_split_count(nwg, max_k_len, sure), head_dim);
 }
 
 int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int num_seqs,
@@ -501,7 +503,8 @@ int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int nu
   p.groups = (int32_t)at_most(groups, kMaxGroups);  // 1-D: no more than its workgroups
   p.splits = 1;
   if (ws && elem == kElemF32 && !p.decode) {
-    const int32_t n = f32_split_count(nwg, max_k_len);
+    const int64_t sure = num_seqs == 1 ? (int64_t)max_q_len * p.num_heads : 0;
+    const int32_t n = f32_split_count(nwg, max_k_len, sure);
     if (n > 1 && f32_split_bytes(nwg, n, head_dim) <= ws_bytes) {
       const size_t parts = (size_t)nwg * n * kF32BlockM;
       p.splits = n;

@@ -192,10 +192,12 @@ constexpr int kF32BlockN = 32;  // keys per LDS tile
 // Key ranges of about kF32RangeTiles tiles, so that no workgroup is left behind on a long row
 // block (a tile takes 4.3 us and every workgroup's SIMDs are busy): four prompts of 128-1024
 // tokens 217 us uncut, 183-186 in ranges of 5, 8 or 12 tiles; one of 500 77 us, 51 / 47 / 64.
-// The caller leaves out calls whose blocks fill the chip (ops.py); the partials stay below
-// kF32MaxParts x 33 KB (135 MB).
+// More than kF32SplitMaxRows rows (640 blocks) fill the chip evenly enough uncut: four prompts of
+// 1000 tokens of 16 heads 281 us uncut, 314 in ranges; one 151 and 111.  The partials stay
+// below kF32MaxParts x 33 KB (135 MB).
 constexpr int kF32RangeTiles = 8;
 constexpr int kF32SplitTiles = 12;   // fewer at most: uncut (the merge is a second launch)
+constexpr int64_t kF32SplitMaxRows = 640 * kF32BlockM;  // NIA_PREFILL_F32_SPLIT_MAX_ROWS
 constexpr int64_t kF32MaxParts = 4096;
 
 NIA_BOTH int f32_ranges(int tiles, int splits) {
@@ -249,7 +251,9 @@ inline int32_t f32_run(int64_t nwg, int32_t m_blocks, bool top_left, bool cut) {
   return top_left ? (m_blocks >= 4 ? 4 : 1) : m_blocks;
 }
 
-inline int32_t f32_split_count(int64_t nwg, int64_t max_k_len) {
+// `sure_rows`: query rows of the call as far as the launcher knows them (a single sequence's).
+inline int32_t f32_split_count(int64_t nwg, int64_t max_k_len, int64_t sure_rows) {
+  if (sure_rows > kF32SplitMaxRows) return 1;
   const int64_t tiles = (max_k_len + kF32BlockN - 1) / kF32BlockN;
   if (tiles < kF32SplitTiles) return 1;
   int64_t n = (tiles + kF32RangeTiles - 1) / kF32RangeTiles;

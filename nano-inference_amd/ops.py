@@ -470,9 +470,9 @@ def _i32(name: str, t: torch.Tensor, n: int) -> torch.Tensor:
 # bf16 calls with fewer keys a sequence, or more query rows, are not worth cutting
 # (nia_prefill_split_workspace_size says which of the others are): they skip the question.
 _SPLIT_MIN_KEYS, _SPLIT_MAX_ROWS = 768, 256 * 128
-# fp32 calls of more rows (640 blocks of 64) fill the chip evenly enough uncut: four prompts
-# of 1000 tokens of 16 heads 279 us uncut, 315 in ranges of 256 keys; one 146 and 114.
-_SPLIT_MAX_ROWS_F32 = 640 * 64
+# fp32 calls of more rows fill the chip evenly enough uncut (the bound the library states: it
+# knows only the longest sequence's).
+_SPLIT_MAX_ROWS_F32 = _lib.PREFILL_F32_SPLIT_MAX_ROWS
 
 
 def _split_workspace(n, max_q_len, keys, h, hkv, d, causal, dt, dev) -> Optional[torch.Tensor]:

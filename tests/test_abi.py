@@ -186,6 +186,27 @@ def test_workspace_size():
     assert lib.nia_paged_decode_workspace_size(64, 32, 3, 512, 16, 128, 0) == 0  # 32 % 3
 
 
+def test_prefill_split_workspace_size():
+    """0 for what is not cut; fp32 calls past the row bound of the header are among them as far
+    as the library knows their rows."""
+    lib = _lib.load()
+    text = open(os.path.join(ROOT, "include", "nia_attn.h")).read()
+    bound = int(re.search(r"#define NIA_PREFILL_F32_SPLIT_MAX_ROWS (\d+)", text).group(1))
+    assert bound == _lib.PREFILL_F32_SPLIT_MAX_ROWS
+
+    def size(n, q, keys, h, hkv, causal, dt, d=128):
+        return lib.nia_prefill_split_workspace_size(n, q, keys, h, hkv, d, causal, dt)
+
+    rows = bound // 16
+    assert size(1, rows, rows, 16, 8, 1, 1) > 0 and size(1, rows + 1, rows + 1, 16, 8, 1, 1) == 0
+    assert size(4, 1000, 1000, 16, 8, 1, 1) > 0  # a bound of the rows only: the caller knows them
+    assert size(1, 100, 32 * 11, 16, 8, 0, 1) == 0  # fewer than 12 key tiles
+    for causal, cut in ((0, True), (1, False), (2, True)):  # bf16: top-left calls stay uncut
+        assert (size(1, 64, 8000, 32, 8, causal, 0) > 0) == cut
+    assert size(64, 128, 8000, 32, 8, 2, 0) == 0  # a full grid
+    assert size(0, 64, 8000, 32, 8, 2, 0) == size(1, 64, 8000, 32, 7, 2, 0) == 0
+
+
 def test_qk_norm_rope_validation_without_launching():
     lib = _lib.load()
     p = ctypes.c_void_p(16)  # never dereferenced: validation fails or returns first

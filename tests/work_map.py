@@ -70,7 +70,9 @@ int64_t t_range_tile(int tiles, int s, int n) { return range_tile(tiles, s, n); 
 int t_split_count(int64_t nwg, int64_t tiles, int top_left) {
   return split_count(nwg, tiles, top_left);
 }
-int t_f32_split_count(int64_t nwg, int64_t keys) { return f32_split_count(nwg, keys); }
+int t_f32_split_count(int64_t nwg, int64_t keys, int64_t rows) {
+  return f32_split_count(nwg, keys, rows);
+}
 int t_few(int64_t total, int64_t alone) { return few_units(total, alone); }
 int t_merge_waves(int64_t pairs, int64_t ranges, int64_t sequences) {
   return merge_waves(pairs, ranges, sequences);
@@ -103,7 +105,7 @@ def lib():
     so.t_f32_grid.argtypes = [ctypes.c_void_p, i64, ctypes.c_int, ctypes.c_int]
     so.t_span.argtypes = [i64, i64, ctypes.c_int, ctypes.c_int]
     so.t_split_count.argtypes = [i64, i64, ctypes.c_int]
-    so.t_f32_split_count.argtypes = [i64, i64]
+    so.t_f32_split_count.argtypes = [i64, i64, i64]
     so.t_merge_waves.argtypes = [i64, i64, i64]
     so.t_few.argtypes = [i64, i64]
     so.t_few_per.argtypes = [i64, i64, i64, i64]
