@@ -136,7 +136,7 @@ NIA_DEVICE void rank_sequences(const PrefillParams& p, int* s_key, int* s_order)
 }
 
 // The workgroup's (sequence, head, m-block) under either map.
-template <bool PAGED>
+template <bool PAGED, bool RUNS>
 NIA_DEVICE bool map_workgroup(const PrefillParams& p, int& seq, int& h, int& mb) {
   if (p.order_by_len) {
     __shared__ int s_key[kOrderMaxSeqs];
@@ -144,7 +144,7 @@ NIA_DEVICE bool map_workgroup(const PrefillParams& p, int& seq, int& h, int& mb)
     rank_sequences<PAGED>(p, s_key, s_order);
     return prefill_map_ranked(p, blockIdx.x, s_order, seq, h, mb);
   }
-  return prefill_map(p, blockIdx.x, seq, h, mb);
+  return prefill_map<RUNS>(p, blockIdx.x, seq, h, mb);
 }
 
 // XOR swizzle of the 4-key groups inside a transposed-V row (row = head dim d).
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kPrefillThreads, 2) void prefill_kernel(PrefillPara
   __shared__ __attribute__((aligned(16))) uint8_t vt_lds[DP * VT_PITCH];
 
   int seq, h, mb;
-  if (!map_workgroup<PAGED>(p, seq, h, mb)) return;
+  if (!map_workgroup<PAGED, false>(p, seq, h, mb)) return;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid / kWave;
@@ -519,7 +519,7 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
   if constexpr (PAIR) {
     if (!pair_map(p, blockIdx.x, seq, h, mb)) return;
   } else {
-    if (!map_workgroup<PAGED>(p, seq, h, mb)) return;
+    if (!map_workgroup<PAGED, PACK>(p, seq, h, mb)) return;
   }
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -775,9 +775,8 @@ __global__ __launch_bounds__(kPrefillThreads, COMPACT ? 3 : 2) void prefill_dma_
   const float sl = BIAS ? kLog2e : p.scale_log2;
   const float* bias_row = nullptr;  // BIAS: this lane's query row of the mask
   if constexpr (BIAS)
-    bias_row = p.bias + (int64_t)seq * p.bias_seq +
-               (int64_t)(h + (row_ok ? qhead : 0)) * p.bias_head +
-               (int64_t)(row_ok ? qtok : 0) * p.bias_q;
+    bias_row = p.bias + (int64_t)seq * p.bias_seq + (int64_t)h * p.bias_head +
+               (int64_t)(row_ok ? qrow : 0) * p.bias_q;
   auto compute_tile = [&](int n0, int stage) __attribute__((always_inline)) {
     const uint8_t* kt = tile_k(stage);
     const uint8_t* vt = tile_v(stage);
@@ -1088,7 +1087,7 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_merge_kernel(PrefillP
   constexpr int kAhead = 8 / ROWS;  // ranges loaded together
   constexpr int kStep = kPrefillThreads / kMergeLanes;  // rows of the workgroup at a time
   int seq, h, mb;
-  if (!map_workgroup<PAGED>(p, seq, h, mb)) return;
+  if (!map_workgroup<PAGED, true>(p, seq, h, mb)) return;
   const int qlen = p.q_len[seq];
   const int pack = p.pack;
   const int rows = qlen * pack;
@@ -1477,15 +1476,15 @@ extern "C" int32_t nia_prefill_masked(void* out, int64_t out_tok_stride, int64_t
 namespace {
 
 int32_t prefill_paged_entry(void* out, int64_t out_tok_stride, int64_t out_head_stride,
-                                     const void* q, int64_t q_tok_stride, int64_t q_head_stride,
-                                     const void* k_cache, const void* v_cache,
-                                     const int32_t* block_tables, int32_t bt_stride,
-                                     int32_t max_blocks_per_seq, const int32_t* q_start,
-                                     const int32_t* q_len, const int64_t* context_lens,
-                                     int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
-                                     int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
-                                     int64_t num_blocks, float scale, int32_t causal,
-                                     int32_t dtype, void* stream, const SplitArgs& split) {
+                            const void* q, int64_t q_tok_stride, int64_t q_head_stride,
+                            const void* k_cache, const void* v_cache,
+                            const int32_t* block_tables, int32_t bt_stride,
+                            int32_t max_blocks_per_seq, const int32_t* q_start,
+                            const int32_t* q_len, const int64_t* context_lens,
+                            int32_t num_seqs, int32_t max_q_len, int32_t num_heads,
+                            int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
+                            int64_t num_blocks, float scale, int32_t causal,
+                            int32_t dtype, void* stream, const SplitArgs& split) {
   if (num_seqs < 0 || max_q_len < 0 || num_heads <= 0 || num_kv_heads <= 0 ||
       num_heads % num_kv_heads != 0 || max_blocks_per_seq < 0 ||
       bt_stride < max_blocks_per_seq || num_blocks < 0)

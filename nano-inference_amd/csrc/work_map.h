@@ -51,13 +51,14 @@ NIA_BOTH int key_ranges(int tiles, int splits) {
 // instead of 320-335.  With one query head per KV head the levels go out in turn: in runs, 12
 // prompts of up to 489 tokens (16 heads) took 26 us instead of 24, 40 of up to 180 (8 heads of
 // 64) 12.7 instead of 8.7.
-template <typename P>
+// RUNS: the grid may have packed heads (p.pack says whether it has).
+template <bool RUNS, typename P>
 NIA_BOTH bool prefill_map(const P& p, int id, int& seq, int& h, int& mb) {
   const int x = id % kXcds;
   const int t = id / kXcds;
   // `run` workgroups of one group follow each other: its heads of one level, or (packed heads)
   // kLevelRun levels of it, fewer where the levels end
-  const bool heads = p.pack == 1;
+  const bool heads = !RUNS || p.pack == 1;
   const int run = heads ? p.map_group : kLevelRun;
   const int per_z = p.groups_per_xcd * run;
   const int z0 = t / per_z;
@@ -67,7 +68,7 @@ NIA_BOTH bool prefill_map(const P& p, int id, int& seq, int& h, int& mb) {
   const int g = rem - j * len;
   const int gid = x + kXcds * j;
   const int z = heads ? z0 : z0 * kLevelRun + g;
-  if (gid >= p.num_seqs * p.num_kv_heads) return false;
+  if (z >= p.num_m_blocks || gid >= p.num_seqs * p.num_kv_heads) return false;
   seq = gid / p.num_kv_heads;
   h = (gid - seq * p.num_kv_heads) * p.map_group + (heads ? g : 0);
   mb = p.num_m_blocks - 1 - z;
@@ -130,7 +131,7 @@ inline int64_t q_span_bytes(int64_t q_tok, int64_t q_head, int32_t pack, int hea
 // keys 139 -> 75; 1024 rows after 12000 keys 242 -> 216.  Top-left causal calls (`top_left`)
 // stay uncut: their m-blocks average half the longest one's tiles, and a prompt of 2000 tokens
 // (16 and 8 heads) in two ranges ran 42-44 us, uncut 38.
-constexpr int kSplitSlots = 512;
+constexpr int kSplitSlots = 512;  // workgroups the chip holds at once
 constexpr int kSplitMax = 32;
 constexpr int kSplitGain = 12;
 
@@ -175,7 +176,7 @@ template <typename P>
 bool pack_uncut(const P& p, int max_q_len) {
   const int64_t own = head_blocks(p.group, max_q_len);
   return packed_blocks(p.group, max_q_len) * 16 <= own * 15 &&
-         own * p.num_seqs * p.num_kv_heads > 512;
+         own * p.num_seqs * p.num_kv_heads > kSplitSlots;
 }
 
 // The workgroups of a packed or unpacked grid.

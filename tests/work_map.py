@@ -37,7 +37,8 @@ int64_t t_f32_grid(Grid* p, int64_t rows, int top_left, int cut) {
 void t_map(const Grid* p, int kind, int n, const int* order, int* out) {
   for (int id = 0; id < n; ++id, out += 3) {
     int s = 0, h = 0, m = 0;
-    const bool ok = kind == 0   ? prefill_map(*p, id, s, h, m)
+    const bool ok = kind == 0   ? (p->pack > 1 ? prefill_map<true>(*p, id, s, h, m)
+                                             : prefill_map<false>(*p, id, s, h, m))
                     : kind == 1 ? prefill_map_ranked(*p, id, order, s, h, m)
                     : kind == 2 ? pair_map(*p, id, s, h, m)
                     : p->level_run
