@@ -11,10 +11,14 @@
 // uses them from registers (a row a wave, 2-byte accesses and a sine and cosine per row
 // before: 125 us at 8192 tokens of 32 + 8 heads in bf16, 1.75 TB/s; now 48-50 us, 4.4-4.5
 // TB/s, where a large device copy reaches 5.0; 1000 tokens 16.4 -> 9.4 us; an fp8 cache at
-// 4000 tokens of 28 + 4 heads 61 -> 18 us).  Few tokens: a token's rows are spread over
-// several waves (kRowsFillWaves), each with its own sines.  Measured and not taken: no
-// prefetch of the next group (6 instead of 5 waves per SIMD, +-2%), 72 registers for 7 waves
-// (spills, 77 us).
+// 4000 tokens of 28 + 4 heads 61 -> 18 us).  A token's rows may be spread over several waves
+// (kRowsFillWaves), each with its own sines.  Measured and not taken: no prefetch of the next
+// group (6 instead of 5 waves per SIMD, +-2%), 72 registers for 7 waves (spills, 77 us).
+//
+// Few rows (kFewRows; every decode step): qk_norm_rope_row_kernel, a wave per row, lane l holding
+// dims l and l + 64.  All rows fit the chip at once, so the call takes one wave's time, and 16
+// elements a lane take longer than two: 64 tokens of 28 + 4 heads 3.9 us in groups, 3.2 by rows;
+// over an fp8 cache, where every element is divided by its row's scale, 5.3 and 3.7.
 //
 // Every rounding point of the PyTorch form is kept (T = the model dtype):
 //   RMSNorm (src/nano_inference/layers/norm.py:35-47):
@@ -75,6 +79,11 @@ struct Num<float> {
 };
 
 constexpr int kRopeWaves = 4;  // waves per workgroup
+// Rows up to which the call takes a wave per row.  By rows and in groups, us, bf16 / fp8 cache:
+// 3200 rows 4.0 / 4.7 and 4.0 / 5.2, 4800 4.2 / 4.7 and 4.0 / 5.2, 6400 5.2 / 6.6 and 4.0 / 5.4.
+// Over an fp8 cache also where a token's rows do not fill a group (4 + 1 heads, 2100 tokens: 7.1
+// and 13.0): all lanes wait for the few that divide.
+constexpr int64_t kFewRows = 5120;
 constexpr int kRowGroup = 8;   // rows a wave handles at once (8 lanes each)
 constexpr int kHalf = 8;       // dims per lane and row half
 // Waves below which a token's row groups are spread over several waves (two per SIMD:
@@ -279,6 +288,86 @@ __global__ __launch_bounds__(kRopeWaves * kWave) void qk_norm_rope_kernel(RopePa
   }
 }
 
+// Row maximum of |x| over the wave's 128 values (two per lane); NaN as in octet_amax.
+NIA_DEVICE float row_amax(float a, float b) {
+  float m = fmaxf(fabsf(a), fabsf(b));
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, kWave));
+  return m;
+}
+
+// e4m3 code of x for a row scale (zero row: scale 0, code 0).
+NIA_DEVICE uint8_t fp8_code(float x, float scale) {
+  return scale > 0.f ? (uint8_t)(fp8x2_from_f32(x / scale, 0.f) & 0xffu) : (uint8_t)0;
+}
+
+// One wave per (token, head) row: rows 0 .. H - 1 of a token are its query heads, the others its
+// key heads.
+template <typename T, bool FP8>
+__global__ __launch_bounds__(kRopeWaves * kWave) void qk_norm_rope_row_kernel(RopeParams p) {
+  using N = Num<T>;
+  constexpr int D = 128;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int per_tok = p.num_heads + p.num_kv_heads;
+  const int64_t row = (int64_t)blockIdx.x * kRopeWaves + (threadIdx.x >> 6);
+  if (row >= (int64_t)p.num_tokens * per_tok) return;
+  const int tok = (int)(row / per_tok);
+  const int hh = (int)(row - (int64_t)tok * per_tok);
+  const bool is_q = hh < p.num_heads;
+  const int hk = hh - p.num_heads;
+  T* x = is_q ? reinterpret_cast<T*>(p.q) + tok * p.q_tok + (int64_t)hh * p.q_head
+              : reinterpret_cast<T*>(p.k) + tok * p.k_tok + (int64_t)hk * p.k_head;
+  const T* w = reinterpret_cast<const T*>(is_q ? p.q_w : p.k_w);
+
+  float y0 = N::f(x[lane]);
+  float y1 = N::f(x[lane + 64]);
+  if (w != nullptr) {
+    float ss = y0 * y0 + y1 * y1;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) ss += __shfl_xor(ss, off, kWave);
+    const float r = rsqrtf(ss / (float)D + p.eps);
+    y0 = N::f(N::t(N::f(N::t(y0 * r)) * N::f(w[lane])));
+    y1 = N::f(N::t(N::f(N::t(y1 * r)) * N::f(w[lane + 64])));
+  }
+  const int axis = p.num_axes == 1 ? 0 : (lane < p.sec0 ? 0 : (lane < p.sec0 + p.sec1 ? 1 : 2));
+  const float ang = (float)p.pos[axis * p.pos_axis + tok] * p.inv_freq[lane];
+  const float c = N::f(N::t(cosf(ang)));
+  const float s = N::f(N::t(sinf(ang)));
+  const T o0 = N::t(N::f(N::t(y0 * c)) + N::f(N::t(-y1 * s)));
+  const T o1 = N::t(N::f(N::t(y1 * c)) + N::f(N::t(y0 * s)));
+  x[lane] = o0;
+  x[lane + 64] = o1;
+  if (is_q || p.k_cache == nullptr) return;
+  const int64_t slot = p.slots[tok];
+  if (slot < 0 || slot >= p.num_slots) return;
+  const int64_t blk = slot / p.block_size;
+  const int64_t cache_row =
+      (blk * p.num_kv_heads + hk) * p.block_size + (slot - blk * p.block_size);
+  const T* vr = reinterpret_cast<const T*>(p.v) + tok * p.v_tok + (int64_t)hk * p.v_head;
+  const T v0 = vr[lane], v1 = vr[lane + 64];
+  if constexpr (FP8) {
+    const float ks = row_amax(N::f(o0), N::f(o1)) / kE4m3Max;
+    const float vs = row_amax(N::f(v0), N::f(v1)) / kE4m3Max;
+    uint8_t* kc = reinterpret_cast<uint8_t*>(p.k_cache) + cache_row * D + lane;
+    uint8_t* vc = reinterpret_cast<uint8_t*>(p.v_cache) + cache_row * D + lane;
+    kc[0] = fp8_code(N::f(o0), ks);
+    kc[64] = fp8_code(N::f(o1), ks);
+    vc[0] = fp8_code(N::f(v0), vs);
+    vc[64] = fp8_code(N::f(v1), vs);
+    if (lane == 0) {
+      p.k_scale[cache_row] = ks;
+      p.v_scale[cache_row] = vs;
+    }
+  } else {
+    T* kc = reinterpret_cast<T*>(p.k_cache) + cache_row * D + lane;
+    T* vc = reinterpret_cast<T*>(p.v_cache) + cache_row * D + lane;
+    kc[0] = o0;
+    kc[64] = o1;
+    vc[0] = v0;
+    vc[64] = v1;
+  }
+}
+
 // 16-byte accesses: aligned pointers, strides of whole 16-byte groups.
 bool rope_vec_ok(const RopeParams& p, int es, bool write, bool fp8) {
   auto ptr = [](const void* x, int a) { return (uintptr_t)x % a == 0; };
@@ -292,9 +381,11 @@ bool rope_vec_ok(const RopeParams& p, int es, bool write, bool fp8) {
 }
 
 template <typename T, bool FP8>
-void launch_rope(const RopeParams& p, dim3 grid, bool vec, hipStream_t s) {
+void launch_rope(const RopeParams& p, dim3 grid, bool by_rows, bool vec, hipStream_t s) {
   const dim3 block(kRopeWaves * kWave);
-  if (vec)
+  if (by_rows)
+    nia_launch((qk_norm_rope_row_kernel<T, FP8>), grid, block, s, p);
+  else if (vec)
     nia_launch((qk_norm_rope_kernel<T, FP8, true>), grid, block, s, p);
   else
     nia_launch((qk_norm_rope_kernel<T, FP8, false>), grid, block, s, p);
@@ -368,20 +459,22 @@ int32_t launch_qk_norm_rope(
   parts = (row_groups + per_part - 1) / per_part;  // no empty part
   p.parts = (int32_t)parts;
   p.part_rows = (int32_t)(per_part * kRowGroup);
-  const int64_t wgs = ((int64_t)num_tokens * parts + kRopeWaves - 1) / kRopeWaves;
+  const bool by_rows = num_tokens * rows <= kFewRows || (fp8 && rows < kRowGroup);
+  const int64_t wgs =
+      ((int64_t)num_tokens * (by_rows ? rows : parts) + kRopeWaves - 1) / kRopeWaves;
   if (wgs > kMaxGroups) return NIA_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
   const dim3 grid((unsigned)wgs);
   const bool bf16 = dtype == NIA_DTYPE_BF16;
   const bool vec = rope_vec_ok(p, bf16 ? 2 : 4, write, fp8);
   if (bf16 && fp8)
-    launch_rope<bf16_t, true>(p, grid, vec, s);
+    launch_rope<bf16_t, true>(p, grid, by_rows, vec, s);
   else if (bf16)
-    launch_rope<bf16_t, false>(p, grid, vec, s);
+    launch_rope<bf16_t, false>(p, grid, by_rows, vec, s);
   else if (fp8)
-    launch_rope<float, true>(p, grid, vec, s);
+    launch_rope<float, true>(p, grid, by_rows, vec, s);
   else
-    launch_rope<float, false>(p, grid, vec, s);
+    launch_rope<float, false>(p, grid, by_rows, vec, s);
   return hipGetLastError() == hipSuccess ? NIA_OK : NIA_ERR_LAUNCH;
 }
 

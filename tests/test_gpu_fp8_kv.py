@@ -310,13 +310,14 @@ def test_paged_layer_with_fp8_cache_matches_reference_pipeline():
         close(out, exp, f"fp8 decode step {t}")
 
 
+@pytest.mark.parametrize("n", [20, 500])  # a wave a row, groups of rows
 @pytest.mark.parametrize("norm", [True, False])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-def test_nan_rows_stay_nan(dtype, norm):
+def test_nan_rows_stay_nan(dtype, norm, n):
     """A K or V row that is all NaN keeps a NaN scale (and zero codes), in the separate and in
     the fused write; a lone NaN shows in its own element, or behind the norm in its whole row."""
     g = torch.Generator().manual_seed(15)
-    n, hkv, nb, nan = 20, 4, 4, float("nan")
+    hkv, nb, nan = 4, n // 16 + 2, float("nan")
     q = torch.randn(n, 8, 128, generator=g).to(dtype)
     k, v = (torch.randn(n, hkv, 128, generator=g).to(dtype) for _ in range(2))
     k[1, 0] = nan

@@ -1,6 +1,7 @@
-"""The fused QK step at the edges of its row layout: rows that do not fill a group of
-eight, a token's rows in one wave or spread over several (few tokens), query and key rows
-in one group, and views whose rows are not 16-byte aligned (element accesses).  Bars as in
+"""The fused QK step at the edges of its row layouts: a wave a row and groups of eight, on both
+sides of their bound, rows that do not fill a group, a token's rows in one wave or spread over
+several, query and key rows in one group, and views whose rows are not 16-byte aligned
+(element accesses).  Bars as in
 test_gpu_qk_rope; cache rows bit-identical to the write of the kernel's own k and the
 input v."""
 import pytest
@@ -29,7 +30,10 @@ def _rows(x, shift):
 @pytest.mark.parametrize("shift", [0, 1])
 @pytest.mark.parametrize("store", ["bf16", "fp8", "f32"])
 @pytest.mark.parametrize("n,h,hkv,mrope", [(1, 16, 8, False), (3, 7, 1, False), (33, 28, 4, True),
-                                           (700, 32, 8, False), (2051, 3, 1, False)])
+                                           (700, 32, 8, False), (2051, 3, 1, False),
+                                           # a wave a row up to 5120 rows, groups past them
+                                           (128, 32, 8, True), (129, 32, 8, False),
+                                           (161, 31, 1, False), (2561, 1, 1, False)])
 def test_row_groups(n, h, hkv, mrope, store, shift):
     print(f"rope rows n={n} h={h} hkv={hkv} mrope={mrope} {store} shift={shift}", flush=True)
     dtype = torch.float32 if store == "f32" else torch.bfloat16
