@@ -30,7 +30,7 @@
 // out but two stages kept), 109 decodes of up to 40 keys (16 heads of 64) 27.7 and 18.1.
 // Against one head a block, tiles loaded behind a barrier each and the shortest blocks
 // first: four prompts of 128-1024 tokens (16 and 8 heads, D 128) 268 -> 182 us, one of 1000
-// 192 -> 114, four of 1000 551 -> 280.  The fp64 products bound it: v_mfma_f64_16x16x4 issues
+// 192 -> 111, four of 1000 551 -> 281.  The fp64 products bound it: v_mfma_f64_16x16x4 issues
 // every 115-128 cycles (probe; 64 at the nominal rate), so a 16 x 32 tile is ~10k cycles,
 // 4.3 us, and a second wave on the SIMD adds nothing.  v_mfma_f64_4x4x4 issues every 16.6 (1.7
 // times the rate), but with its keys broadcast over the four blocks it reads and widens every

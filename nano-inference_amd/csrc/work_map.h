@@ -126,11 +126,11 @@ inline int64_t q_span_bytes(int64_t q_tok, int64_t q_head, int32_t pack, int hea
 // 512 workgroups about 13.6 us to write and read back, so n ranges cost 1.1 tiles / n +
 // 13.6 n nwg / 512 us: least at n = sqrt(41 tiles / nwg).  At most what the chip holds at
 // once (two workgroups a CU), and none where fewer than kSplitGain tiles are saved (the
-// second launch).  A 64-row chunk after 8000 keys (32 and 8 heads) 145 us uncut, 30 in 31
-// ranges, 26 in 15; 24 rows after 16000 keys 279 -> 26; eight 40-row chunks after 500-8192
-// keys 139 -> 75; 1024 rows after 12000 keys 242 -> 216.  Top-left causal calls (`top_left`)
-// stay uncut: their m-blocks average half the longest one's tiles, and a prompt of 2000 tokens
-// (16 and 8 heads) in two ranges ran 42-44 us, uncut 38.
+// second launch).  Uncut, and in the ranges this takes (32 and 8 heads, one GPU): 64 rows after
+// 8000 keys 146 us, 30 in 17; 24 rows after 16000 282, 26 in 32; eight 40-row chunks after
+// 500-8192 keys 144, 64 in 4; 1024 rows after 12000 252, 222 in 2.  Top-left causal calls
+// (`top_left`) stay uncut: their m-blocks average half the longest one's tiles, and a prompt of
+// 2000 tokens (16 and 8 heads) in two ranges ran 42-44 us, uncut 38.
 constexpr int kSplitSlots = 512;  // workgroups the chip holds at once
 constexpr int kSplitMax = 32;
 constexpr int kSplitGain = 12;
