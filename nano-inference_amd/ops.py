@@ -562,13 +562,15 @@ def prefill(
         )
         _lib.check("nia_prefill_masked", st)
         return out
-    # The keys of a sequence choose its ranges: the lengths are on the device, so the longest
-    # query run where there are as many keys as queries, else the mean.  For the sum of 16
-    # sequences of 1000 keys, 32 rows each, the call was cut: 24.9 us instead of 22.2.
+    # The keys of a sequence choose its ranges.  The lengths are on the device: the longest query
+    # run where there are as many keys as queries, else half as many again as the mean, about
+    # the longest of lengths that vary.  For the sum of all, 16 sequences of 32 rows over 1000
+    # keys took 24.4 us instead of 22.4; for the mean, 3 of one row over 560-2235 keys (32 and 8
+    # heads) 19 us instead of 13.
     if keys == rows:
         keys = max_q_len
     elif n > 1:
-        keys = -(-keys // n)
+        keys = min(keys, -(-3 * keys // (2 * n)))
     ws = None
     if dt != _lib.DTYPE_BF16:
         if rows * h <= _SPLIT_MAX_ROWS_F32:

@@ -182,7 +182,8 @@ def test_captured_call_replays():
 
 
 @pytest.mark.parametrize("dtype,ql,kl,cut", [
-    (torch.bfloat16, [32] * 16, [1000] * 16, False), (torch.bfloat16, [64], [8000], True),
+    (torch.bfloat16, [32] * 16, [700] * 16, False), (torch.bfloat16, [64], [8000], True),
+    (torch.bfloat16, [1] * 3, [2235, 560, 1300], True),
     (torch.float32, [8] * 20, [100] * 20, False), (torch.float32, [200], [900], True),
     (torch.float32, [30, 400, 10], [30, 400, 10], True), (torch.float32, [30] * 14, [30] * 14, False)])
 def test_ranges_are_chosen_for_one_sequence_not_for_the_sum(monkeypatch, dtype, ql, kl, cut):
