@@ -27,7 +27,8 @@
 // stage and no read-ahead, which leaves room for three workgroups a CU (D 64: four) that hide
 // each other's loads: four images of 784-3072 rows (16 heads of 80) 1633 us with two stages and
 // two workgroups, 1528 so, 114 windows of 16-64 rows 61.5 and 52.0 (54 with 512-byte rows left
-// out but two stages kept), 109 decodes of up to 40 keys (16 heads of 64) 27.7 and 18.1.
+// out but two stages kept), 109 decodes of up to 40 keys (16 heads of 64) 27.7 and 18.1.  Decodes
+// of at most two workgroups a CU keep two stages (f32_two_stages).
 // Against one head a block, tiles loaded behind a barrier each and the shortest blocks
 // first: four prompts of 128-1024 tokens (16 and 8 heads, D 128) 268 -> 182 us, one of 1000
 // 192 -> 111, four of 1000 551 -> 281.  The fp64 products bound it: v_mfma_f64_16x16x4 issues
@@ -69,15 +70,16 @@ NIA_DEVICE int f32_tok(const PrefillF32Params& p, int r) {
   return p.group == 1 ? r : key_block(r, p.group_magic, p.group_shift);
 }
 
-template <int D>
-constexpr int kF32PerSimd = D == 64 ? 4 : D < 128 ? 3 : 2;  // waves a SIMD: workgroups a CU
+// Waves a SIMD (workgroups a CU) that the registers and LDS of one stage (two: PIPE) leave room for.
+template <int D, bool PIPE>
+constexpr int kF32PerSimd = D == 64 ? (PIPE ? 3 : 4) : D < 128 && !PIPE ? 3 : 2;
 
 // Element kinds: fp32 rows, bf16 rows, or a paged fp8 cache (e4m3 codes with one fp32
 // scale per cache row; q and o in bf16).  Every element is widened to fp32 in LDS (fp8 as
 // code * row scale in fp32, the rows the fp8 format stands for), so one kernel serves the
 // cache layouts the bf16 and fp8 kernels do not take: any block size, any group.
-template <int D, bool PAGED, int E>
-__global__ __launch_bounds__(kF32Threads, kF32PerSimd<D>) void prefill_f32_kernel(
+template <int D, bool PAGED, int E, bool PIPE>
+__global__ __launch_bounds__(kF32Threads, (kF32PerSimd<D, PIPE>)) void prefill_f32_kernel(
     PrefillF32Params p) {
   static_assert(D % 16 == 0 && D <= 128, "head_dim a multiple of 16, at most 128");
   static_assert(E == kElemF32 || PAGED, "bf16 and fp8 elements come from a paged cache");
@@ -88,7 +90,7 @@ __global__ __launch_bounds__(kF32Threads, kF32PerSimd<D>) void prefill_f32_kerne
   constexpr int kChunks = kF32BlockN * kC4;  // per operand
   constexpr int kItems = (kChunks + kF32Threads - 1) / kF32Threads;  // of a thread
   constexpr int kAhead = D == 128;  // operands read from LDS a step ahead
-  constexpr int kStages = D == 128 ? 2 : 1;  // of LDS
+  constexpr int kStages = PIPE ? 2 : 1;  // of LDS
   __shared__ __attribute__((aligned(16))) float sk[kStages][kF32BlockN * kRow];
   __shared__ __attribute__((aligned(16))) float sv[kStages][kF32BlockN * kRow];
   __shared__ int sok[kStages][kF32BlockN];  // key of the tile lies in a valid block
@@ -466,10 +468,21 @@ __global__ __launch_bounds__(kF32Threads) void prefill_f32_merge_kernel(PrefillF
   *reinterpret_cast<float4*>(o) = make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
 }
 
+template <int D, bool PAGED, int E>
+void launch_f32(const PrefillF32Params& p, dim3 grid, hipStream_t s) {
+  if constexpr (PAGED && D < 128) {
+    const int64_t nwg = (int64_t)grid.x * grid.y * grid.z;
+    if (p.decode && f32_two_stages(D, nwg, (int64_t)p.max_blocks * p.block_size)) {
+      nia_launch((prefill_f32_kernel<D, PAGED, E, true>), grid, dim3(kF32Threads), s, p);
+      return;
+    }
+  }
+  nia_launch((prefill_f32_kernel<D, PAGED, E, D == 128>), grid, dim3(kF32Threads), s, p);
+}
+
 template <int D, bool PAGED>
 void launch_f32_split(const PrefillF32Params& p, dim3 grid, hipStream_t s) {
-  nia_launch((prefill_f32_kernel<D, PAGED, kElemF32>), dim3(grid.x, (unsigned)p.splits),
-             dim3(kF32Threads), s, p);
+  launch_f32<D, PAGED, kElemF32>(p, dim3(grid.x, (unsigned)p.splits), s);
   nia_launch((prefill_f32_merge_kernel<D, PAGED>), dim3(grid.x, kF32BlockM * 32 / kF32Threads),
              dim3(kF32Threads), s, p);
 }
@@ -518,7 +531,7 @@ int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int nu
                                 : dim3((unsigned)p.num_m_blocks, (unsigned)p.num_kv_heads,
                                        (unsigned)num_seqs);
   if (elem == kElemFp8) {
-    nia_launch((prefill_f32_kernel<128, true, kElemFp8>), grid, dim3(kF32Threads), stream, p);
+    launch_f32<128, true, kElemFp8>(p, grid, stream);
     return hipGetLastError() == hipSuccess ? NIA_OK : NIA_ERR_LAUNCH;
   }
   switch (head_dim) {
@@ -528,12 +541,12 @@ int32_t launch_prefill_f32(PrefillF32Params& p, bool paged, int head_dim, int nu
       launch_f32_split<DD, true>(p, grid, stream);                                            \
     else if (p.splits > 1)                                                                    \
       launch_f32_split<DD, false>(p, grid, stream);                                           \
-    else if (!paged)                                                                               \
-      nia_launch((prefill_f32_kernel<DD, false, kElemF32>), grid, dim3(kF32Threads), stream, p); \
+    else if (!paged)                                                                          \
+      launch_f32<DD, false, kElemF32>(p, grid, stream);                                       \
     else if (elem == kElemF32)                                                                \
-      nia_launch((prefill_f32_kernel<DD, true, kElemF32>), grid, dim3(kF32Threads), stream, p); \
+      launch_f32<DD, true, kElemF32>(p, grid, stream);                                        \
     else                                                                                      \
-      nia_launch((prefill_f32_kernel<DD, true, kElemBf16>), grid, dim3(kF32Threads), stream, p); \
+      launch_f32<DD, true, kElemBf16>(p, grid, stream);                                       \
     break;
     NIA_F32_CASE(64)
     NIA_F32_CASE(80)

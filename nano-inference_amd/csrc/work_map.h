@@ -205,6 +205,21 @@ NIA_BOTH int f32_ranges(int tiles, int splits) {
   return at_least(at_most(splits, (tiles + kF32RangeTiles - 1) / kF32RangeTiles), 1);
 }
 
+// Decode at a head dim below 128: two LDS stages where no CU has more than two workgroups, so
+// that no third hides their loads (fp32, one stage and two): 32 sequences of 70 keys (16 heads of
+// 96) 18.0 and 16.9 us, of 250 48.2 and 41.9, 76 of up to 827 (28 and 4 heads of 64) 101.7 and
+// 86.5, 3 of 6032 601 and 572; 1016 workgroups of up to 786 keys (32 and 8 heads of 96) 234 and
+// 250.  A context of two tiles gains nothing from the second stage (45 of up to 49, 6 and 2 heads
+// of 96, 10.8 and 11.2), nor do 64 workgroups at a head dim of 80, which is no multiple of the
+// four tiles a 16-byte read feeds (7 sequences of 2301 keys, 6 and 2 heads, 252.9 and 259.4; 112
+// workgroups of 7920 keys 1154 and 1102).
+constexpr int kF32PipeGroups = 512;
+constexpr int kF32PipeKeys = 2 * kF32BlockN;
+NIA_BOTH bool f32_two_stages(int head_dim, int64_t workgroups, int64_t table_keys) {
+  return workgroups <= kF32PipeGroups && table_keys > kF32PipeKeys &&
+         (head_dim != 80 || workgroups > 64);
+}
+
 // The workgroup's (sequence, KV head, row block).  `id`: its number in the 1-D grid, or x in a
 // 3-D one (level_run 0) of row blocks, KV heads and sequences.  Runs of level_run adjacent
 // levels of one (sequence, KV head) group follow each other (f32_run); the groups lie over all

@@ -110,7 +110,6 @@ def lib():
     so.t_merge_waves.argtypes = [i64, i64, i64]
     so.t_few.argtypes = [i64, i64]
     so.t_few_per.argtypes = [i64, i64, i64, i64]
-    so.t_few_per.argtypes = [i64, i64]
     return so
 
 
